@@ -396,31 +396,41 @@ struct NbrSrc {
     uint32_t cap;
 };
 
-struct LoadX {  // lo = hi = {x_t, -}
+// Cache policy bits of a buffer load on gfx950: bit 1 = non-temporal.
+constexpr int kBufferNonTemporal = 2;
+struct LoadTraits {
+    static constexpr int kListCache = kBufferNonTemporal;  // policy of the staged list's loads: read once per launch
+    static constexpr bool kAlwaysSplit = false;            // HaloRec's 16 + 8 byte form whatever VFD_PACK_RECORDS says
+};
+
+struct LoadX : LoadTraits {  // lo = hi = {x_t, -}
     static constexpr int kLo = 3, kHi = 0;  // floats of lo and hi that the neighbour terms read
     static constexpr bool kShortSqrt = false;  // the table code's square root: sqrt_rn (true) or sqrtf
     const float4* __restrict__ pos;
+    __device__ __forceinline__ LoadX(const float4* p) : pos(p) {}
     __device__ __forceinline__ void operator()(uint32_t t, float4& lo, float4& hi) const {
         lo = pos[t];
         hi = lo;
     }
 };
-struct LoadXS {  // lo = hi = {x_t, s_t}
+struct LoadXS : LoadTraits {  // lo = hi = {x_t, s_t}
     static constexpr int kLo = 4, kHi = 0;
     static constexpr bool kShortSqrt = true;
     const float4* __restrict__ pos;
     const float* __restrict__ s;
+    __device__ __forceinline__ LoadXS(const float4* p, const float* s_) : pos(p), s(s_) {}
     __device__ __forceinline__ void operator()(uint32_t t, float4& lo, float4& hi) const {
         const float4 x = pos[t];
         lo = make_float4(x.x, x.y, x.z, s[t]);
         hi = lo;
     }
 };
-struct LoadXV {  // lo = {x_t, -}, hi = {v_t, -}
+struct LoadXV : LoadTraits {  // lo = {x_t, -}, hi = {v_t, -}
     static constexpr int kLo = 3, kHi = 3;
     static constexpr bool kShortSqrt = false;
     const float4* __restrict__ pos;
     const float4* __restrict__ v;
+    __device__ __forceinline__ LoadXV(const float4* p, const float4* v_) : pos(p), v(v_) {}
     __device__ __forceinline__ void operator()(uint32_t t, float4& lo, float4& hi) const {
         lo = pos[t];
         hi = v[t];
@@ -429,37 +439,40 @@ struct LoadXV {  // lo = {x_t, -}, hi = {v_t, -}
 // Viscosity records: lo = {x_t, m / rho_t} (hi = {v_t, -}). The division is the one the neighbour terms take per pair
 // (m / rho_j, DFSPHKernels.cu:638, :790), formed once per halo record instead; m is the same for every scene of a
 // batch (all scenes share the particle radius).
-struct LoadXQ {
+struct LoadXQ : LoadTraits {
     static constexpr int kLo = 4, kHi = 0;
     static constexpr bool kShortSqrt = true;
     const float4* __restrict__ pos;
     const float* __restrict__ rho;
     float m;
+    __device__ __forceinline__ LoadXQ(const float4* p, const float* r, float m_) : pos(p), rho(r), m(m_) {}
     __device__ __forceinline__ void operator()(uint32_t t, float4& lo, float4& hi) const {
         const float4 x = pos[t];
         lo = make_float4(x.x, x.y, x.z, m / rho[t]);
         hi = lo;
     }
 };
-struct LoadXQV {
+struct LoadXQV : LoadTraits {
     static constexpr int kLo = 4, kHi = 3;
     static constexpr bool kShortSqrt = true;
     const float4* __restrict__ pos;
     const float* __restrict__ rho;
     const float4* __restrict__ v;
     float m;
+    __device__ __forceinline__ LoadXQV(const float4* p, const float* r, const float4* v_, float m_) : pos(p), rho(r), v(v_), m(m_) {}
     __device__ __forceinline__ void operator()(uint32_t t, float4& lo, float4& hi) const {
         const float4 x = pos[t];
         lo = make_float4(x.x, x.y, x.z, m / rho[t]);
         hi = v[t];
     }
 };
-struct LoadXSV {  // lo = {x_t, s_t}, hi = {v_t, -}
+struct LoadXSV : LoadTraits {  // lo = {x_t, s_t}, hi = {v_t, -}
     static constexpr int kLo = 4, kHi = 3;
     static constexpr bool kShortSqrt = true;
     const float4* __restrict__ pos;
     const float* __restrict__ s;
     const float4* __restrict__ v;
+    __device__ __forceinline__ LoadXSV(const float4* p, const float* s_, const float4* v_) : pos(p), s(s_), v(v_) {}
     __device__ __forceinline__ void operator()(uint32_t t, float4& lo, float4& hi) const {
         const float4 x = pos[t];
         lo = make_float4(x.x, x.y, x.z, s[t]);
@@ -508,7 +521,7 @@ template <int R> struct ListShape {
 #define VFD_SCHED_PHASES 1
 #endif
 template <class Load> struct HaloRec {
-    static constexpr bool kSplit = VFD_PACK_RECORDS == 2 && Load::kLo == 3 && Load::kHi == 3;
+    static constexpr bool kSplit = (VFD_PACK_RECORDS == 2 || Load::kAlwaysSplit) && Load::kLo == 3 && Load::kHi == 3;
     static constexpr int L = kSplit ? 4 : (VFD_PACK_RECORDS ? Load::kLo : 4);
     static constexpr int H = Load::kHi == 0 ? 0 : (kSplit ? 2 : (VFD_PACK_RECORDS ? Load::kHi : 4));
     static constexpr size_t kBytes = (size_t)(L + H) * sizeof(float) * kHaloMax;  // LDS of the records
@@ -556,8 +569,6 @@ constexpr int kRawBufferWord3 = 0x00020000;
 // keeps the load in the instruction stream (so the compiler still counts it in flight) but takes it off the memory
 // path. Valid offsets stay below 2^31 bytes (a simulation holds at most 2^28 slots: 8-byte row-pair entries).
 constexpr uint32_t kBufferOutOfRange = 0x80000000u;
-// Cache policy bits of a buffer load on gfx950: bit 1 = non-temporal.
-constexpr int kBufferNonTemporal = 2;
 
 template <int R, class TV, class Load, class Fn>
 __device__ __forceinline__ void each_neighbor_rec(const NbrSrc& src, uint32_t i, float cutR, float invStep, f3 xi,
@@ -585,7 +596,7 @@ __device__ __forceinline__ void each_neighbor_rec(const NbrSrc& src, uint32_t i,
                     const_cast<uint32_t*>(src.local + (size_t)(r >> 1) * cap * 2), (short)0, (int)(cap * 8),
                     kRawBufferWord3);
                 const uint32_t off = i * 8u + (r <= last ? 0u : kBufferOutOfRange);
-                const auto v = __builtin_amdgcn_raw_buffer_load_b64(rows, (int)off, 0, kBufferNonTemporal);
+                const auto v = __builtin_amdgcn_raw_buffer_load_b64(rows, (int)off, 0, Load::kListCache);
                 e[2 * u] = v[0];
                 e[2 * u + 1] = v[1];
             }

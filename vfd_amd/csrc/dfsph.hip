@@ -10,19 +10,9 @@
 //     host only polls every few iterations instead of copying a scalar back per iteration;
 //   - ClearAcceleration is fused into the divergence finaliser; the position update into the pressure finaliser.
 // Floating-point expressions keep the reference's association order (no implicit contraction; -ffp-contract=off).
-#include "device.h"
-#include "kernels.h"
+#include "terms.h"
 
 namespace vfd {
-
-__device__ __forceinline__ KTab ktab(const KTabHost& h) { return KTab{h.tab, h.R, h.R2, h.invStep, h.W0}; }
-__device__ __forceinline__ uint32_t nbr(const Fields& F, uint32_t cap, uint32_t i, uint32_t j) {
-    return F.nbrList[(size_t)j * cap + i];
-}
-__device__ __forceinline__ HaloView halo(const Fields& F) { return HaloView{F.haloCount, F.haloIds}; }
-__device__ __forceinline__ NbrSrc global_src(const Fields& F, uint32_t cap) {
-    return NbrSrc{nullptr, F.nbrLocal, F.nbrList, F.nbrCount, cap};
-}
 
 // Dynamic LDS of the staged kernels: the kernel table, then the halo records of the current group.
 constexpr size_t kLdsDensity = kLdsWG + HaloRec<LoadX>::kBytes;
@@ -82,75 +72,6 @@ void launch_density_factor(const Launch& L, const KTabHost& kt, const Fields& F)
     hipLaunchKernelGGL(k_density_factor, dim3(L.gridGroups), dim3(kGroupSize), kLdsDensity,
                        L.stream, L.P, L.tileScene, kt, F, L.capacity, TileGrid(L.tg));
 }
-
-// ---- shared neighbour sums --------------------------------------------------------------------------------------
-// v_i-weighted divergence sum_j (v_i - v_j).gradW_ij * V + sum_b V_b v_i.gradW_ib (:233-278, :483-529);
-// records lo = {x_j}, hi = {v_j}
-__device__ __forceinline__ float velocity_divergence(const SceneParams& p, const KLds& k, const Fields& F,
-                                                     uint32_t cap, uint32_t i, const NbrSrc& src) {
-    const f3 xi = ld3(F.pos[i]), vi = ld3(F.vel[i]);
-    float d = 0.0f;
-    each_neighbor_rec<2>(src, i, k.R, k.invStep, xi, k.sG, LoadXV{F.pos, F.vel}, [&](float4 lo, float4 hi, float g) {
-        d += dot3(vi - ld3(hi), g * (xi - ld3(lo)));
-    });
-    d *= p.V;
-    for (uint32_t b = 0; b < p.bodyCount; ++b) {
-        const float vb = F.vb[(size_t)b * cap + i];
-        if (vb > 0.0f) d += vb * dot3(vi, gradW(k, xi - ld3(F.xb[(size_t)b * cap + i])));
-    }
-    return d;
-}
-
-// pressure acceleration from kappa (ComputePressureAccelerationKernel :342-386 and its three siblings);
-// records lo = {x_j, kappa_j}
-__device__ __forceinline__ f3 pressure_accel(const SceneParams& p, const KLds& k, const Fields& F, uint32_t cap,
-                                             uint32_t i, const float* __restrict__ kap, const NbrSrc& src) {
-    const f3 xi = ld3(F.pos[i]);
-    const float ki = kap[i];
-    const float negV = -p.V;  // read before the loop: a global read inside it would wait for the list prefetch
-    f3 a = mk3(0.0f, 0.0f, 0.0f);
-    each_neighbor_rec<1>(src, i, k.R, k.invStep, xi, k.sG, LoadXS{F.pos, kap}, [&](float4 lo, float4, float g) {
-        const float s = ki + lo.w;
-        if (above_eps(fabsf(s))) {
-            const f3 gj = negV * (g * (xi - ld3(lo)));
-            a = a + s * gj;
-        }
-    });
-    if (above_eps(fabsf(ki))) {
-        for (uint32_t b = 0; b < p.bodyCount; ++b) {
-            const float vb = F.vb[(size_t)b * cap + i];
-            if (vb > 0.0f) {
-                const f3 gj = (-vb) * gradW(k, xi - ld3(F.xb[(size_t)b * cap + i]));
-                a = a + ki * gj;
-            }
-        }
-    }
-    return a;
-}
-
-// ComputeDensityPressureForce (:280-315); records lo = {x_j}, hi = {a_j}
-__device__ __forceinline__ float density_pressure_force(const SceneParams& p, const KLds& k, const Fields& F,
-                                                        uint32_t cap, uint32_t i, const NbrSrc& src) {
-    const f3 xi = ld3(F.pos[i]), ai = ld3(F.ap[i]);
-    float f = 0.0f;
-    each_neighbor_rec<2>(src, i, k.R, k.invStep, xi, k.sG, LoadXV{F.pos, F.ap}, [&](float4 lo, float4 hi, float g) {
-        f += dot3(ai - ld3(hi), g * (xi - ld3(lo)));
-    });
-    f *= p.V;
-    for (uint32_t b = 0; b < p.bodyCount; ++b) {
-        const float vb = F.vb[(size_t)b * cap + i];
-        if (vb > 0.0f) f += vb * dot3(ai, gradW(k, xi - ld3(F.xb[(size_t)b * cap + i])));
-    }
-    return f;
-}
-
-// Every gradient-loop kernel stages the G table in LDS, followed by the halo records of the current group.
-#define VFD_HALO_KERNEL_PROLOGUE(kh)                                   \
-    extern __shared__ float4 lds[];                                    \
-    float* sG = reinterpret_cast<float*>(lds);                         \
-    load_table_g(sG, (kh).tab);                                        \
-    const KLds K{sG, (kh).R, (kh).invStep};                            \
-    float* rec = reinterpret_cast<float*>(lds + kLdsG / sizeof(float4));
 
 // ---- Jacobi solver control (DFSPHImplementation.cu:455-461, 526-532) -------------------------------------------
 // The per-scene finalisers (Jacobi, CG) run one 1024-thread block per scene: the tile partials of a 2M scene are then
@@ -216,7 +137,7 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_div_init(const Sce
         const TileCtx c = tile_ctx4(tile, ok, tileScene, P);
         const SceneParams& p = P[c.s];
         if (!c.valid || !p.enableDiv) return;
-        float d = velocity_divergence(p, K, F, cap, c.i, src);
+        float d = field_divergence(p, K, F, cap, c.i, ld3(F.vel[c.i]), LoadXV{F.pos, F.vel}, src);
         d = F.nbrCount[c.i] < 20u ? 0.0f : fmaxf(d, 0.0f);
         F.densAdv[c.i] = d;
         const float f = F.factor[c.i] * F.state[c.s].dtInv;
@@ -234,7 +155,7 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_div_accel(const Sc
     group_loop<1>(tg, halo(F), rec, global_src(F, cap), LoadXS{F.pos, F.kappaV}, [&](uint32_t tile, bool ok, const NbrSrc& src) {
         const TileCtx c = tile_ctx4(tile, ok, tileScene, P);
         if (!F.state[c.s].div.active || !c.valid) return;
-        F.ap[c.i] = st4(pressure_accel(P[c.s], K, F, cap, c.i, F.kappaV, src));
+        F.ap[c.i] = st4(pressure_accel(P[c.s], K, F, cap, c.i, F.kappaV[c.i], LoadXS{F.pos, F.kappaV}, src));
     });
 }
 
@@ -251,7 +172,7 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_div_iter(const Sce
         const SceneParams& p = P[c.s];
         double part = 0.0;
         if (act && c.valid) {
-            const float f = density_pressure_force(p, K, F, cap, c.i, src) * st.dt;
+            const float f = field_divergence(p, K, F, cap, c.i, ld3(F.ap[c.i]), LoadXV{F.pos, F.ap}, src) * st.dt;
             const float r = F.nbrCount[c.i] < 20u ? 0.0f : fminf(-F.densAdv[c.i] - f, 0.0f);
             F.residuum[c.i] = r;
             F.kappaV[c.i] -= r * F.factor[c.i];
@@ -273,7 +194,7 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_div_final(const Sc
         const SceneParams& p = P[c.s];
         if (p.enableDiv) {
             const float dt = F.state[c.s].dt;
-            const f3 a = pressure_accel(p, K, F, cap, c.i, F.kappaV, src);
+            const f3 a = pressure_accel(p, K, F, cap, c.i, F.kappaV[c.i], LoadXS{F.pos, F.kappaV}, src);
             F.ap[c.i] = st4(a);
             F.vel[c.i] = st4(ld3(F.vel[c.i]) + dt * a);
             F.factor[c.i] *= dt;
@@ -317,7 +238,7 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_pres_init(const Sc
         if (!c.valid) return;
         const SceneParams& p = P[c.s];
         const SceneState& st = F.state[c.s];
-        const float d = velocity_divergence(p, K, F, cap, c.i, src);
+        const float d = field_divergence(p, K, F, cap, c.i, ld3(F.vel[c.i]), LoadXV{F.pos, F.vel}, src);
         const float da = F.density[c.i] / p.rho0 + st.dt * d;
         F.densAdv[c.i] = da;
         const float f = F.factor[c.i] * st.dt2Inv;
@@ -336,7 +257,7 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_pres_accel(const S
     group_loop<1>(tg, halo(F), rec, global_src(F, cap), LoadXS{F.pos, F.kappa}, [&](uint32_t tile, bool ok, const NbrSrc& src) {
         const TileCtx c = tile_ctx4(tile, ok, tileScene, P);
         if (!F.state[c.s].pres.active || !c.valid) return;
-        F.ap[c.i] = st4(pressure_accel(P[c.s], K, F, cap, c.i, F.kappa, src));
+        F.ap[c.i] = st4(pressure_accel(P[c.s], K, F, cap, c.i, F.kappa[c.i], LoadXS{F.pos, F.kappa}, src));
     });
 }
 
@@ -353,7 +274,7 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_pres_iter(const Sc
         const SceneParams& p = P[c.s];
         double part = 0.0;
         if (act && c.valid) {
-            const float f = density_pressure_force(p, K, F, cap, c.i, src) * st.dt2;
+            const float f = field_divergence(p, K, F, cap, c.i, ld3(F.ap[c.i]), LoadXV{F.pos, F.ap}, src) * st.dt2;
             const float r = fminf(1.0f - F.densAdv[c.i] - f, 0.0f);
             F.residuum[c.i] = r;
             F.kappa[c.i] -= r * F.factor[c.i];
@@ -367,14 +288,16 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_pres_iter(const Sc
 // ComputePressureAccelerationAndVelocityKernel (:434-481) + ComputePositionKernel (:54-67) into posNext
 __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_pres_final(const SceneParams* __restrict__ P,
                                                       const uint32_t* __restrict__ tileScene, KTabHost kh, Fields F,
-                                                      uint32_t cap, TileGrid tg, int writeNext) {
+                                                      uint32_t cap, TileGrid tg, int writeNext,
+                                                      const uint32_t* aborted) {
+    if (aborted && *aborted) writeNext = 0;  // the step is taken again from the old positions
     VFD_HALO_KERNEL_PROLOGUE(kh)
     group_loop<1>(tg, halo(F), rec, global_src(F, cap), LoadXS{F.pos, F.kappa}, [&](uint32_t tile, bool ok, const NbrSrc& src) {
         const TileCtx c = tile_ctx4(tile, ok, tileScene, P);
         if (!c.valid) return;
         const SceneParams& p = P[c.s];
         const float dt = F.state[c.s].dt;
-        const f3 a = pressure_accel(p, K, F, cap, c.i, F.kappa, src);
+        const f3 a = pressure_accel(p, K, F, cap, c.i, F.kappa[c.i], LoadXS{F.pos, F.kappa}, src);
         F.ap[c.i] = st4(a);
         const f3 v = ld3(F.vel[c.i]) + dt * a;
         F.vel[c.i] = st4(v);
@@ -401,9 +324,9 @@ void launch_pres_iter(const Launch& L, const KTabHost& kt, const Fields& F) {
     hipLaunchKernelGGL(k_pres_iter, dim3(L.gridGroups), dim3(kGroupSize), kLdsXV, L.stream, L.P, L.tileScene, kt, F, L.capacity,
                        TileGrid(L.tg));
 }
-void launch_pres_final(const Launch& L, const KTabHost& kt, const Fields& F, int writeNext) {
+void launch_pres_final(const Launch& L, const KTabHost& kt, const Fields& F, int writeNext, const uint32_t* aborted) {
     hipLaunchKernelGGL(k_pres_final, dim3(L.gridGroups), dim3(kGroupSize), kLdsXS, L.stream, L.P, L.tileScene, kt, F,
-                       L.capacity, TileGrid(L.tg), writeNext);
+                       L.capacity, TileGrid(L.tg), writeNext, aborted);
 }
 
 // ---- time step (ComputeTimeStepSize, DFSPHImplementation.cu:395-441) --------------------------------------------
@@ -486,70 +409,7 @@ void launch_velocity(const Launch& L, const Fields& F) {
     hipLaunchKernelGGL(k_velocity, dim3(L.gridAll), dim3(kTile), 0, L.stream, L.P, L.tileScene, F, TileGrid(L.tg));
 }
 
-// ---- implicit viscosity (ComputeViscosity, DFSPHImplementation.cu:577-615; Weiler et al. 2018) ------------------
-struct M3 {
-    float m[9];  // row-major
-};
-__device__ __forceinline__ M3 inverse3(const M3& A) {
-    const float a = A.m[0], b = A.m[1], c = A.m[2];
-    const float d = A.m[3], e = A.m[4], f = A.m[5];
-    const float g = A.m[6], h = A.m[7], i = A.m[8];
-    const float c00 = e * i - f * h, c01 = f * g - d * i, c02 = d * h - e * g;
-    const float det = a * c00 + b * c01 + c * c02;
-    const float s = 1.0f / det;
-    M3 r;
-    r.m[0] = c00 * s;
-    r.m[1] = (c * h - b * i) * s;
-    r.m[2] = (b * f - c * e) * s;
-    r.m[3] = c01 * s;
-    r.m[4] = (a * i - c * g) * s;
-    r.m[5] = (c * d - a * f) * s;
-    r.m[6] = c02 * s;
-    r.m[7] = (b * g - a * h) * s;
-    r.m[8] = (a * e - b * d) * s;
-    return r;
-}
-__device__ __forceinline__ f3 minv_mul(const float* __restrict__ minv, uint32_t cap, uint32_t i, f3 v) {
-    float m[9];
-#pragma unroll
-    for (int e = 0; e < 9; ++e) m[e] = minv[(size_t)e * cap + i];
-    return mk3(m[0] * v.x + m[1] * v.y + m[2] * v.z, m[3] * v.x + m[4] * v.y + m[5] * v.z,
-               m[6] * v.x + m[7] * v.y + m[8] * v.z);
-}
-
-// GetOrthogonalVectors (Core/Math/Math.h:19-33)
-__device__ __forceinline__ void orthogonal_vectors(f3 vec, f3& x, f3& y) {
-    f3 v = mk3(1.0f, 0.0f, 0.0f);
-    if ((double)fabsf(dot3(v, vec)) > 0.999) v = mk3(0.0f, 1.0f, 0.0f);
-    x = cross(vec, v);
-    y = cross(vec, x);
-    x = normalize(x);
-    y = normalize(y);
-}
-
-// four tangential boundary samples (DFSPHKernels.cu:643-671, 713-742, 800-829)
-struct Tangential {
-    f3 pd[4];
-    f3 gw[4];
-    float vol;
-};
-__device__ __forceinline__ bool tangential(const SceneParams& p, const KLds& k, f3 xi, f3 xb, float vb, Tangential& t) {
-    f3 normal = -(xi - xb);
-    const float nl = length(normal);
-    if (!(nl > 0.0001f)) return false;
-    normal = normal / nl;
-    f3 t1, t2;
-    orthogonal_vectors(normal, t1, t2);
-    const f3 pos[4] = {xb - t1 * p.td, xb + t1 * p.td, xb - t2 * p.td, xb + t2 * p.td};
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        t.pd[q] = xi - pos[q];
-        t.gw[q] = gradW(k, t.pd[q]);
-    }
-    t.vol = 0.25f * vb;
-    return true;
-}
-
+// ---- implicit viscosity (ComputeViscosity, DFSPHImplementation.cu:577-615; Weiler et al. 2018; terms.h) ----------
 // ComputeViscosityPreconditionerKernel (:604-684) + ComputeViscosityGradientKernel (:686-756): inverse diagonal
 // block, right-hand side b = v (the boundary rhs term is dot(0, .) = 0) and initial guess x0 = v + dv.
 __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_visc_precond(const SceneParams* __restrict__ P,
@@ -561,82 +421,11 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_visc_precond(const
         const TileCtx c = tile_ctx4(tile, ok, tileScene, P);
         const SceneParams& p = P[c.s];
         if (!c.valid || !p.enableVisc) return;
-        const f3 xi = ld3(F.pos[c.i]);
-        const float d001 = 0.01f * p.R2;
-        const float mu10 = 10.0f * p.mu;  // read before the loop (see pressure_accel)
-        float M[9];
-#pragma unroll
-        for (int e = 0; e < 9; ++e) M[e] = 0.0f;
-        each_neighbor_rec<1>(src, c.i, K.R, K.invStep, xi, K.sG, load, [&](float4 lo, float4, float gt) {
-            const f3 xij = xi - ld3(lo);
-            const f3 gw = gt * xij;
-            const float s = mu10 * lo.w / (length2(xij) + d001);
-            const float a[3] = {xij.x, xij.y, xij.z}, g[3] = {gw.x, gw.y, gw.z};
-#pragma unroll
-            for (int r = 0; r < 3; ++r)
-#pragma unroll
-                for (int cc = 0; cc < 3; ++cc) M[3 * r + cc] += s * (a[r] * g[cc]);
-        });
-        if (p.muB != 0.0f) {
-            for (uint32_t b = 0; b < p.bodyCount; ++b) {
-                const float vb = F.vb[(size_t)b * cap + c.i];
-                if (!(vb > 0.0f)) continue;
-                Tangential t;
-                if (!tangential(p, K, xi, ld3(F.xb[(size_t)b * cap + c.i]), vb, t)) continue;
-                const float a[3] = {t.pd[0].x, t.pd[0].y, t.pd[0].z};  // the reference uses direction 1 for all four
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float s = 10.0f * p.muB * t.vol / (length2(t.pd[q]) + d001);
-                    const float g[3] = {t.gw[q].x, t.gw[q].y, t.gw[q].z};
-#pragma unroll
-                    for (int r = 0; r < 3; ++r)
-#pragma unroll
-                        for (int cc = 0; cc < 3; ++cc) M[3 * r + cc] += s * (a[r] * g[cc]);
-                }
-            }
-        }
-        const float f = F.state[c.s].dt / F.density[c.i];
-        M3 A;
-#pragma unroll
-        for (int e = 0; e < 9; ++e) A.m[e] = (e % 4 == 0 ? 1.0f : 0.0f) - f * M[e];
-        const M3 inv = inverse3(A);
+        const M3 inv = visc_precond(p, K, F, cap, c.i, F.state[c.s].dt, load, src);
 #pragma unroll
         for (int e = 0; e < 9; ++e) F.minv[(size_t)e * cap + c.i] = inv.m[e];
         F.cgX[c.i] = st4(ld3(F.vel[c.i]) + ld3(F.dv[c.i]));
     });
-}
-
-// ComputeMatrixVecProdFunctionKernel (:758-842): y_i = x_i - dt/rho_i * (viscous acceleration of x)
-// records lo = {x_j, m / rho_j}, hi = {in_j}
-__device__ __forceinline__ f3 visc_matvec(const SceneParams& p, const KLds& k, const Fields& F, uint32_t cap,
-                                          uint32_t i, const float4* __restrict__ in, float dt, const NbrSrc& src,
-                                          const LoadXQV& load) {
-    const f3 xi = ld3(F.pos[i]), vi = ld3(in[i]);
-    const float d001 = 0.01f * p.R2;
-    const float mu10 = 10.0f * p.mu;  // read before the loop (see pressure_accel)
-    f3 acc = mk3(0.0f, 0.0f, 0.0f);
-    each_neighbor_rec<2>(src, i, k.R, k.invStep, xi, k.sG, load, [&](float4 lo, float4 hi, float g) {
-        const f3 xij = xi - ld3(lo);
-        const f3 gw = g * xij;
-        const float s = mu10 * lo.w * dot3(vi - ld3(hi), xij) / (length2(xij) + d001);
-        acc = acc + s * gw;
-    });
-    if (p.muB != 0.0f) {
-        for (uint32_t b = 0; b < p.bodyCount; ++b) {
-            const float vb = F.vb[(size_t)b * cap + i];
-            if (!(vb > 0.0f)) continue;
-            Tangential t;
-            if (!tangential(p, k, xi, ld3(F.xb[(size_t)b * cap + i]), vb, t)) continue;
-            f3 s4;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float s = 10.0f * p.muB * t.vol * dot3(vi, t.pd[q]) / (length2(t.pd[q]) + d001);
-                s4 = q == 0 ? s * t.gw[q] : s4 + s * t.gw[q];
-            }
-            acc = acc + s4;
-        }
-    }
-    return vi - (dt / F.density[i]) * acc;
 }
 
 // SolveViscosity set-up (DFSPHImplementation.cu:627-691): r = b - A x0, ||b||^2, ||r||^2, p = M^-1 r, |r.p|
@@ -653,7 +442,7 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_cg_begin(const Sce
         double v[3] = {0.0, 0.0, 0.0};
         if (act && c.valid) {
             const f3 b = ld3(F.vel[c.i]);
-            const f3 ax = visc_matvec(p, K, F, cap, c.i, F.cgX, st.dt, src, load);
+            const f3 ax = visc_matvec(p, K, F, cap, c.i, ld3(F.cgX[c.i]), st.dt, load, src);
             const f3 r = b - ax;
             const f3 z = minv_mul(F.minv, cap, c.i, r);
             F.cgR[c.i] = st4(r);
@@ -708,7 +497,7 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_cg_matvec(const Sc
         const bool act = ok && st.cg.active;
         double v[1] = {0.0};
         if (act && c.valid) {
-            const f3 ap = visc_matvec(P[c.s], K, F, cap, c.i, F.cgP, st.dt, src, load);
+            const f3 ap = visc_matvec(P[c.s], K, F, cap, c.i, ld3(F.cgP[c.i]), st.dt, load, src);
             F.cgAp[c.i] = st4(ap);
             v[0] = (double)dot3(ld3(F.cgP[c.i]), ap);
         }
@@ -990,6 +779,6 @@ int configure_kernels() {
     };
     for (const auto& e : k)
         if (hipFuncSetAttribute(e.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)e.bytes) != hipSuccess) return 1;
-    return configure_search_kernels() || configure_adjoint_kernels();
+    return configure_search_kernels() || configure_solve_kernels() || configure_adjoint_kernels();
 }
 }  // namespace vfd

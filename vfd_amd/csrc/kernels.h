@@ -169,6 +169,7 @@ struct KTabHost {
 // ---- search.hip -----------------------------------------------------------------------------------------------
 uint32_t scan_scratch_words(uint32_t n);
 void exclusive_scan(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* scratch, hipStream_t st);
+void launch_fill_u32(hipStream_t st, uint32_t* p, uint32_t v, uint32_t n);
 void launch_minmax(const Launch& L, const float4* pos, int* part, int* mm);
 void launch_sort(const Launch& L, const SceneGrid* G, uint32_t totalCells, const float4* posIn, const float4* velIn,
                  const float4* dvIn, const float* dkIn, const uint32_t* idIn, float4* posOut, float4* velOut,
@@ -282,7 +283,25 @@ void launch_scene_init_pres(const Launch& L, const Fields& F);
 void launch_pres_init(const Launch& L, const KTabHost& kt, const Fields& F);
 void launch_pres_accel(const Launch& L, const KTabHost& kt, const Fields& F);
 void launch_pres_iter(const Launch& L, const KTabHost& kt, const Fields& F);
-void launch_pres_final(const Launch& L, const KTabHost& kt, const Fields& F, int writeNext);
+// aborted (null: none): positions are not written when *aborted is set
+void launch_pres_final(const Launch& L, const KTabHost& kt, const Fields& F, int writeNext, const uint32_t* aborted);
+// ---- solve.hip: whole solves as one launch ----------------------------------------------------------------------
+constexpr uint32_t kResidentScenes = 256;        // scenes of a resident solve (their scalars live in LDS)
+constexpr uint32_t kResidentTiles = kGroupSize;  // tiles: a thread each when a block adds up a scene's partials
+// Barrier words (32-bit), zero between launches; words[kResidentAbortedAt] is set when a solve was aborted, and then
+// the host clears all of them.
+constexpr uint32_t kResidentWords = 1024, kResidentAbortedAt = 18 * 32;
+struct Resident {
+    uint32_t* words;
+    uint32_t waitTicks;  // longest wait at a barrier, in ticks of the 100 MHz wall clock
+};
+// every group of the simulation has a block of its own on numCU CUs
+bool resident_fits(const Launch& L, uint32_t numCU);
+void launch_div_solve(const Launch& L, const KTabHost& kt, const Fields& F, const Resident& r);
+void launch_pres_solve(const Launch& L, const KTabHost& kt, const Fields& F, const Resident& r, int writeNext);
+void launch_visc_solve(const Launch& L, const KTabHost& kt, const Fields& F, const Resident& r,
+                       const uint32_t* haloStats);
+int configure_solve_kernels();
 void launch_scene_state_init(const Launch& L, SceneState* state, const float* dt0);
 
 }  // namespace vfd

@@ -527,6 +527,10 @@ void exclusive_scan(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* scr
     hipLaunchKernelGGL(k_scan_add, dim3(chunks), dim3(kScanThreads), 0, st, out, (const uint32_t*)scratch, n);
 }
 
+void launch_fill_u32(hipStream_t st, uint32_t* p, uint32_t v, uint32_t n) {
+    if (n) hipLaunchKernelGGL(k_fill_u32, dim3((n + 255) / 256), dim3(256), 0, st, p, v, n);
+}
+
 // ---- host launchers ---------------------------------------------------------------------------------------------
 void launch_minmax(const Launch& L, const float4* pos, int* part, int* mm) {
     hipLaunchKernelGGL(k_minmax, dim3(L.tiles), dim3(kTile), 0, L.stream, pos, L.P, L.tileScene, part);

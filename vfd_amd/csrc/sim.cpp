@@ -17,6 +17,7 @@
 #include <climits>
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <deque>
 #include <memory>
@@ -535,6 +536,17 @@ public:
     // (with SolverCheckInterval 1 or 2), within run-to-run noise.
     bool predictIterations = VFD_DEFAULT_PREDICT_ITERATIONS != 0;
     uint32_t lastIterations[3] = {0, 0, 0};
+    // Resident solvers (solve.hip): used when every neighbour group has a block of its own and UseGraphs is on. After
+    // an aborted one (other work held the CUs past the barrier's limit) the step is taken again with launched
+    // iterations, and so are the next kResidentPause steps.
+    DevBuf<uint32_t> residentWords;
+    uint32_t* hostAborted = nullptr;  // pinned
+    uint32_t residentPause = 0;
+    static constexpr uint32_t kResidentPause = 64;
+    // longest wait at a resident solve's barrier: 100 ms, or VFD_RESIDENT_WAIT_US from the environment (the aborted
+    // solves of a short limit are a testing aid; results do not depend on it)
+    uint32_t residentWait = 10000000;
+    Resident resident_words() const { return Resident{residentWords.p, residentWait}; }
     hipStream_t ownStream = nullptr;  // default stream (capture needs a stream other than the legacy null stream)
     // frame output: frames are packed in original order on the simulation's stream into one of two device staging
     // buffers and copied to pinned host memory on copyStream, so that the copy overlaps the next steps
@@ -732,7 +744,10 @@ public:
         for (auto& e : ev) VFD_HIP(hipEventCreate(&e));
         for (auto& e : pollEv) VFD_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         eventsMade = true;
-        VFD_HIP(hipHostMalloc((void**)&hostLive, 2 * sizeof(uint32_t), hipHostMallocDefault));
+        VFD_HIP(hipHostMalloc((void**)&hostLive, 4 * sizeof(uint32_t), hipHostMallocDefault));
+        hostAborted = hostLive + 2;
+        if (const char* us = std::getenv("VFD_RESIDENT_WAIT_US"))
+            residentWait = (uint32_t)std::min(std::max(std::atol(us), 0L), 1000000L) * 100u;
         VFD_HIP(hipStreamCreateWithFlags(&ownStream, hipStreamNonBlocking));
         stream = ownStream;
         VFD_HIP(hipStreamCreateWithFlags(&copyStream, hipStreamNonBlocking));
@@ -990,6 +1005,8 @@ public:
         VFD_TRY(dMM.alloc((size_t)S * 6));
         VFD_TRY(dMMPart.alloc((size_t)std::max<uint32_t>(tiles, 1) * 6));
         VFD_TRY(live.alloc(4));
+        VFD_TRY(residentWords.alloc(kResidentWords));
+        VFD_HIP(hipMemset(residentWords.p, 0, kResidentWords * sizeof(uint32_t)));
         VFD_TRY(dTileScene.alloc(std::max<uint32_t>(tiles, 1)));
         DevBuf<float4>* f4[] = {&pos, &posNext, &vel[0], &vel[1], &dv[0], &dv[1], &acc, &ap, &nMC, &nS,
                                 &cgX, &cgR, &cgP, &cgZ, &cgAp};
@@ -1248,6 +1265,33 @@ public:
     int step(int last) {
         if (!committed) VFD_TRY(commit());
         if (tiles == 0) return VFD_OK;  // OnUpdate returns for N = 0 (:65-67)
+        bool resident = useGraphs && residentPause == 0 && resident_fits(launch(), numCU);
+        if (residentPause) --residentPause;
+        const int before = cur;
+        const size_t records = tapeCount;
+        int rc = step_once(last, resident);
+        if (rc == kStepAborted) {  // the state the step started from is still whole: posNext, [before] and the host's
+            residentPause = kResidentPause;
+            cur = before;
+            tapeCount = records;
+            launch_fill_u32(stream, residentWords.p, 0u, kResidentWords);
+            VFD_TRY(push_state());
+            rc = step_once(last, false);
+        }
+        return rc;
+    }
+    static constexpr int kStepAborted = -1;
+    // waits for the step's launches; kStepAborted when a resident solve was aborted
+    int drain(bool resident) {
+        *hostAborted = 0;
+        if (resident)
+            VFD_HIP(hipMemcpyAsync(hostAborted, residentWords.p + kResidentAbortedAt, sizeof(uint32_t),
+                                   hipMemcpyDeviceToHost, stream));
+        VFD_HIP(hipStreamSynchronize(stream));
+        return *hostAborted ? kStepAborted : VFD_OK;
+    }
+    int step_once(int last, bool resident) {
+        const bool residentJacobi = resident && !taping;  // (a recorded solve stores every iteration)
         const Launch L = launch();
         const KTabHost K = ktab();
         bool anyST = false, anyVisc = false;
@@ -1261,7 +1305,7 @@ public:
         VFD_HIP(hipEventRecord(ev[0], stream));
         VFD_TRY(search());
         VFD_HIP(hipEventRecord(ev[1], stream));
-        if (last == VFD_PHASE_SEARCH) return finish_partial();
+        if (last == VFD_PHASE_SEARCH) return finish_partial(resident);
         Fields F = fields();
         if (taping) VFD_TRY(tape_copy(tapeXpre, pos.p, cap));
         VFD_TRY(timed("boundary", [&] { launch_boundary(L, dMaps.p, pos.p, vel[cur].p, xb.p, vb.p); }));
@@ -1271,7 +1315,7 @@ public:
             launch_build_halo(L, nbrCount.p, nbrList.p, haloLimit, haloCount.p, haloIds.p, nbrLocal.p, haloStats.p,
                               pos.p, K);
         }));
-        if (last == VFD_PHASE_BOUNDARY) return finish_partial();
+        if (last == VFD_PHASE_BOUNDARY) return finish_partial(resident);
         DevTape* tp = nullptr;
         if (taping) {
             if (tapeCount == tapes.size()) tapes.emplace_back(new DevTape());
@@ -1316,25 +1360,29 @@ public:
             VFD_TRY(tape_copy(tp->alpha, factor.p, tp->n));
         }
         VFD_HIP(hipEventRecord(ev[2], stream));
-        if (last == VFD_PHASE_DENSITY || last == VFD_PHASE_FACTOR) return finish_partial();
+        if (last == VFD_PHASE_DENSITY || last == VFD_PHASE_FACTOR) return finish_partial(resident);
         // divergence solve (ComputeDivergence :506-575)
-        launch_scene_init_div(L, F);
-        VFD_TRY(timed("div_init", [&] { launch_div_init(L, K, F); }));
-        if (tp) VFD_TRY(tape_copy(tp->D, densAdv.p, tp->n));
-        VFD_TRY(poll_loop(
-            [&](uint32_t k) {
-                if (tp && k == 0) (void)tape_slot(tp->kv, 0, kappaV.p, tp->n);
-                (void)timed("div_accel", [&] { launch_div_accel(L, K, F); }, 0, k);
-                (void)timed("div_iter", [&] { launch_div_iter(L, K, F); }, 0, k);
-                (void)timed("jacobi_finish", [&] { launch_jacobi_finish(L, F, 0); }, 0, k);
-                if (tp) (void)tape_iteration(tp->kv, tp->av, tp->rv, k, tp->n, kappaV.p, ap.p, residuum.p);
-            },
-            minDiv, 0));
-        if (tp) VFD_TRY(tape_copy(tp->kvEnd, kappaV.p, tp->n));
-        VFD_TRY(timed("div_final", [&] { launch_div_final(L, K, F); }));  // also ClearAccelerationKernel
+        if (residentJacobi) {
+            VFD_TRY(timed("div_solve", [&] { launch_div_solve(L, K, F, resident_words()); }));
+        } else {
+            launch_scene_init_div(L, F);
+            VFD_TRY(timed("div_init", [&] { launch_div_init(L, K, F); }));
+            if (tp) VFD_TRY(tape_copy(tp->D, densAdv.p, tp->n));
+            VFD_TRY(poll_loop(
+                [&](uint32_t k) {
+                    if (tp && k == 0) (void)tape_slot(tp->kv, 0, kappaV.p, tp->n);
+                    (void)timed("div_accel", [&] { launch_div_accel(L, K, F); }, 0, k);
+                    (void)timed("div_iter", [&] { launch_div_iter(L, K, F); }, 0, k);
+                    (void)timed("jacobi_finish", [&] { launch_jacobi_finish(L, F, 0); }, 0, k);
+                    if (tp) (void)tape_iteration(tp->kv, tp->av, tp->rv, k, tp->n, kappaV.p, ap.p, residuum.p);
+                },
+                minDiv, 0));
+            if (tp) VFD_TRY(tape_copy(tp->kvEnd, kappaV.p, tp->n));
+            VFD_TRY(timed("div_final", [&] { launch_div_final(L, K, F); }));  // also ClearAccelerationKernel
+        }
         if (tp) VFD_TRY(tape_copy(tp->v1, vel[cur].p, tp->n));
         VFD_HIP(hipEventRecord(ev[3], stream));
-        if (last == VFD_PHASE_DIVERGENCE || last == VFD_PHASE_CLEAR_ACCELERATION) return finish_partial();
+        if (last == VFD_PHASE_DIVERGENCE || last == VFD_PHASE_CLEAR_ACCELERATION) return finish_partial(resident);
         if (anyST) {
             if (tp && tp->stTemporal) VFD_TRY(tape_copy(tp->dK0, dk[cur].p, tp->n));
             VFD_TRY(upload_mc_tables(F));
@@ -1345,8 +1393,10 @@ public:
             VFD_TRY(tape_copy(tp->kMC, kMC.p, tp->n));
         }
         VFD_HIP(hipEventRecord(ev[4], stream));
-        if (last == VFD_PHASE_SURFACE_TENSION) return finish_partial();
-        if (anyVisc) {
+        if (last == VFD_PHASE_SURFACE_TENSION) return finish_partial(resident);
+        if (anyVisc && resident) {
+            VFD_TRY(timed("visc_solve", [&] { launch_visc_solve(L, K, F, resident_words(), haloStats.p); }));
+        } else if (anyVisc) {
             VFD_TRY(timed("visc_precond", [&] { launch_visc_precond(L, K, F); }));
             VFD_TRY(timed("cg_begin", [&] { launch_cg_begin(L, K, F); }));
             VFD_TRY(timed("cg_begin_finish", [&] { launch_cg_begin_finish(L, F); }));
@@ -1360,34 +1410,43 @@ public:
                 },
                 minVisc, 2));
             VFD_TRY(timed("visc_apply", [&] { launch_visc_apply(L, F); }));
-            if (tp) VFD_TRY(tape_copy(tp->y, cgX.p, tp->n));
         }
+        if (tp && anyVisc) VFD_TRY(tape_copy(tp->y, cgX.p, tp->n));
         VFD_HIP(hipEventRecord(ev[5], stream));
-        if (last == VFD_PHASE_VISCOSITY) return finish_partial();
+        if (last == VFD_PHASE_VISCOSITY) return finish_partial(resident);
         VFD_TRY(timed("time_step", [&] { launch_time_step(L, F); }));
         VFD_TRY(timed("time_step_finish", [&] { launch_time_step_finish(L, F); }));
-        if (last == VFD_PHASE_TIME_STEP) return finish_partial();
+        if (last == VFD_PHASE_TIME_STEP) return finish_partial(resident);
         VFD_TRY(timed("velocity", [&] { launch_velocity(L, F); }));
         if (tp) VFD_TRY(tape_copy(tp->v2, vel[cur].p, tp->n));
-        if (last == VFD_PHASE_VELOCITY) return finish_partial();
-        launch_scene_init_pres(L, F);
-        VFD_TRY(timed("pres_init", [&] { launch_pres_init(L, K, F); }));
-        if (tp) VFD_TRY(tape_copy(tp->rhoadv, densAdv.p, tp->n));
-        VFD_TRY(poll_loop(
-            [&](uint32_t k) {
-                if (tp && k == 0) (void)tape_slot(tp->kp, 0, kappa.p, tp->n);
-                (void)timed("pres_accel", [&] { launch_pres_accel(L, K, F); }, 1, k);
-                (void)timed("pres_iter", [&] { launch_pres_iter(L, K, F); }, 1, k);
-                (void)timed("jacobi_finish", [&] { launch_jacobi_finish(L, F, 1); }, 1, k);
-                if (tp) (void)tape_iteration(tp->kp, tp->ap, tp->rp, k, tp->n, kappa.p, ap.p, residuum.p);
-            },
-            minPres, 1));
-        if (tp) VFD_TRY(tape_copy(tp->kpEnd, kappa.p, tp->n));
-        VFD_TRY(timed("pres_final", [&] { launch_pres_final(L, K, F, last >= VFD_PHASE_POSITION ? 1 : 0); }));
+        if (last == VFD_PHASE_VELOCITY) return finish_partial(resident);
+        if (residentJacobi) {
+            VFD_TRY(timed("pres_solve", [&] {
+                launch_pres_solve(L, K, F, resident_words(), last >= VFD_PHASE_POSITION ? 1 : 0);
+            }));
+        } else {
+            launch_scene_init_pres(L, F);
+            VFD_TRY(timed("pres_init", [&] { launch_pres_init(L, K, F); }));
+            if (tp) VFD_TRY(tape_copy(tp->rhoadv, densAdv.p, tp->n));
+            VFD_TRY(poll_loop(
+                [&](uint32_t k) {
+                    if (tp && k == 0) (void)tape_slot(tp->kp, 0, kappa.p, tp->n);
+                    (void)timed("pres_accel", [&] { launch_pres_accel(L, K, F); }, 1, k);
+                    (void)timed("pres_iter", [&] { launch_pres_iter(L, K, F); }, 1, k);
+                    (void)timed("jacobi_finish", [&] { launch_jacobi_finish(L, F, 1); }, 1, k);
+                    if (tp) (void)tape_iteration(tp->kp, tp->ap, tp->rp, k, tp->n, kappa.p, ap.p, residuum.p);
+                },
+                minPres, 1));
+            if (tp) VFD_TRY(tape_copy(tp->kpEnd, kappa.p, tp->n));
+            VFD_TRY(timed("pres_final", [&] {
+                launch_pres_final(L, K, F, last >= VFD_PHASE_POSITION ? 1 : 0,
+                                  resident ? residentWords.p + kResidentAbortedAt : nullptr);
+            }));
+        }
         VFD_HIP(hipEventRecord(ev[6], stream));
-        if (last == VFD_PHASE_PRESSURE) return finish_partial();
+        if (last == VFD_PHASE_PRESSURE) return finish_partial(resident);
         VFD_HIP(hipGetLastError());
-        VFD_HIP(hipStreamSynchronize(stream));
+        VFD_TRY(drain(resident));
         std::unique_lock<std::mutex> lk(hostMu);  // the host bookkeeping that polling threads read
         VFD_TRY(pull_state());
         solver_debug();
@@ -1651,7 +1710,8 @@ public:
     }
 
     // after a partial step the working positions become the state the next step starts from
-    int finish_partial() {
+    int finish_partial(bool resident) {
+        VFD_TRY(drain(resident));
         VFD_HIP(hipMemcpyAsync(posNext.p, pos.p, (size_t)cap * sizeof(float4), hipMemcpyDeviceToDevice, stream));
         VFD_HIP(hipGetLastError());
         VFD_HIP(hipStreamSynchronize(stream));
