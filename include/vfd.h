@@ -139,7 +139,8 @@ typedef struct vfd_debug_info {
     float MaxVelocityMagnitude;
     uint32_t MaxNeighborCount;
     uint64_t TotalNeighborCount;
-    uint32_t StagedGroupCount;   /* neighbour groups of the whole simulation whose halo was staged in LDS */
+    uint32_t StagedGroupCount;   /* neighbour groups (of 256 to 1024 particles, by the simulation's size) whose halo was
+                                    staged in LDS, whole simulation */
     uint32_t GatheredGroupCount; /* groups whose halo exceeded the limit (neighbour data gathered from HBM) */
     uint32_t MaxHaloSize;        /* distinct neighbours of the largest staged group */
 } vfd_debug_info;
@@ -425,7 +426,9 @@ int vfd_batch_adjoint(vfd_sim* sim, uint32_t scene, const float* lx_out, const f
 typedef struct vfd_tuning {
     uint32_t SolverCheckInterval; /* Jacobi / CG iterations enqueued between two convergence checks, >= 1 */
     uint32_t HaloLimit;           /* largest group halo staged in LDS (<= 3808); 0: every neighbour from HBM */
-    uint32_t UseGraphs;           /* 1: each chunk of iterations is one launch of a captured HIP graph */
+    uint32_t UseGraphs;           /* 1: each chunk of iterations is one launch of a captured HIP graph, and in a
+                                     simulation of at most 1024 particles per compute unit each solve is one launch;
+                                     0: every kernel of an iteration is launched by itself */
     uint32_t PredictIterations;   /* 1: a solver's first chunk is one iteration short of what it ran in the
                                      previous step, so that few empty iterations follow its convergence (default 0) */
     uint32_t AdjointGroupLoops;   /* vfd_adjoint's transposed neighbour loops (the pressure solves' and the

@@ -54,8 +54,14 @@ constexpr unsigned kGroupSize = kTile * kGroupTiles;
 constexpr unsigned kHaloMax = VFD_HALO_MAX;
 constexpr unsigned kGroupsPerCU = VFD_GROUPS_PER_CU;
 static_assert(kGroupTiles == 1 || kGroupTiles == 2 || kGroupTiles == 4, "a group is 1, 2 or 4 tiles");
-static_assert(kHaloMax <= 4 * kGroupSize && kHaloMax <= 65535, "halo slots are 16-bit, filled four per thread");
+static_assert(kHaloMax <= 65535, "halo slots are 16-bit");
 constexpr uint32_t kHaloNone = 0xFFFFFFFFu;
+// Halo entries each thread of a `tiles`-tile group copies, and the largest halo that a group of that size stages.
+constexpr unsigned halo_fill(unsigned tiles) { return tiles >= 4 ? 4u : 8u; }
+constexpr unsigned halo_cap(unsigned tiles) {
+    return halo_fill(tiles) * tiles * kTile < kHaloMax ? halo_fill(tiles) * tiles * kTile : kHaloMax;
+}
+static_assert(halo_cap(kGroupTiles) == kHaloMax, "a launched group's fill covers its halo");
 
 // Constant per-scene parameters (DFSPHSimulationInfo + DFSPHSimulationDescription, DFSPHImplementation.cu:318-368).
 struct SceneParams {

@@ -396,11 +396,29 @@ struct NbrSrc {
     uint32_t cap;
 };
 
+#ifndef VFD_LIST_CHUNK
+#define VFD_LIST_CHUNK 8
+#endif
+#ifndef VFD_LIST_PREFETCH
+#define VFD_LIST_PREFETCH 1
+#endif
+#ifndef VFD_LIST_CHUNK2
+#define VFD_LIST_CHUNK2 4
+#endif
+#ifndef VFD_LIST_PREFETCH2
+#define VFD_LIST_PREFETCH2 1
+#endif
+template <int R> struct ListShape {
+    static constexpr uint32_t chunk = R == 1 ? VFD_LIST_CHUNK : VFD_LIST_CHUNK2;
+    static constexpr uint32_t depth = 1u + (R == 1 ? VFD_LIST_PREFETCH : VFD_LIST_PREFETCH2);  // chunks in flight
+};
 // Cache policy bits of a buffer load on gfx950: bit 1 = non-temporal.
 constexpr int kBufferNonTemporal = 2;
+// What a loader's kernel wants of its neighbour loop besides the records.
 struct LoadTraits {
     static constexpr int kListCache = kBufferNonTemporal;  // policy of the staged list's loads: read once per launch
     static constexpr bool kAlwaysSplit = false;            // HaloRec's 16 + 8 byte form whatever VFD_PACK_RECORDS says
+    template <int R> using Shape = ListShape<R>;           // chunk length and chunks in flight
 };
 
 struct LoadX : LoadTraits {  // lo = hi = {x_t, -}
@@ -492,22 +510,6 @@ struct LoadXSV : LoadTraits {  // lo = {x_t, s_t}, hi = {v_t, -}
 // chunks; two-record loops hold twice the registers per entry and take short ones. VFD_LIST_PREFETCH(2) is the
 // number of further chunks whose list loads are in flight while a chunk is consumed (0: none), since the list
 // latency, not the LDS, bounds these loops at one 1024-thread block per CU.
-#ifndef VFD_LIST_CHUNK
-#define VFD_LIST_CHUNK 8
-#endif
-#ifndef VFD_LIST_PREFETCH
-#define VFD_LIST_PREFETCH 1
-#endif
-#ifndef VFD_LIST_CHUNK2
-#define VFD_LIST_CHUNK2 4
-#endif
-#ifndef VFD_LIST_PREFETCH2
-#define VFD_LIST_PREFETCH2 1
-#endif
-template <int R> struct ListShape {
-    static constexpr uint32_t chunk = R == 1 ? VFD_LIST_CHUNK : VFD_LIST_CHUNK2;
-    static constexpr uint32_t depth = 1u + (R == 1 ? VFD_LIST_PREFETCH : VFD_LIST_PREFETCH2);  // chunks in flight
-};
 // Halo records in LDS, as two arrays of kHaloMax records: lo of slot s at rec[L * s], hi at rec[L * kHaloMax + H * s]
 // (H = 0 for one-record loops). With VFD_PACK_RECORDS a half that the neighbour terms read as three floats is stored
 // in 12 bytes (L or H = 3), which spreads a wave's random reads over all 32 banks instead of 8 groups of 4; otherwise
@@ -573,7 +575,7 @@ constexpr uint32_t kBufferOutOfRange = 0x80000000u;
 template <int R, class TV, class Load, class Fn>
 __device__ __forceinline__ void each_neighbor_rec(const NbrSrc& src, uint32_t i, float cutR, float invStep, f3 xi,
                                                   const TV* tab, const Load& load, Fn&& f) {
-    constexpr uint32_t C = ListShape<R>::chunk;
+    constexpr uint32_t C = Load::template Shape<R>::chunk;
     const uint32_t n = src.count[i];
     const size_t cap = src.cap;
     uint32_t j = 0;
@@ -625,7 +627,7 @@ __device__ __forceinline__ void each_neighbor_rec(const NbrSrc& src, uint32_t i,
         // The requests are unconditional (rows past a list's end are out-of-range reads that return 0): under a
         // per-lane condition the compiler cannot count the loads in flight and waits for all of them, the prefetch
         // included, before the current chunk's first use.
-        constexpr uint32_t D = ListShape<R>::depth;
+        constexpr uint32_t D = Load::template Shape<R>::depth;
         uint32_t e[D][C];
 #pragma unroll
         for (uint32_t k = 0; k + 1 < D; ++k) fetch(e[k], k * C);
@@ -665,36 +667,34 @@ struct HaloView {
 // the tiles it owns, so that its L2 holds the data of one contiguous stretch of the Morton order. For a staged group
 // every thread first copies halo records to LDS; body(tile, ok, src) is then called by every thread of the block
 // (ok = false past the last tile) and may contain block barriers.
-template <int R, class Load, class Body>
+// kTiles: tiles per group (kTiles * kTile threads per block).
+template <int R, unsigned kTiles = kGroupTiles, class Load, class Body>
 __device__ __forceinline__ void group_loop(const TileGrid& tg, const HaloView& H, float* rec, const NbrSrc& global,
                                            const Load& load, Body&& body) {
+    constexpr uint32_t kThreads = kTiles * kTile, kFill = halo_fill(kTiles);
     const uint32_t sub = threadIdx.x / kTile;
-    const uint32_t perG = tg.per / kGroupTiles;
+    const uint32_t perG = tg.per / kTiles;
     for (uint32_t q = blockIdx.x; q < 8u * perG; q += gridDim.x) {
         const uint32_t g = (q & 7u) * perG + (q >> 3);
-        if (g * kGroupTiles >= tg.tiles) continue;  // block-uniform
-        const uint32_t tile = g * kGroupTiles + sub;
+        if (g * kTiles >= tg.tiles) continue;  // block-uniform
+        const uint32_t tile = g * kTiles + sub;
         const uint32_t m = H.count[g];
         if (m <= kHaloMax) {
-            // every thread copies up to four records: the four slot loads first (indices past the halo repeat its
-            // last entry, so they stay in bounds), then the four record gathers, then the LDS stores
-            static_assert(kHaloMax <= 4 * kGroupSize, "fill covers four records per thread");
+            // every thread copies up to kFill records: the slot loads first (indices past the halo repeat its last
+            // entry, so they stay in bounds), then the record gathers, then the LDS stores
             if (m) {
                 const uint32_t* ids = H.ids + (size_t)g * kHaloMax;
-                const uint32_t k0 = threadIdx.x, k1 = k0 + kGroupSize, k2 = k1 + kGroupSize, k3 = k2 + kGroupSize;
-                const uint32_t mm = m - 1u;
-                const uint32_t t0 = ids[min(k0, mm)], t1 = ids[min(k1, mm)];
-                const uint32_t t2 = ids[min(k2, mm)], t3 = ids[min(k3, mm)];
-                float4 lo0, hi0, lo1, hi1, lo2, hi2, lo3, hi3;
-                load(t0, lo0, hi0);
-                if (k1 < m) load(t1, lo1, hi1);
-                if (k2 < m) load(t2, lo2, hi2);
-                if (k3 < m) load(t3, lo3, hi3);
-                auto put = [&](uint32_t k, const float4& lo, const float4& hi) { HaloRec<Load>::store(rec, k, lo, hi); };
-                if (k0 < m) put(k0, lo0, hi0);
-                if (k1 < m) put(k1, lo1, hi1);
-                if (k2 < m) put(k2, lo2, hi2);
-                if (k3 < m) put(k3, lo3, hi3);
+                uint32_t t[kFill];
+                float4 lo[kFill], hi[kFill];
+#pragma unroll
+                for (uint32_t u = 0; u < kFill; ++u) t[u] = ids[min(threadIdx.x + u * kThreads, m - 1u)];
+#pragma unroll
+                for (uint32_t u = 0; u < kFill; ++u)
+                    if (u == 0 || threadIdx.x + u * kThreads < m) load(t[u], lo[u], hi[u]);
+#pragma unroll
+                for (uint32_t u = 0; u < kFill; ++u)
+                    if (threadIdx.x + u * kThreads < m)
+                        HaloRec<Load>::store(rec, threadIdx.x + u * kThreads, lo[u], hi[u]);
             }
             __syncthreads();
             NbrSrc src = global;

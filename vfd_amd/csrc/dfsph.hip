@@ -26,7 +26,8 @@ static_assert(kLdsDensity <= 160 * 1024 && kLdsXS <= 160 * 1024 && kLdsXV <= 160
 
 // ---- ComputeDensityKernel (DFSPHKernels.cu:152-187) + ComputeDFSPHFactorKernel (:189-231) ----------------------
 // One table fetch per pair gives W (cutoff r^2 <= R^2) and gradW (cutoff |r| <= R); the {W, G} table sits in LDS.
-__global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_density_factor(const SceneParams* __restrict__ P,
+template <unsigned kTiles>
+__global__ void __launch_bounds__(kTiles * kTile, kTiles == kGroupTiles ? kGroupsPerCU : 1) k_density_factor(const SceneParams* __restrict__ P,
                                                            const uint32_t* __restrict__ tileScene, KTabHost kh,
                                                            Fields F, uint32_t cap, TileGrid tg) {
     extern __shared__ float4 lds[];
@@ -34,7 +35,7 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_density_factor(con
     load_table_wg(sWG, kh.tab);
     const KTab k{sWG, kh.R, kh.R2, kh.invStep, kh.W0};
     float* rec = reinterpret_cast<float*>(lds + kLdsWG / sizeof(float4));
-    group_loop<1>(tg, halo(F), rec, global_src(F, cap), LoadX{F.pos}, [&](uint32_t tile, bool ok, const NbrSrc& src) {
+    group_loop<1, kTiles>(tg, halo(F), rec, global_src(F, cap), LoadX{F.pos}, [&](uint32_t tile, bool ok, const NbrSrc& src) {
         const TileCtx c = tile_ctx4(tile, ok, tileScene, P);
         if (!c.valid) return;
         const SceneParams& p = P[c.s];
@@ -68,9 +69,19 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_density_factor(con
     });
 }
 
-void launch_density_factor(const Launch& L, const KTabHost& kt, const Fields& F) {
-    hipLaunchKernelGGL(k_density_factor, dim3(L.gridGroups), dim3(kGroupSize), kLdsDensity,
-                       L.stream, L.P, L.tileScene, kt, F, L.capacity, TileGrid(L.tg));
+void launch_density_factor(const Launch& L, uint32_t groupTiles, const KTabHost& kt, const Fields& F) {
+    const auto run = [&](auto kernel, uint32_t grid) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(groupTiles * kTile), kLdsDensity, L.stream, L.P, L.tileScene, kt, F,
+                           L.capacity, TileGrid(L.tg));
+    };
+    if (groupTiles == kGroupTiles)
+        run(k_density_factor<kGroupTiles>, L.gridGroups);
+    else if (groupTiles == 1)
+        run(k_density_factor<1>, L.group_count(1));
+    else if (groupTiles == 2)
+        run(k_density_factor<2>, L.group_count(2));
+    else
+        run(k_density_factor<4>, L.group_count(4));
 }
 
 // ---- Jacobi solver control (DFSPHImplementation.cu:455-461, 526-532) -------------------------------------------
@@ -764,7 +775,9 @@ int configure_kernels() {
         const void* fn;
         size_t bytes;
     } const k[] = {
-        {(const void*)k_density_factor, kLdsDensity},
+        {(const void*)k_density_factor<1>, kLdsDensity},
+        {(const void*)k_density_factor<2>, kLdsDensity},
+        {(const void*)k_density_factor<4>, kLdsDensity},
         {(const void*)k_div_init, kLdsXV},
         {(const void*)k_div_accel, kLdsXS},
         {(const void*)k_div_iter, kLdsXV},

@@ -24,6 +24,8 @@ struct Launch {
     uint32_t gridGroups;         // persistent grid of kGroupSize-thread blocks (one group at a time), 1 per CU
     uint32_t groups;             // 8 * per / kGroupTiles
     struct { uint32_t tiles, per; } tg;  // per = tiles of one XCD chunk, a multiple of 4
+    // groups of `tiles` tiles, those of no particles in the chunks' ends included
+    uint32_t group_count(uint32_t tiles) const { return 8u * (tg.per / tiles); }
 };
 
 // ---- adjoint.hip -----------------------------------------------------------------------------------------------
@@ -175,8 +177,8 @@ void launch_sort(const Launch& L, const SceneGrid* G, uint32_t totalCells, const
                  const float4* dvIn, const float* dkIn, const uint32_t* idIn, float4* posOut, float4* velOut,
                  float4* dvOut, float* dkOut, uint32_t* idOut, uint32_t* cellOf, uint32_t* rank, uint32_t* tmpId,
                  uint32_t* cellCount, uint32_t* cellStart, uint32_t* scanScratch);
-void launch_build_halo(const Launch& L, const uint32_t* nbrCount, const uint32_t* nbrList, uint32_t haloLimit,
-                       uint32_t* haloCount, uint32_t* haloIds, uint32_t* nbrLocal, uint32_t* haloStats,
+void launch_build_halo(const Launch& L, uint32_t groupTiles, const uint32_t* nbrCount, const uint32_t* nbrList,
+                       uint32_t haloLimit, uint32_t* haloCount, uint32_t* haloIds, uint32_t* nbrLocal, uint32_t* haloStats,
                        const float4* pos, const KTabHost& kt);
 void launch_build_lists(const Launch& L, const SceneGrid* G, const float4* pos, const uint32_t* cellStart,
                         const uint32_t* cellCount, uint32_t* nbrCount, uint32_t* nbrList,
@@ -257,7 +259,7 @@ struct Fields {
     const uint32_t* mcOff;
 };
 
-void launch_density_factor(const Launch& L, const KTabHost& kt, const Fields& F);
+void launch_density_factor(const Launch& L, uint32_t groupTiles, const KTabHost& kt, const Fields& F);
 void launch_scene_init_div(const Launch& L, const Fields& F);
 void launch_div_init(const Launch& L, const KTabHost& kt, const Fields& F);
 void launch_div_accel(const Launch& L, const KTabHost& kt, const Fields& F);
@@ -287,7 +289,6 @@ void launch_pres_iter(const Launch& L, const KTabHost& kt, const Fields& F);
 void launch_pres_final(const Launch& L, const KTabHost& kt, const Fields& F, int writeNext, const uint32_t* aborted);
 // ---- solve.hip: whole solves as one launch ----------------------------------------------------------------------
 constexpr uint32_t kResidentScenes = 256;        // scenes of a resident solve (their scalars live in LDS)
-constexpr uint32_t kResidentTiles = kGroupSize;  // tiles: a thread each when a block adds up a scene's partials
 // Barrier words (32-bit), zero between launches; words[kResidentAbortedAt] is set when a solve was aborted, and then
 // the host clears all of them.
 constexpr uint32_t kResidentWords = 1024, kResidentAbortedAt = 18 * 32;
@@ -295,11 +296,13 @@ struct Resident {
     uint32_t* words;
     uint32_t waitTicks;  // longest wait at a barrier, in ticks of the 100 MHz wall clock
 };
-// every group of the simulation has a block of its own on numCU CUs
-bool resident_fits(const Launch& L, uint32_t numCU);
-void launch_div_solve(const Launch& L, const KTabHost& kt, const Fields& F, const Resident& r);
-void launch_pres_solve(const Launch& L, const KTabHost& kt, const Fields& F, const Resident& r, int writeNext);
-void launch_visc_solve(const Launch& L, const KTabHost& kt, const Fields& F, const Resident& r,
+// Tiles per group with which every group has a block of its own on numCU CUs, the fewest of 1, 2 and 4; 0: none, or
+// too many scenes. Solves, halo build and density of a step take the same value.
+uint32_t resident_group_tiles(const Launch& L, uint32_t numCU);
+void launch_div_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt, const Fields& F, const Resident& r);
+void launch_pres_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt, const Fields& F, const Resident& r,
+                       int writeNext);
+void launch_visc_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt, const Fields& F, const Resident& r,
                        const uint32_t* haloStats);
 int configure_solve_kernels();
 void launch_scene_state_init(const Launch& L, SceneState* state, const float* dt0);

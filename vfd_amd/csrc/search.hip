@@ -8,6 +8,7 @@
 //     contiguous cells; the reference keeps particles in input order and only sorts index arrays;
 //   - the order inside a cell is ascending original id (deterministic) instead of atomicAdd order;
 //   - lists hold slot indices in a transposed [j][i] layout with a fixed capacity of 70 per particle.
+#include <algorithm>
 #include <mutex>
 
 #include "device.h"
@@ -558,7 +559,7 @@ __global__ void k_fill_u64(unsigned long long* p, uint32_t n) {
 }
 
 // ---- halos of the neighbour groups ------------------------------------------------------------------------------
-// One block per group. The distinct particle slots among the lists of its kGroupSize particles are collected in an
+// One block per group of kTiles tiles. The distinct particle slots among the lists of its particles are collected in an
 // LDS hash set of 32-slot buckets (bucket = slot >> 5, Fibonacci-hashed, linear probing) with a presence mask each;
 // halo numbers are handed out bucket by bucket, ascending inside a bucket, so runs of consecutive particle slots stay
 // consecutive in the halo. Every list entry is then rewritten as its halo number, packed with the pair's
@@ -570,27 +571,29 @@ __global__ void k_fill_u64(unsigned long long* p, uint32_t n) {
 constexpr uint32_t kBucketSlots = 2048;
 constexpr uint32_t kBucketLimit = 896;  // + one bucket per thread in flight < kBucketSlots: probing always ends
 constexpr uint32_t kHashEmpty = 0xFFFFFFFFu;
-static_assert(kBucketLimit + kGroupSize < kBucketSlots, "bucket table must never fill");
+static_assert(kBucketLimit + 4 * kTile < kBucketSlots, "bucket table must never fill");
 
 __device__ __forceinline__ uint32_t bucket_hash(uint32_t b) { return (b * 0x9E3779B1u) >> 21; }  // 11 bits
 constexpr size_t kLdsHaloPos = (size_t)kHaloMax * 3 * sizeof(float);  // halo positions of k_build_halo
 
-__global__ void __launch_bounds__(kGroupSize) k_build_halo(const SceneParams* __restrict__ P,
+template <unsigned kTiles>
+__global__ void __launch_bounds__(kTiles * kTile) k_build_halo(const SceneParams* __restrict__ P,
                                                            const uint32_t* __restrict__ tileScene, uint32_t tiles,
                                                            const uint32_t* __restrict__ nbrCount,
                                                            const uint32_t* __restrict__ nbrList, uint32_t cap,
                                                            uint32_t limit, uint32_t* haloCount, uint32_t* haloIds,
                                                            uint32_t* nbrLocal, uint32_t* haloStats,
                                                            const float4* __restrict__ pos, float R, float invStep) {
+    constexpr uint32_t kThreads = kTiles * kTile, kFill = halo_fill(kTiles);
     __shared__ uint32_t bkey[kBucketSlots];
     __shared__ uint32_t bmask[kBucketSlots];
     __shared__ uint16_t bbase[kBucketSlots];
-    __shared__ uint32_t waveTotal[kGroupSize / kWave];
+    __shared__ uint32_t waveTotal[kThreads / kWave];
     __shared__ uint32_t used, rows;
     extern __shared__ float hpos[];  // [kHaloMax * 3]: positions of the halo, by halo number
     const uint32_t g = blockIdx.x;
-    const uint32_t tile = g * kGroupTiles + threadIdx.x / kTile;
-    const uint32_t i = g * kGroupSize + threadIdx.x;
+    const uint32_t tile = g * kTiles + threadIdx.x / kTile;
+    const uint32_t i = g * kThreads + threadIdx.x;
     uint32_t n = 0;
     if (tile < tiles) {
         const SceneParams& p = P[tileScene[tile]];
@@ -642,7 +645,7 @@ __global__ void __launch_bounds__(kGroupSize) k_build_halo(const SceneParams* __
     }
     __syncthreads();
     // halo numbers: thread t owns bucket slots [2t, 2t + 2)
-    constexpr uint32_t kPer = kBucketSlots / kGroupSize;
+    constexpr uint32_t kPer = kBucketSlots / kThreads;
     uint32_t own = 0;
 #pragma unroll
     for (uint32_t k = 0; k < kPer; ++k) own += __popc(bmask[kPer * threadIdx.x + k]);
@@ -656,7 +659,7 @@ __global__ void __launch_bounds__(kGroupSize) k_build_halo(const SceneParams* __
     if (lane == kWave - 1) waveTotal[w] = incl;
     __syncthreads();
     uint32_t m = 0;
-    for (int k = 0; k < (int)(kGroupSize / kWave); ++k) m += waveTotal[k];
+    for (int k = 0; k < (int)(kThreads / kWave); ++k) m += waveTotal[k];
     if (used > kBucketLimit || m > limit) {  // block-uniform
         if (threadIdx.x == 0) {
             haloCount[g] = kHaloNone;
@@ -686,16 +689,16 @@ __global__ void __launch_bounds__(kGroupSize) k_build_halo(const SceneParams* __
     }
     __syncthreads();
     // the halo's positions, by halo number (ids written above by the block, visible after the barrier)
-    if (m) {  // up to four entries per thread (kHaloMax <= 4 kGroupSize): all id loads, then all gathers
-        uint32_t t[4];
-        float4 x[4];
+    if (m) {  // up to kFill entries per thread: all id loads, then all gathers
+        uint32_t t[kFill];
+        float4 x[kFill];
 #pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) t[u] = ids[min(threadIdx.x + u * kGroupSize, m - 1u)];
+        for (uint32_t u = 0; u < kFill; ++u) t[u] = ids[min(threadIdx.x + u * kThreads, m - 1u)];
 #pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) x[u] = pos[t[u]];
+        for (uint32_t u = 0; u < kFill; ++u) x[u] = pos[t[u]];
 #pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-            const uint32_t k = threadIdx.x + u * kGroupSize;
+        for (uint32_t u = 0; u < kFill; ++u) {
+            const uint32_t k = threadIdx.x + u * kThreads;
             if (k < m) {
                 hpos[3 * k] = x[u].x;
                 hpos[3 * k + 1] = x[u].y;
@@ -735,13 +738,22 @@ __global__ void __launch_bounds__(kGroupSize) k_build_halo(const SceneParams* __
     }
 }
 
-void launch_build_halo(const Launch& L, const uint32_t* nbrCount, const uint32_t* nbrList, uint32_t haloLimit,
-                       uint32_t* haloCount, uint32_t* haloIds, uint32_t* nbrLocal, uint32_t* haloStats,
-                       const float4* pos, const KTabHost& kt) {
+void launch_build_halo(const Launch& L, uint32_t groupTiles, const uint32_t* nbrCount, const uint32_t* nbrList,
+                       uint32_t haloLimit, uint32_t* haloCount, uint32_t* haloIds, uint32_t* nbrLocal,
+                       uint32_t* haloStats, const float4* pos, const KTabHost& kt) {
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, L.stream, haloStats, 0u, 3u);
-    hipLaunchKernelGGL(k_build_halo, dim3(L.groups), dim3(kGroupSize), kLdsHaloPos, L.stream, L.P, L.tileScene, L.tiles,
-                       nbrCount, nbrList, L.capacity, haloLimit < kHaloMax ? haloLimit : kHaloMax, haloCount, haloIds,
-                       nbrLocal, haloStats, pos, kt.R, kt.invStep);
+    const auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(L.group_count(groupTiles)), dim3(groupTiles * kTile), kLdsHaloPos, L.stream,
+                           L.P, L.tileScene, L.tiles, nbrCount, nbrList, L.capacity,
+                           std::min<uint32_t>(haloLimit, halo_cap(groupTiles)), haloCount, haloIds, nbrLocal,
+                           haloStats, pos, kt.R, kt.invStep);
+    };
+    if (groupTiles == 1)
+        run(k_build_halo<1>);
+    else if (groupTiles == 2)
+        run(k_build_halo<2>);
+    else
+        run(k_build_halo<4>);
 }
 
 void launch_build_lists(const Launch& L, const SceneGrid* G, const float4* pos, const uint32_t* cellStart,
@@ -758,9 +770,9 @@ void launch_build_lists(const Launch& L, const SceneGrid* G, const float4* pos, 
 }
 
 int configure_search_kernels() {
-    if (hipFuncSetAttribute((const void*)k_build_halo, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)kLdsHaloPos) != hipSuccess)
-        return 1;
+    for (const void* fn : {(const void*)k_build_halo<1>, (const void*)k_build_halo<2>, (const void*)k_build_halo<4>})
+        if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsHaloPos) != hipSuccess)
+            return 1;
     if (kLdsListStage == 0) return 0;
     return hipFuncSetAttribute((const void*)k_build_lists, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)kLdsListStage) == hipSuccess ? 0 : 1;

@@ -162,13 +162,14 @@ struct KernelTable {
         }
         G[kTableResolution] = 0.0f;
     }
-    // averaged entries: the value GetW/GetGradientW return for table index p
+    // averaged entries: the value GetW/GetGradientW return for table index p, and the one of code kGCodeZero
     std::vector<float2> averaged() const {
         std::vector<float2> t(kTableEntries);
         for (unsigned p = 0; p < kTableEntries; ++p) {
             t[p].x = 0.5f * (W[p] + W[p + 1]);
             t[p].y = 0.5f * (G[p] + G[p + 1]);
         }
+        t.push_back(make_float2(t.back().x, 0.0f));  // kGCodeZero: beyond the gradient cutoff
         return t;
     }
 };
@@ -1024,8 +1025,10 @@ public:
         VFD_TRY(nbStats.alloc((size_t)2 * S));
         {
             const Launch L = launch();
-            VFD_TRY(haloCount.alloc(std::max<uint32_t>(L.groups, 1)));
-            VFD_TRY(haloIds.alloc((size_t)std::max<uint32_t>(L.groups, 1) * kHaloMax));
+            const uint32_t rt = resident_group_tiles(L, numCU);
+            const uint32_t groups = std::max(std::max<uint32_t>(L.groups, 1), rt ? L.group_count(rt) : 0u);
+            VFD_TRY(haloCount.alloc(groups));
+            VFD_TRY(haloIds.alloc((size_t)groups * kHaloMax));
             VFD_TRY(haloStats.alloc(3));
             VFD_TRY(nbrLocal.alloc(c * kMaxNeighbors));
         }
@@ -1265,7 +1268,8 @@ public:
     int step(int last) {
         if (!committed) VFD_TRY(commit());
         if (tiles == 0) return VFD_OK;  // OnUpdate returns for N = 0 (:65-67)
-        bool resident = useGraphs && residentPause == 0 && resident_fits(launch(), numCU);
+        uint32_t resident = useGraphs && residentPause == 0 ? resident_group_tiles(launch(), numCU) : 0u;
+        if (taping && resident) resident = kGroupTiles;  // recorded Jacobi solves are launched, over these groups
         if (residentPause) --residentPause;
         const int before = cur;
         const size_t records = tapeCount;
@@ -1276,13 +1280,13 @@ public:
             tapeCount = records;
             launch_fill_u32(stream, residentWords.p, 0u, kResidentWords);
             VFD_TRY(push_state());
-            rc = step_once(last, false);
+            rc = step_once(last, 0);
         }
         return rc;
     }
     static constexpr int kStepAborted = -1;
     // waits for the step's launches; kStepAborted when a resident solve was aborted
-    int drain(bool resident) {
+    int drain(uint32_t resident) {
         *hostAborted = 0;
         if (resident)
             VFD_HIP(hipMemcpyAsync(hostAborted, residentWords.p + kResidentAbortedAt, sizeof(uint32_t),
@@ -1290,8 +1294,10 @@ public:
         VFD_HIP(hipStreamSynchronize(stream));
         return *hostAborted ? kStepAborted : VFD_OK;
     }
-    int step_once(int last, bool resident) {
-        const bool residentJacobi = resident && !taping;  // (a recorded solve stores every iteration)
+    // resident: tiles per group of the step's resident solves, 0: launched iterations
+    int step_once(int last, uint32_t resident) {
+        const uint32_t groupTiles = resident ? resident : kGroupTiles;
+        const bool residentJacobi = resident != 0 && !taping;  // (a recorded solve stores every iteration)
         const Launch L = launch();
         const KTabHost K = ktab();
         bool anyST = false, anyVisc = false;
@@ -1312,7 +1318,7 @@ public:
         // halos are built after the boundary has pushed penetrating particles out (the lists themselves come from the
         // positions before)
         VFD_TRY(timed("build_halo", [&] {
-            launch_build_halo(L, nbrCount.p, nbrList.p, haloLimit, haloCount.p, haloIds.p, nbrLocal.p, haloStats.p,
+            launch_build_halo(L, groupTiles, nbrCount.p, nbrList.p, haloLimit, haloCount.p, haloIds.p, nbrLocal.p, haloStats.p,
                               pos.p, K);
         }));
         if (last == VFD_PHASE_BOUNDARY) return finish_partial(resident);
@@ -1354,7 +1360,7 @@ public:
                                          vb.p, xb.p, tp->con.p, tp->push.p, tp->flags.p);
             }
         }
-        VFD_TRY(timed("density_factor", [&] { launch_density_factor(L, K, F); }));
+        VFD_TRY(timed("density_factor", [&] { launch_density_factor(L, groupTiles, K, F); }));
         if (tp) {
             VFD_TRY(tape_copy(tp->rho, density.p, tp->n));
             VFD_TRY(tape_copy(tp->alpha, factor.p, tp->n));
@@ -1363,7 +1369,7 @@ public:
         if (last == VFD_PHASE_DENSITY || last == VFD_PHASE_FACTOR) return finish_partial(resident);
         // divergence solve (ComputeDivergence :506-575)
         if (residentJacobi) {
-            VFD_TRY(timed("div_solve", [&] { launch_div_solve(L, K, F, resident_words()); }));
+            VFD_TRY(timed("div_solve", [&] { launch_div_solve(L, resident, K, F, resident_words()); }));
         } else {
             launch_scene_init_div(L, F);
             VFD_TRY(timed("div_init", [&] { launch_div_init(L, K, F); }));
@@ -1395,7 +1401,7 @@ public:
         VFD_HIP(hipEventRecord(ev[4], stream));
         if (last == VFD_PHASE_SURFACE_TENSION) return finish_partial(resident);
         if (anyVisc && resident) {
-            VFD_TRY(timed("visc_solve", [&] { launch_visc_solve(L, K, F, resident_words(), haloStats.p); }));
+            VFD_TRY(timed("visc_solve", [&] { launch_visc_solve(L, resident, K, F, resident_words(), haloStats.p); }));
         } else if (anyVisc) {
             VFD_TRY(timed("visc_precond", [&] { launch_visc_precond(L, K, F); }));
             VFD_TRY(timed("cg_begin", [&] { launch_cg_begin(L, K, F); }));
@@ -1422,7 +1428,7 @@ public:
         if (last == VFD_PHASE_VELOCITY) return finish_partial(resident);
         if (residentJacobi) {
             VFD_TRY(timed("pres_solve", [&] {
-                launch_pres_solve(L, K, F, resident_words(), last >= VFD_PHASE_POSITION ? 1 : 0);
+                launch_pres_solve(L, resident, K, F, resident_words(), last >= VFD_PHASE_POSITION ? 1 : 0);
             }));
         } else {
             launch_scene_init_pres(L, F);
@@ -1574,7 +1580,7 @@ public:
             VFD_TRY(aHaloIds.alloc((size_t)std::max<uint32_t>(L.groups, 1) * kHaloMax));
             VFD_TRY(aNbrLocal.alloc((size_t)cap * kMaxNeighbors));
             VFD_TRY(aHaloStats.alloc(3));
-            launch_build_halo(L, t.count.p, t.list.p, haloLimit, aHaloCount.p, aHaloIds.p, aNbrLocal.p, aHaloStats.p,
+            launch_build_halo(L, kGroupTiles, t.count.p, t.list.p, haloLimit, aHaloCount.p, aHaloIds.p, aNbrLocal.p, aHaloStats.p,
                               t.x.p, ktab());
             A.groups.grid = L.gridGroups;
             A.groups.tiles = L.tg.tiles;
@@ -1710,7 +1716,7 @@ public:
     }
 
     // after a partial step the working positions become the state the next step starts from
-    int finish_partial(bool resident) {
+    int finish_partial(uint32_t resident) {
         VFD_TRY(drain(resident));
         VFD_HIP(hipMemcpyAsync(posNext.p, pos.p, (size_t)cap * sizeof(float4), hipMemcpyDeviceToDevice, stream));
         VFD_HIP(hipGetLastError());

@@ -1,14 +1,16 @@
-// solve.hip - resident solvers: a whole divergence, pressure or viscosity solve as one launch (no reference counterpart;
-// the reference launches every iteration's kernels and synchronises after each, DFSPHImplementation.cu:443-808).
+// solve.hip - resident solvers: a whole divergence, pressure or viscosity solve as one launch (no reference
+// counterpart; the reference launches every iteration's kernels and synchronises after each,
+// DFSPHImplementation.cu:443-808).
 //
-// For a simulation whose neighbour groups all fit the chip at once (one group of 1024 particles per block, one block
-// per CU: 262,144 particles on 256 CUs) an iteration launched as separate kernels is bound by the launches: each pays
-// about 4.5 us of start and end, 4-5 us to copy the kernel table into LDS and the latency of refilling the halo's
+// For a simulation whose neighbour groups all fit the chip at once (one group of 256, 512 or 1024 particles per block,
+// one block per CU: 262,144 particles on 256 CUs) an iteration launched as separate kernels is bound by the launches:
+// each pays about 4.5 us of start and end, 4-5 us to copy the kernel table into LDS and the latency of refilling the halo's
 // positions, around 2-5 us of neighbour sums; iterations enqueued past convergence pay the launches too. Here a block
 // keeps the table, its halo's positions and slots and its particles' own data for the whole solve, and the blocks
 // meet at grid barriers: after every acceleration and every update, twice an iteration (Jacobi and CG alike). An
-// iteration of the 8,000-particle dam break (8 groups) takes 21 us instead of 30, and none runs past convergence;
-// beyond one group per block the launched kernels stay, bound by memory there (k_div_iter: 118 us at 2M particles).
+// iteration of the 8,000-particle dam break takes 9.2 us instead of 30 (21 with groups of 1024), and none runs past
+// convergence; beyond 1024 particles per CU the launched kernels stay, bound by memory there (k_div_iter: 118 us at 2M
+// particles).
 //
 // Memory. What blocks exchange (kappa, pressure accelerations, CG directions, tile partials) is written with
 // write-through stores at agent scope, waited for before the barrier's arrival, and read with agent-scope loads that
@@ -22,6 +24,9 @@
 //
 // Results are the launched kernels' bits: the same sums in the same list order (terms.h), the same per-tile and
 // per-scene FP64 trees, the same loop conditions.
+#include <algorithm>
+#include <type_traits>
+
 #include "terms.h"
 
 namespace vfd {
@@ -161,6 +166,7 @@ __device__ __forceinline__ void grid_leave(const GridSync& g, bool aborted) {
 struct ResidentTraits {
     static constexpr int kListCache = 0;
     static constexpr bool kAlwaysSplit = true;
+    template <int R> using Shape = ListShape<R>;
 };
 struct LoadXSr : ResidentTraits {  // {x_t, s_t}
     static constexpr int kLo = 4, kHi = 0;
@@ -216,10 +222,18 @@ struct LoadXQVr : ResidentTraits {  // {x_t, m / rho_t} {u_t, -}, u_t = a_t + b_
     }
 };
 
-struct Group {
-    float* rec;      // halo records in LDS
-    uint32_t m;      // halo size (0 when not staged: nothing to fill)
-    uint32_t t[4];   // slots of this thread's halo entries threadIdx.x + u * kGroupSize, u < 4
+// v as a value of this point of the program: keeps what is formed from it - addresses, every pair's unpacked slot,
+// scaled gradient or bound - from being formed once outside the iterations, in registers of its own
+template <class T> __device__ __forceinline__ T here(T v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+template <unsigned kTiles> struct Group {
+    static constexpr uint32_t kThreads = kTiles * kTile, kFill = halo_fill(kTiles);
+    float* rec;         // halo records in LDS
+    uint32_t m;         // halo size (0 when not staged: nothing to fill)
+    uint32_t t[kFill];  // slots of this thread's halo entries threadIdx.x + u * kThreads, u < kFill
     uint32_t g, tile;
     TileCtx c;
     NbrSrc src;
@@ -227,16 +241,17 @@ struct Group {
 };
 // The block's group (false: past the last tile, the block takes no part) and its halo's slots. Same group to block
 // mapping as group_loop.
-__device__ __forceinline__ bool resident_group(Group& r, const SceneParams* P, const uint32_t* tileScene,
+template <unsigned kTiles>
+__device__ __forceinline__ bool resident_group(Group<kTiles>& r, const SceneParams* P, const uint32_t* tileScene,
                                                const Fields& F, uint32_t cap, const TileGrid& tg, uint32_t* words,
                                                uint32_t waitTicks, float* rec) {
-    const uint32_t perG = tg.per / kGroupTiles, chunk = blockIdx.x & 7u;
+    const uint32_t perG = tg.per / kTiles, chunk = blockIdx.x & 7u;
     r.g = chunk * perG + (blockIdx.x >> 3);
-    if (r.g * kGroupTiles >= tg.tiles) return false;
-    const uint32_t blocks = (tg.tiles + kGroupTiles - 1) / kGroupTiles;
+    if (r.g * kTiles >= tg.tiles) return false;
+    const uint32_t blocks = (tg.tiles + kTiles - 1) / kTiles;
     r.gs = GridSync{words, blocks, chunk, min(perG, blocks - chunk * perG), (blocks + perG - 1) / perG, 0u,
                     waitTicks};
-    r.tile = r.g * kGroupTiles + threadIdx.x / kTile;
+    r.tile = r.g * kTiles + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / kTile));  // (a scalar)
     r.c = tile_ctx4(r.tile, r.tile < tg.tiles, tileScene, P);
     const uint32_t m = F.haloCount[r.g];
     const bool staged = m <= kHaloMax;
@@ -244,36 +259,30 @@ __device__ __forceinline__ bool resident_group(Group& r, const SceneParams* P, c
     r.m = staged ? m : 0u;
     const uint32_t* ids = F.haloIds + (size_t)r.g * kHaloMax;
 #pragma unroll
-    for (uint32_t u = 0; u < 4; ++u) r.t[u] = r.m ? ids[min(threadIdx.x + u * kGroupSize, r.m - 1u)] : 0u;
+    for (uint32_t u = 0; u < r.kFill; ++u) r.t[u] = r.m ? ids[min(threadIdx.x + u * r.kThreads, r.m - 1u)] : 0u;
     r.src = NbrSrc{staged ? rec : nullptr, F.nbrLocal, F.nbrList, F.nbrCount, cap};
     return true;
 }
 // get(t) for every halo entry of this thread (loads together), then put(k, value)
-template <class Get, class Put> __device__ __forceinline__ void fill_halo(const Group& r, Get&& get, Put&& put) {
-    decltype(get(0u)) v[4];
-#pragma unroll
-    for (uint32_t u = 0; u < 4; ++u)
-        if (threadIdx.x + u * kGroupSize < r.m) v[u] = get(r.t[u]);
-#pragma unroll
-    for (uint32_t u = 0; u < 4; ++u)
-        if (threadIdx.x + u * kGroupSize < r.m) put(threadIdx.x + u * kGroupSize, v[u]);
-}
-// the halo's records of the Jacobi solves: {x, s} and, sharing the first 16 bytes, {x, v.x} {v.y, v.z}
-static_assert(HaloRec<LoadXSr>::L == 4 && HaloRec<LoadXVr>::kSplit, "both record forms keep x in the first 12 bytes");
-__device__ __forceinline__ void put_scalar(float* rec, uint32_t k, float s) { rec[4 * k + 3] = s; }
-__device__ __forceinline__ void put_vector(float* rec, uint32_t k, f3 v) {
-    rec[4 * k + 3] = v.x;
-    *reinterpret_cast<float2*>(rec + 4 * kHaloMax + 2 * k) = make_float2(v.y, v.z);
-}
 struct PosVec {
     f3 x, v;
 };
-
+template <unsigned kTiles, class Get, class Put>
+__device__ __forceinline__ void fill_halo(const Group<kTiles>& r, Get&& get, Put&& put) {
+    constexpr uint32_t kFill = Group<kTiles>::kFill, kThreads = Group<kTiles>::kThreads;
+    decltype(get(0u)) v[kFill];
+#pragma unroll
+    for (uint32_t u = 0; u < kFill; ++u)
+        if (threadIdx.x + u * kThreads < r.m) v[u] = get(here(r.t[u]));
+#pragma unroll
+    for (uint32_t u = 0; u < kFill; ++u)
+        if (threadIdx.x + u * kThreads < r.m) put(threadIdx.x + u * kThreads, v[u]);
+}
 // per-tile sums as tile_partials4, stored for other blocks; `first` = the first of the tile's slots written
-template <int NV>
+template <unsigned kTiles, int NV>
 __device__ __forceinline__ void exchange_partials(double (&v)[NV], double* partials, uint32_t tile, uint32_t first,
                                                   bool store) {
-    __shared__ double sh[kGroupSize / kWave][NV];
+    __shared__ double sh[kTiles * kTile / kWave][NV];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
 #pragma unroll
     for (int i = 0; i < NV; ++i) v[i] = wave_sum(v[i]);
@@ -301,13 +310,13 @@ struct SceneCtl {
     uint32_t pad;
 };
 // decide(s, ctl, sums) by one lane for every active scene; returns whether any scene is still active (block-uniform)
-template <int NV, class Decide>
+template <unsigned kTiles, int NV, class Decide>
 __device__ __forceinline__ bool decide_scenes(const SceneParams* P, uint32_t sceneCount, SceneCtl* ctl,
                                               const double* partials, uint32_t first, Decide&& decide) {
-    __shared__ double sh[kGroupSize / kWave][NV];
+    __shared__ double sh[kTiles * kTile / kWave][NV];
     __shared__ uint32_t live;
     const uint32_t lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-    constexpr uint32_t kWaves = kGroupSize / kWave;
+    constexpr uint32_t kWaves = kTiles * kTile / kWave;
     auto chunk_sum = [&](uint32_t begin, uint32_t end, double (&v)[NV]) {  // tiles begin + lane, zero past the end
         const uint32_t t = begin + lane;
 #pragma unroll
@@ -317,7 +326,7 @@ __device__ __forceinline__ bool decide_scenes(const SceneParams* P, uint32_t sce
         for (int i = 0; i < NV; ++i) v[i] = wave_sum(v[i]);
     };
     if (threadIdx.x == 0) live = 0u;
-    if (sceneCount == 1) {  // the block's waves take 64 tiles each (at most kWaves * 64 tiles, see kResidentTiles)
+    if (sceneCount == 1) {  // the block's waves take 64 tiles each: kTiles * 256 in all, as many as 256 blocks have
         if (ctl[0].active) {  // block-uniform
             double v[NV];
             chunk_sum(P[0].tileBegin + kWave * w, P[0].tileEnd, v);
@@ -344,9 +353,8 @@ __device__ __forceinline__ bool decide_scenes(const SceneParams* P, uint32_t sce
             const uint32_t b = P[s].tileBegin, e = P[s].tileEnd;
             double sum[NV], v[NV];
             chunk_sum(b, e, sum);
-            for (uint32_t q = 1; q < kWaves; ++q) {  // zero chunks past the scene add nothing, as in the block's tree
-                if (b + kWave * q >= e) break;
-                chunk_sum(b + kWave * q, e, v);
+            for (uint32_t t = b + kWave; t < e; t += kWave) {  // (zero chunks past the scene would add nothing)
+                chunk_sum(t, e, v);
 #pragma unroll
                 for (int i = 0; i < NV; ++i) sum[i] += v[i];
             }
@@ -360,20 +368,221 @@ __device__ __forceinline__ bool decide_scenes(const SceneParams* P, uint32_t sce
     return live != 0u;
 }
 
+// ---- the sums of the Jacobi solves ----------------------------------------------------------------------------------
+// What a solve asks of its block's neighbour sums: the divergence of a field (begin), and per half iteration the halo's
+// kappa or accelerations filled in (fill_*, then a block barrier) and the sum over the particle's own list.
+
+// Lists and halo records in LDS, as the launched kernels have them; four waves per SIMD leave no registers for more.
+static_assert(HaloRec<LoadXSr>::L == 4 && HaloRec<LoadXVr>::kSplit, "both record forms keep x in the first 12 bytes");
+template <unsigned kTiles> struct ListSums {
+    static constexpr size_t kLds = kLdsG + HaloRec<LoadXVr>::kBytes;
+    const SceneParams& p;
+    const Fields& F;
+    const Group<kTiles>& r;
+    float* sG;
+    float* rec;
+    KLds K;
+    __device__ __forceinline__ ListSums(const SceneParams& p_, const Fields& F_, const Group<kTiles>& r_, float4* lds,
+                                        const KTabHost& kh)
+        : p(p_), F(F_), r(r_), sG(reinterpret_cast<float*>(lds)),
+          rec(reinterpret_cast<float*>(lds + kLdsG / sizeof(float4))), K{sG, kh.R, kh.invStep} {
+        load_table_g(sG, kh.tab);
+    }
+    __device__ __forceinline__ float* records() const { return rec; }
+    // {x, v.x} {v.y, v.z}; afterwards the fourth word holds kappa or a.x
+    __device__ __forceinline__ void begin() {
+        fill_halo(r, [&](uint32_t t) { return PosVec{ld3(F.pos[t]), ld3(F.vel[t])}; },
+                  [&](uint32_t k, const PosVec& q) { HaloRec<LoadXVr>::store(rec, k, st4(q.x), st4(q.v)); });
+        __syncthreads();
+    }
+    __device__ __forceinline__ float velocity_divergence(f3 v) const {
+        return field_divergence(p, K, F, r.src.cap, r.c.i, v, LoadXVr(F.pos, F.vel, false), r.src);
+    }
+    __device__ __forceinline__ void fill_scalar(const float* kap) const {
+        fill_halo(r, [&](uint32_t t) { return get_agent(kap + t); },
+                  [&](uint32_t k, float v) { rec[4 * k + 3] = v; });
+    }
+    __device__ __forceinline__ f3 accel(float k, const float* kap) const {
+        return pressure_accel(p, K, F, r.src.cap, r.c.i, k, LoadXSr(F.pos, kap), r.src);
+    }
+    __device__ __forceinline__ void fill_accel() const {
+        fill_halo(r, [&](uint32_t t) { return get_agent(F.ap + t); },
+                  [&](uint32_t k, f3 v) {
+                      rec[4 * k + 3] = v.x;
+                      *reinterpret_cast<float2*>(rec + 4 * kHaloMax + 2 * k) = make_float2(v.y, v.z);
+                  });
+    }
+    __device__ __forceinline__ float accel_divergence(f3 a) const {
+        return field_divergence(p, K, F, r.src.cap, r.c.i, a, LoadXVr(F.pos, F.ap, true), r.src);
+    }
+};
+
+// The pairs in registers: with one or two waves per SIMD a thread has room for gradW of its first kPairs neighbours and
+// their halo slots, which do not change during a solve, so that a half iteration reads nothing but the exchanged value
+// of each neighbour from LDS: no list, position or table reads. Those bound the loops of these block sizes, one list
+// chunk's latency after another: an iteration of 8,000 particles took 17.3 us with ListSums and takes 9.2 us, half of it
+// its two barriers. Neighbours past kPairs are looked up as they come (one-tile groups have room for every list); a
+// group whose halo is not staged takes ListSums.
+template <unsigned kTiles> struct PairSums {
+    static constexpr uint32_t kPairs = kTiles == 1 ? 72 : 44;  // of 512 and 256 registers a thread
+    static constexpr uint32_t kPairChunk = kTiles == 1 ? 8 : 4;
+    static constexpr bool kRest = kPairs < kMaxNeighbors;
+    static constexpr size_t kLds = (size_t)kHaloMax * 8 * sizeof(float);
+    const SceneParams& p;
+    const Fields& F;
+    const Group<kTiles>& r;
+    const float2* __restrict__ tab;
+    float R, invStep;
+    float4* sV;  // the vectors summed over
+    float *sK, *sX;  // kappa; positions
+    uint32_t n, rows;  // neighbours; the wave's longest list
+    f3 q[kPairs];
+    uint32_t slots[kPairs / 2];
+    f3 contact[kMaxBodies];  // gradW of the boundary samples
+    float vb[kMaxBodies];
+    __device__ __forceinline__ PairSums(const SceneParams& p_, const Fields& F_, const Group<kTiles>& r_, float4* lds,
+                                        const KTabHost& kh)
+        : p(p_), F(F_), r(r_), tab(kh.tab), R(kh.R), invStep(kh.invStep), sV(lds),
+          sK(reinterpret_cast<float*>(lds + kHaloMax)),
+          sX(sK + kHaloMax), n(0), rows(0) {}
+    __device__ __forceinline__ uint32_t slot(uint32_t j) const {
+        return (here(slots[j / 2]) >> (16 * (j & 1u))) & 0xFFFFu;
+    }
+    // staged entries 2j, 2j + 1 (0 past the list's end, without a memory access; see each_neighbor_rec)
+    __device__ __forceinline__ uint2 entries(uint32_t j) const {
+        const __amdgpu_buffer_rsrc_t row = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint32_t*>(r.src.local + (size_t)j * r.src.cap * 2), (short)0, (int)(r.src.cap * 8),
+            kRawBufferWord3);
+        const uint32_t off = r.c.i * 8u + (2 * j < n ? 0u : kBufferOutOfRange);
+        const auto v = __builtin_amdgcn_raw_buffer_load_b64(row, (int)off, 0, 0);
+        return make_uint2(v[0], v[1]);
+    }
+    __device__ __forceinline__ void begin() {
+        fill_halo(r, [&](uint32_t t) { return PosVec{ld3(F.pos[t]), ld3(F.vel[t])}; },
+                  [&](uint32_t k, const PosVec& h) {
+                      sX[3 * k] = h.x.x;
+                      sX[3 * k + 1] = h.x.y;
+                      sX[3 * k + 2] = h.x.z;
+                      sV[k] = st4(h.v);
+                  });
+        if (r.c.valid) n = F.nbrCount[r.c.i];
+        rows = n;
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) rows = max(rows, (uint32_t)__shfl_xor((int)rows, o, kWave));
+        rows = __builtin_amdgcn_readfirstlane(rows);
+        __syncthreads();
+        const f3 xi = r.c.valid ? ld3(F.pos[r.c.i]) : mk3(0.0f, 0.0f, 0.0f);
+#pragma unroll
+        for (uint32_t j = 0; j < kPairs; j += kPairChunk) {
+            if (j < rows) {  // wave-uniform
+                uint2 e[kPairChunk / 2];
+                float g[kPairChunk];
+#pragma unroll
+                for (uint32_t u = 0; u < kPairChunk / 2; ++u) e[u] = entries(j / 2 + u);
+#pragma unroll
+                for (uint32_t u = 0; u < kPairChunk; ++u) g[u] = tab[(u & 1u ? e[u / 2].y : e[u / 2].x) >> 16].y;
+#pragma unroll
+                for (uint32_t u = 0; u < kPairChunk; ++u) {
+                    const uint32_t s = (u & 1u ? e[u / 2].y : e[u / 2].x) & 0xFFFFu;
+                    q[j + u] = g[u] * (xi - position(s));
+                    if (u & 1u)
+                        slots[(j + u) / 2] |= s << 16;
+                    else
+                        slots[(j + u) / 2] = s;
+                }
+            }
+        }
+        const KTab k{tab, R, 0.0f, invStep, 0.0f};
+#pragma unroll
+        for (uint32_t b = 0; b < kMaxBodies; ++b) {
+            vb[b] = r.c.valid && b < p.bodyCount ? F.vb[(size_t)b * r.src.cap + r.c.i] : 0.0f;
+            contact[b] = mk3(0.0f, 0.0f, 0.0f);
+            if (vb[b] > 0.0f) contact[b] = gradW(k, xi - ld3(F.xb[(size_t)b * r.src.cap + r.c.i]));
+        }
+    }
+    __device__ __forceinline__ f3 position(uint32_t s) const { return mk3(sX[3 * s], sX[3 * s + 1], sX[3 * s + 2]); }
+    // f(slot, gradW) for the neighbours past kPairs, in list order
+    template <class Fn> __device__ __forceinline__ void rest(Fn&& f) const {
+        const f3 xi = ld3(F.pos[r.c.i]);
+        for (uint32_t j = kPairs; j < n; ++j) {
+            const uint2 e = entries(j / 2);
+            const uint32_t w = j & 1u ? e.y : e.x, s = w & 0xFFFFu;
+            f(s, tab[w >> 16].y * (xi - position(s)));
+        }
+    }
+    // sum_j (u - u_j) . gradW_ij V + sum_b V_b u . gradW_ib (field_divergence), u_j in sV
+    __device__ __forceinline__ float divergence(f3 ui) const {
+        const uint32_t cnt = here(n);
+        float d = 0.0f;
+#pragma unroll
+        for (uint32_t j = 0; j < kPairs; j += kPairChunk) {
+            if (j < rows) {
+                f3 uj[kPairChunk];
+#pragma unroll
+                for (uint32_t u = 0; u < kPairChunk; ++u) uj[u] = ld3(sV[slot(j + u)]);
+#pragma unroll
+                for (uint32_t u = 0; u < kPairChunk; ++u) {
+                    const float s = d + dot3(ui - uj[u], q[j + u]);
+                    d = j + u < cnt ? s : d;
+                }
+            }
+        }
+        if (kRest && n > kPairs) rest([&](uint32_t s, f3 g) { d += dot3(ui - ld3(sV[s]), g); });
+        d *= p.V;
+#pragma unroll
+        for (uint32_t b = 0; b < kMaxBodies; ++b)
+            if (vb[b] > 0.0f) d += vb[b] * dot3(ui, contact[b]);
+        return d;
+    }
+    __device__ __forceinline__ float velocity_divergence(f3 v) const { return divergence(v); }
+    __device__ __forceinline__ void fill_scalar(const float* kap) const {
+        fill_halo(r, [&](uint32_t t) { return get_agent(kap + t); }, [&](uint32_t k, float v) { sK[k] = v; });
+    }
+    __device__ __forceinline__ f3 accel(float ki, const float*) const {  // pressure_accel
+        const float negV = here(-p.V);
+        const uint32_t cnt = here(n);
+        f3 a = mk3(0.0f, 0.0f, 0.0f);
+        auto term = [&](float kj, f3 g, bool in) {
+            const float s = ki + kj;
+            const f3 gj = negV * g, t = a + s * gj;
+            const bool take = in && above_eps(fabsf(s));
+            a = mk3(take ? t.x : a.x, take ? t.y : a.y, take ? t.z : a.z);
+        };
+#pragma unroll
+        for (uint32_t j = 0; j < kPairs; j += kPairChunk) {
+            if (j < rows) {
+                float kj[kPairChunk];
+#pragma unroll
+                for (uint32_t u = 0; u < kPairChunk; ++u) kj[u] = sK[slot(j + u)];
+#pragma unroll
+                for (uint32_t u = 0; u < kPairChunk; ++u) term(kj[u], q[j + u], j + u < cnt);
+            }
+        }
+        if (kRest && n > kPairs) rest([&](uint32_t s, f3 g) { term(sK[s], g, true); });
+        if (above_eps(fabsf(ki))) {
+#pragma unroll
+            for (uint32_t b = 0; b < kMaxBodies; ++b)
+                if (vb[b] > 0.0f) {
+                    const f3 gj = (-vb[b]) * contact[b];
+                    a = a + ki * gj;
+                }
+        }
+        return a;
+    }
+    __device__ __forceinline__ void fill_accel() const {
+        fill_halo(r, [&](uint32_t t) { return get_agent(F.ap + t); }, [&](uint32_t k, f3 v) { sV[k] = st4(v); });
+    }
+    __device__ __forceinline__ float accel_divergence(f3 a) const { return divergence(a); }
+};
+
 // ---- Jacobi solves ------------------------------------------------------------------------------------------------
 // kPressure = false: k_div_init, the divergence iterations and k_div_final; true: k_pres_init, the pressure iterations
 // and k_pres_final (dfsph.hip). A block of no particles returns; every other block passes the same barriers.
-template <bool kPressure>
-__global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_jacobi_solve(const SceneParams* __restrict__ P,
-                                                                           const uint32_t* __restrict__ tileScene,
-                                                                           KTabHost kh, Fields F, uint32_t cap,
-                                                                           TileGrid tg, uint32_t sceneCount,
-                                                                           uint32_t* words, uint32_t waitTicks, int writeNext) {
-    __shared__ SceneCtl ctl[kResidentScenes];
-    if (words[kResidentAbortedAt]) return;  // an earlier solve of this step was aborted
-    VFD_HALO_KERNEL_PROLOGUE(kh)
-    Group r;
-    if (!resident_group(r, P, tileScene, F, cap, tg, words, waitTicks, rec)) return;
+template <unsigned kTiles, bool kPressure, class Sums>
+__device__ __forceinline__ void jacobi_solve(const SceneParams* __restrict__ P, const Fields& F, Group<kTiles>& r,
+                                             Sums& sums, SceneCtl* ctl, uint32_t tiles, uint32_t sceneCount,
+                                             int writeNext) {
+    constexpr uint32_t kThreads = kTiles * kTile;
     const TileCtx c = r.c;
     const SceneParams& p = P[c.s];
     const SceneState st = F.state[c.s];  // time step (its solver fields are written below by the first group)
@@ -382,7 +591,7 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_jacobi_solve(const
 
     // loop conditions before the first iteration (k_jacobi_begin)
     uint32_t any = 0;
-    for (uint32_t s = threadIdx.x; s < sceneCount; s += kGroupSize) {
+    for (uint32_t s = threadIdx.x; s < sceneCount; s += kThreads) {
         const SceneParams& q = P[s];
         const float eta = kPressure ? q.presTol * 0.0001f * q.rho0 : F.state[s].dtInv * q.divTol * 0.0001f * q.rho0;
         const uint32_t minIt = kPressure ? q.minPres : q.minDiv, maxIt = kPressure ? q.maxPres : q.maxDiv;
@@ -403,16 +612,13 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_jacobi_solve(const
         F.live[kPressure ? 1 : 0] = 0u;
         if (!kPressure) F.live[2] = 0u;
     }
-    fill_halo(r, [&](uint32_t t) { return PosVec{ld3(F.pos[t]), ld3(F.vel[t])}; },
-              [&](uint32_t k, const PosVec& q) {
-                  HaloRec<LoadXVr>::store(rec, k, st4(q.x), st4(q.v));
-              });
     bool live = __syncthreads_or((int)any) != 0;
+    sums.begin();
 
     float src = 0.0f, f = 0.0f, k = 0.0f, res = 0.0f;  // source term, scaled factor, kappa, residuum
     const uint32_t few = c.valid ? F.nbrCount[c.i] : 0u;
     if (on) {
-        const float d = field_divergence(p, K, F, cap, c.i, ld3(F.vel[c.i]), LoadXVr(F.pos, F.vel, false), r.src);
+        const float d = sums.velocity_divergence(ld3(F.vel[c.i]));
         if (kPressure) {
             src = F.density[c.i] / p.rho0 + st.dt * d;
             f = F.factor[c.i] * st.dt2Inv;
@@ -432,7 +638,8 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_jacobi_solve(const
             return;
         }
         if (iterations)
-            live = decide_scenes<1>(P, sceneCount, ctl, F.partials, 0, [&](uint32_t s, SceneCtl& t, double (&sum)[1]) {
+            live = decide_scenes<kTiles, 1>(P, sceneCount, ctl, F.partials, 0,
+                                            [&](uint32_t s, SceneCtl& t, double (&sum)[1]) {
                 const SceneParams& q = P[s];
                 const uint32_t minIt = kPressure ? q.minPres : q.minDiv, maxIt = kPressure ? q.maxPres : q.maxDiv;
                 const float err = (float)(-sum[0]) / (float)q.count;
@@ -445,24 +652,21 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_jacobi_solve(const
                     J.active = t.active;
                 }
             });
-        fill_halo(r, [&](uint32_t t) { return get_agent(kap + t); },
-                  [&](uint32_t q, float v) { put_scalar(rec, q, v); });
+        sums.fill_scalar(kap);
         __syncthreads();
         const bool act = live && ctl[c.s].active;
-        if (on && (act || !live)) a = pressure_accel(p, K, F, cap, c.i, k, LoadXSr(F.pos, kap), r.src);
+        if (on && (act || !live)) a = sums.accel(k, kap);
         if (!live) break;  // the accelerations of the final kappa
         if (on && act) put_agent(F.ap + c.i, a);
         if (!grid_sync(r.gs)) {
             grid_leave(r.gs, true);
             return;
         }
-        fill_halo(r, [&](uint32_t t) { return get_agent(F.ap + t); },
-                  [&](uint32_t q, f3 v) { put_vector(rec, q, v); });
+        sums.fill_accel();
         __syncthreads();
         double part = 0.0;
         if (on && act) {
-            const float force = field_divergence(p, K, F, cap, c.i, a, LoadXVr(F.pos, F.ap, true), r.src) *
-                                (kPressure ? st.dt2 : st.dt);
+            const float force = sums.accel_divergence(a) * (kPressure ? st.dt2 : st.dt);
             if (kPressure)
                 res = fminf(1.0f - src - force, 0.0f);
             else
@@ -472,7 +676,7 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_jacobi_solve(const
             part = (double)(p.rho0 * res);
         }
         double v[1] = {part};
-        exchange_partials<1>(v, F.partials, r.tile, 0, act && r.tile < tg.tiles);
+        exchange_partials<kTiles, 1>(v, F.partials, r.tile, 0, act && r.tile < tiles);
         ++iterations;
     }
     // the solve has passed its last barrier: results
@@ -496,6 +700,26 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_jacobi_solve(const
     }
     grid_leave(r.gs, false);
 }
+template <unsigned kTiles, bool kPressure>
+__global__ void __launch_bounds__(kTiles * kTile, 1) k_jacobi_solve(const SceneParams* __restrict__ P,
+                                                                    const uint32_t* __restrict__ tileScene, KTabHost kh,
+                                                                    Fields F, uint32_t cap, TileGrid tg,
+                                                                    uint32_t sceneCount, uint32_t* words,
+                                                                    uint32_t waitTicks, int writeNext) {
+    extern __shared__ float4 lds[];
+    __shared__ SceneCtl ctl[kResidentScenes];
+    if (words[kResidentAbortedAt]) return;  // an earlier solve of this step was aborted
+    Group<kTiles> r;
+    if (!resident_group(r, P, tileScene, F, cap, tg, words, waitTicks, reinterpret_cast<float*>(lds))) return;
+    if (kTiles < 4 && r.src.rec) {  // block-uniform
+        PairSums<kTiles> sums(P[r.c.s], F, r, lds, kh);
+        jacobi_solve<kTiles, kPressure>(P, F, r, sums, ctl, tg.tiles, sceneCount, writeNext);
+    } else {
+        ListSums<kTiles> sums(P[r.c.s], F, r, lds, kh);
+        if (r.src.rec) r.src.rec = sums.records();
+        jacobi_solve<kTiles, kPressure>(P, F, r, sums, ctl, tg.tiles, sceneCount, writeNext);
+    }
+}
 
 // ---- viscosity solve ------------------------------------------------------------------------------------------------
 // k_visc_precond, k_cg_begin, the CG iterations and k_visc_apply (dfsph.hip). The halo's second record half holds the
@@ -507,7 +731,8 @@ using RecQV = HaloRec<LoadXQVr>;
 static_assert(RecQV::L == 4 && HaloRec<LoadXQr>::L == 4, "both record forms keep {x, m / rho} in the first 16 bytes");
 __device__ __forceinline__ float* direction(float* rec, uint32_t k) { return rec + 4 * kHaloMax + RecQV::H * k; }
 
-__global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_visc_solve(const SceneParams* __restrict__ P,
+template <unsigned kTiles>
+__global__ void __launch_bounds__(kTiles * kTile, 1) k_visc_solve(const SceneParams* __restrict__ P,
                                                                          const uint32_t* __restrict__ tileScene,
                                                                          KTabHost kh, Fields F, uint32_t cap,
                                                                          TileGrid tg, uint32_t sceneCount,
@@ -516,7 +741,8 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_visc_solve(const S
     __shared__ SceneCtl ctl[kResidentScenes];
     if (words[kResidentAbortedAt]) return;  // an earlier solve of this step was aborted
     VFD_HALO_KERNEL_PROLOGUE(kh)
-    Group r;
+    constexpr uint32_t kThreads = kTiles * kTile;
+    Group<kTiles> r;
     if (!resident_group(r, P, tileScene, F, cap, tg, words, waitTicks, rec)) return;
     const TileCtx c = r.c;
     const SceneParams& p = P[c.s];
@@ -525,7 +751,7 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_visc_solve(const S
     const bool gathered = haloStats[1] != 0u;  // some group is not staged (the same in every block)
     const float m = P[0].m;                    // one particle radius per batch
 
-    for (uint32_t s = threadIdx.x; s < sceneCount; s += kGroupSize) {
+    for (uint32_t s = threadIdx.x; s < sceneCount; s += kThreads) {
         ctl[s].it = 0;
         ctl[s].active = P[s].enableVisc && P[s].count ? 1u : 0u;  // takes part in the set-up
     }
@@ -558,13 +784,14 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_visc_solve(const S
         v3[1] = (double)dot3(res, res);
         v3[2] = (double)dot3(res, z);
     }
-    exchange_partials<3>(v3, F.partials, r.tile, 0, r.tile < tg.tiles && p.enableVisc);
+    exchange_partials<kTiles, 3>(v3, F.partials, r.tile, 0, r.tile < tg.tiles && p.enableVisc);
     if (!grid_sync(r.gs)) {
         grid_leave(r.gs, true);
         return;
     }
     // k_cg_begin_finish
-    bool live = decide_scenes<3>(P, sceneCount, ctl, F.partials, 0, [&](uint32_t s, SceneCtl& t, double (&sum)[3]) {
+    bool live = decide_scenes<kTiles, 3>(P, sceneCount, ctl, F.partials, 0,
+                                         [&](uint32_t s, SceneCtl& t, double (&sum)[3]) {
         const SceneParams& q = P[s];
         CgState G = F.state[s].cg;
         G.it = 0;
@@ -624,13 +851,13 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_visc_solve(const S
             ap = visc_matvec(p, K, F, cap, c.i, dir, dt, LoadXQVr(F.pos, F.density, F.cgP, nullptr, m), r.src);
             v1[0] = (double)dot3(dir, ap);
         }
-        exchange_partials<1>(v1, F.partials, r.tile, 3, act || (r.tile < tg.tiles && ctl[c.s].active));
+        exchange_partials<kTiles, 1>(v1, F.partials, r.tile, 3, act || (r.tile < tg.tiles && ctl[c.s].active));
         if (!grid_sync(r.gs)) {
             grid_leave(r.gs, true);
             return;
         }
         // k_cg_alpha
-        (void)decide_scenes<1>(P, sceneCount, ctl, F.partials, 3, [&](uint32_t, SceneCtl& t, double (&sum)[1]) {
+        (void)decide_scenes<kTiles, 1>(P, sceneCount, ctl, F.partials, 3, [&](uint32_t, SceneCtl& t, double (&sum)[1]) {
             t.alpha = t.absNew / (float)sum[0];
         });
         double v2[2] = {0.0, 0.0};
@@ -644,13 +871,14 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_visc_solve(const S
             v2[0] = (double)dot3(res, res);
             v2[1] = (double)dot3(res, z);
         }
-        exchange_partials<2>(v2, F.partials, r.tile, 0, r.tile < tg.tiles && ctl[c.s].active);
+        exchange_partials<kTiles, 2>(v2, F.partials, r.tile, 0, r.tile < tg.tiles && ctl[c.s].active);
         if (!grid_sync(r.gs)) {
             grid_leave(r.gs, true);
             return;
         }
         // k_cg_update_finish
-        live = decide_scenes<2>(P, sceneCount, ctl, F.partials, 0, [&](uint32_t s, SceneCtl& t, double (&sum)[2]) {
+        live = decide_scenes<kTiles, 2>(P, sceneCount, ctl, F.partials, 0,
+                                        [&](uint32_t s, SceneCtl& t, double (&sum)[2]) {
             const SceneParams& q = P[s];
             const float res2 = (float)sum[0], err = sqrtf(res2 / t.rhs2);
             uint32_t goes = 0;
@@ -690,38 +918,64 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_visc_solve(const S
 }
 
 // ---- host side ----------------------------------------------------------------------------------------------------
-constexpr size_t kLdsJacobi = kLdsG + HaloRec<LoadXVr>::kBytes;
+constexpr size_t kLdsJacobi = ListSums<4>::kLds;
 constexpr size_t kLdsVisc = kLdsG + RecQV::kBytes;
 constexpr size_t kLdsStatic = kResidentScenes * sizeof(SceneCtl) + 2048;  // control and reduction arrays, at most
-static_assert(kLdsVisc + kLdsStatic <= 160 * 1024 / kGroupsPerCU, "a resident group must fit its share of a CU's LDS");
+static_assert(kLdsVisc + kLdsStatic <= 160 * 1024 && PairSums<1>::kLds <= kLdsJacobi, "a resident group must fit a CU's LDS");
 
-bool resident_fits(const Launch& L, uint32_t numCU) {
-    const uint32_t blocks = (L.tiles + kGroupTiles - 1) / kGroupTiles;
-    return L.tiles > 0 && blocks <= numCU * kGroupsPerCU && L.tiles <= kResidentTiles && L.sceneCount <= kResidentScenes;
+// The fewest tiles per group win: a group's neighbour sums are bound by its CU's LDS and VALU (1024 particles 7-8 us a
+// sum, 256 particles about 2), and more blocks cost a barrier at most 1.4 us.
+uint32_t resident_group_tiles(const Launch& L, uint32_t numCU) {
+    if (L.tiles == 0 || L.sceneCount > kResidentScenes) return 0;
+    for (uint32_t t : {1u, 2u, 4u})
+        if ((L.tiles + t - 1) / t <= std::min(numCU, 256u)) return t;
+    return 0;
 }
-void launch_div_solve(const Launch& L, const KTabHost& kt, const Fields& F, const Resident& r) {
-    hipLaunchKernelGGL(k_jacobi_solve<false>, dim3(L.groups), dim3(kGroupSize), kLdsJacobi, L.stream, L.P, L.tileScene,
-                       kt, F, L.capacity, TileGrid(L.tg), L.sceneCount, r.words, r.waitTicks, 0);
+template <class Run> static void with_tiles(uint32_t groupTiles, Run&& run) {
+    if (groupTiles == 1)
+        run(std::integral_constant<unsigned, 1>());
+    else if (groupTiles == 2)
+        run(std::integral_constant<unsigned, 2>());
+    else
+        run(std::integral_constant<unsigned, 4>());
 }
-void launch_pres_solve(const Launch& L, const KTabHost& kt, const Fields& F, const Resident& r, int writeNext) {
-    hipLaunchKernelGGL(k_jacobi_solve<true>, dim3(L.groups), dim3(kGroupSize), kLdsJacobi, L.stream, L.P, L.tileScene,
-                       kt, F, L.capacity, TileGrid(L.tg), L.sceneCount, r.words, r.waitTicks, writeNext);
+void launch_div_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt, const Fields& F, const Resident& r) {
+    with_tiles(groupTiles, [&](auto t) {
+        hipLaunchKernelGGL((k_jacobi_solve<t(), false>), dim3(L.group_count(t())), dim3(t() * kTile), kLdsJacobi,
+                           L.stream, L.P, L.tileScene, kt, F, L.capacity, TileGrid(L.tg), L.sceneCount, r.words,
+                           r.waitTicks, 0);
+    });
 }
-void launch_visc_solve(const Launch& L, const KTabHost& kt, const Fields& F, const Resident& r,
+void launch_pres_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt, const Fields& F, const Resident& r,
+                       int writeNext) {
+    with_tiles(groupTiles, [&](auto t) {
+        hipLaunchKernelGGL((k_jacobi_solve<t(), true>), dim3(L.group_count(t())), dim3(t() * kTile), kLdsJacobi,
+                           L.stream, L.P, L.tileScene, kt, F, L.capacity, TileGrid(L.tg), L.sceneCount, r.words,
+                           r.waitTicks, writeNext);
+    });
+}
+void launch_visc_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt, const Fields& F, const Resident& r,
                        const uint32_t* haloStats) {
-    hipLaunchKernelGGL(k_visc_solve, dim3(L.groups), dim3(kGroupSize), kLdsVisc, L.stream, L.P, L.tileScene, kt, F,
-                       L.capacity, TileGrid(L.tg), L.sceneCount, r.words, r.waitTicks, haloStats);
+    with_tiles(groupTiles, [&](auto t) {
+        hipLaunchKernelGGL((k_visc_solve<t()>), dim3(L.group_count(t())), dim3(t() * kTile), kLdsVisc, L.stream, L.P,
+                           L.tileScene, kt, F, L.capacity, TileGrid(L.tg), L.sceneCount, r.words, r.waitTicks,
+                           haloStats);
+    });
 }
 int configure_solve_kernels() {
-    const struct {
-        const void* fn;
-        size_t bytes;
-    } k[] = {{(const void*)k_jacobi_solve<false>, kLdsJacobi},
-             {(const void*)k_jacobi_solve<true>, kLdsJacobi},
-             {(const void*)k_visc_solve, kLdsVisc}};
-    for (const auto& e : k)
-        if (hipFuncSetAttribute(e.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)e.bytes) != hipSuccess) return 1;
-    return 0;
+    int bad = 0;
+    const auto set = [&](auto kernel, size_t bytes) {
+        if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) !=
+            hipSuccess)
+            bad = 1;
+    };
+    for (uint32_t g : {1u, 2u, 4u})
+        with_tiles(g, [&](auto t) {
+            set(k_jacobi_solve<t(), false>, kLdsJacobi);
+            set(k_jacobi_solve<t(), true>, kLdsJacobi);
+            set(k_visc_solve<t()>, kLdsVisc);
+        });
+    return bad;
 }
 
 }  // namespace vfd
