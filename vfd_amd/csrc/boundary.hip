@@ -9,6 +9,8 @@
 //
 // Step: ComputeVolumeAndBoundaryKernel (DFSPHKernels.cu:69-150) per particle and body: map lookup, boundary
 // neighbour position x_b and volume V_b, push-out of particles inside the solid.
+#include <algorithm>
+
 #include "device.h"
 #include "kernels.h"
 
@@ -290,52 +292,242 @@ __global__ void k_map_field0(ShapeDev shape, MapDev map, float* nodes0) {
     nodes0[l] = shape.sign * (shape_distance(shape, x) - shape.tol);
 }
 
-__global__ void __launch_bounds__(64) k_map_field1(MapDev map, const float* __restrict__ nodes0, float* nodes1,
-                                                   KTabHost kt, const float* __restrict__ glx,
-                                                   const float* __restrict__ glw) {
-    const uint32_t l = blockIdx.x * blockDim.x + threadIdx.x;
-    if (l >= map.nodeCount) return;
+// Field 1 (RigidBody.cu:45-72): 0.8 * the integral over the support ball around node x of {1 where phi <= 0,
+// W(phi) / W(0) where phi < R} by 16 x 16 x 16 Gauss-Legendre points, summed in their order (i, j, k), phi the
+// interpolant of field 0; 0 for a node farther than 2R. One thread per node that evaluates its 4096 points by
+// map_interp_at0 took 4.4 ms for a map of 40^3 cells (406k nodes): six divisions, 32 index products and 32 gathers a
+// point, and the lanes of far nodes idle. Here
+//   - k_map_near lists the nodes that have an integral at all (about a third), and a block takes 64 of them, a lane each;
+//   - what a point's evaluation needs of one axis (cell, local coordinate) is formed once per node, axis and point index;
+//   - points outside the ball, whose terms are zero, are left out (1,008 of 4,096 remain; the test does not depend on
+//     the node);
+//   - 128 consecutive points at a time are divided among the block's eight waves, consecutive ones to a wave, so that the
+//     32 node values of a cell stay in registers until the point leaves it (and come as 16 loads of two consecutive
+//     nodes: with 32 single loads the address unit bound the kernel, 1.26 ms); the weighted terms go to LDS and one wave
+//     adds them in order.
+// The same float expressions as shape_fn and map_locate, so the same bits. 0.72 ms for that map; 0.38 ms of it VALU work,
+// the rest the gathers.
+constexpr uint32_t kGauss = 16, kVolWaves = 8, kVolThreads = kVolWaves * kWave;
+constexpr uint32_t kPoints = 1024, kChunk = 128;  // 1,008 points lie in the ball, none within 0.1% of R of its surface
+__global__ void __launch_bounds__(kTile) k_map_near(MapDev map, const float* __restrict__ nodes0, float* nodes1, float R,
+                                                    uint32_t* list) {
+    const uint32_t l = blockIdx.x * kTile + threadIdx.x;
+    bool near = false;
+    if (l < map.nodeCount) {
+        near = !(map_interp_at0(map, nodes0, node_position(map, l)) > 2.0f * R);
+        if (!near) nodes1[l] = 0.0f;
+    }
+    const unsigned long long b = __ballot(near);
+    if (b == 0ull) return;
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    uint32_t at = 0;
+    if (lane == (uint32_t)__ffsll((long long)b) - 1u) at = atomicAdd(&list[0], (uint32_t)__popcll(b));
+    at = (uint32_t)__shfl((int)at, __ffsll((long long)b) - 1, kWave);
+    if (near) list[1 + at + (uint32_t)__popcll(b & ((1ull << lane) - 1ull))] = l;
+}
+// One axis of map_locate: the cell index, or kOutside, and the local coordinate in it.
+constexpr uint32_t kOutside = 0xFFFFFFFFu;
+__device__ __forceinline__ uint32_t axis_locate(const MapDev& m, int a, float x, float& xi) {
+    if (!(m.domMin[a] <= x && m.domMax[a] >= x)) return kOutside;
+    uint32_t c = (uint32_t)((x - m.domMin[a]) * m.cellSizeInv[a]);
+    if (c >= m.res[a]) c = m.res[a] - 1;
+    const float origin = m.domMin[a] + (float)c * m.cellSize[a];
+    const float top = origin + m.cellSize[a];
+    const float den = top - origin;
+    const float sum = top + origin;
+    xi = (2.0f / den) * x - sum / den;
+    return c;
+}
+struct __attribute__((packed, aligned(4))) NodePair {
+    float a, b;
+};
+// what the shape functions take of one coordinate: 1 -+ s, s^2 and (9/64) times both edge functions
+struct AxisTerms {
+    float l[2], s2, kf[2];
+};
+__device__ __forceinline__ AxisTerms axis_terms(float s) {
+    AxisTerms t;
+    t.l[0] = 1.0f - s;
+    t.l[1] = 1.0f + s;
+    t.s2 = s * s;
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+        float f, df;
+        edge1d(s, side, f, df);
+        t.kf[side] = 9.0f / 64.0f * f;
+    }
+    return t;
+}
+__global__ void __launch_bounds__(kVolThreads) k_map_volume(MapDev map, const float* __restrict__ nodes0, float* nodes1,
+                                                            KTabHost kt, const float* __restrict__ glx,
+                                                            const float* __restrict__ glw,
+                                                            const uint32_t* __restrict__ list) {
+    __shared__ float sXi[3][kGauss][kWave];
+    __shared__ uint32_t sCell[3][kGauss][kWave];
+    __shared__ float sTerm[kChunk][kWave];  // the chunk's weighted terms, point by point
+    __shared__ float sSum[kWave], sX[kGauss], sW[kGauss];
+    __shared__ uint16_t sPoint[kPoints];  // the points in the ball, in order: i << 8 | j << 4 | k
+    __shared__ uint32_t sBase[kVolWaves];
     const KTab k{kt.tab, kt.R, kt.R2, kt.invStep, kt.W0};
     const float R = kt.R;
-    const f3 x = node_position(map, l);
-    const float dX = map_interp_at0(map, nodes0, x);
-    if (dX > 2.0f * R) {
-        nodes1[l] = 0.0f;
-        return;
-    }
     const double c0 = (double)R;
-    float res = 0.0f;
-    for (int i = 0; i < 16; ++i) {
-        const float wi = glw[i];
-        for (int j = 0; j < 16; ++j) {
-            const float wij = wi * glw[j];
-            for (int kk = 0; kk < 16; ++kk) {
-                const float wijk = wij * glw[kk];
-                const f3 xi = mk3((float)(c0 * (double)glx[i]), (float)(c0 * (double)glx[j]), (float)(c0 * (double)glx[kk]));
-                float f = 0.0f;
-                if (!(dot3(xi, xi) > R * R)) {
-                    const float dist = map_interp_at0(map, nodes0, x + xi);
-                    if (dist <= 0.0f)
-                        f = 1.0f;
-                    else if (dist < R)
-                        f = getW_scalar(k, dist) / k.W0;
+    const uint32_t lane = threadIdx.x & (kWave - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const uint32_t nearCount = list[0];
+    const uint32_t nx = map.res[0], ny = map.res[1], nz = map.res[2];
+    const uint32_t nv = (nx + 1) * (ny + 1) * (nz + 1);
+    const uint32_t nex = nx * (ny + 1) * (nz + 1), ney = (nx + 1) * ny * (nz + 1);
+    if (threadIdx.x < kGauss) {
+        sX[threadIdx.x] = (float)(c0 * (double)glx[threadIdx.x]);
+        sW[threadIdx.x] = glw[threadIdx.x];
+    }
+    __syncthreads();
+    uint32_t points = 0;
+    for (uint32_t q0 = 0; q0 < kGauss * kGauss * kGauss; q0 += kVolThreads) {
+        const uint32_t q = q0 + threadIdx.x;
+        const f3 x = mk3(sX[q >> 8], sX[(q >> 4) & 15u], sX[q & 15u]);
+        const bool in = !(dot3(x, x) > R * R);
+        const unsigned long long b = __ballot(in);
+        if (lane == 0) sBase[w] = (uint32_t)__popcll(b);
+        __syncthreads();
+        uint32_t at = points + (uint32_t)__popcll(b & ((1ull << lane) - 1ull));
+        for (uint32_t v = 0; v < kVolWaves; ++v) {
+            at += v < w ? sBase[v] : 0u;
+            points += sBase[v];
+        }
+        if (in && at < kPoints) sPoint[at] = (uint16_t)q;
+        __syncthreads();
+    }
+    points = min(points, kPoints);
+    for (uint32_t n0 = blockIdx.x * kWave; n0 < nearCount; n0 += gridDim.x * kWave) {
+        const uint32_t l = list[1 + min(n0 + lane, nearCount - 1u)];  // lanes past the end repeat the last node
+        __syncthreads();
+        {
+            const f3 x = node_position(map, l);
+            const float xv[3] = {x.x, x.y, x.z};
+            for (uint32_t q = w; q < 3 * kGauss; q += kVolWaves) {
+                const uint32_t a = q / kGauss, g = q % kGauss;
+                float xi = 0.0f;
+                sCell[a][g][lane] = axis_locate(map, (int)a, (a == 0 ? xv[0] : a == 1 ? xv[1] : xv[2]) + sX[g], xi);
+                sXi[a][g][lane] = xi;
+            }
+            if (w == 0) sSum[lane] = 0.0f;
+        }
+        for (uint32_t s0 = 0; s0 < points; s0 += kChunk) {
+            __syncthreads();
+            const uint32_t count = min(kChunk, points - s0);
+            const uint32_t begin = count * w / kVolWaves, end = count * (w + 1) / kVolWaves;
+            uint32_t slab = kOutside, row = kOutside, ci = 0, cj = 0, atI = kOutside, atJ = kOutside, atK = kOutside;
+            AxisTerms X = {}, Y = {};
+            float v[32], ex[2][2], ey[2][2], exy[4] = {}, wi = 0.0f, wij = 0.0f, xy2 = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 32; ++q) v[q] = 0.0f;
+            for (uint32_t s = begin; s < end; ++s) {
+                const uint32_t p = __builtin_amdgcn_readfirstlane(sPoint[s0 + s]), i = p >> 8, j = p >> 4, kk = p & 15u;
+                if (j != row) {  // uniform: terms of the row, and of the slab
+                    row = j;
+                    if (i != slab) {
+                        slab = i;
+                        ci = sCell[0][i][lane];
+                        X = axis_terms(sXi[0][i][lane]);
+                        wi = sW[i];
+                    }
+                    cj = sCell[1][j & 15u][lane];
+                    Y = axis_terms(sXi[1][j & 15u][lane]);
+                    wij = wi * sW[j & 15u];
+                    xy2 = X.s2 + Y.s2;
+#pragma unroll
+                    for (int q = 0; q < 2; ++q)
+#pragma unroll
+                        for (int side = 0; side < 2; ++side) {
+                            ex[q][side] = X.kf[side] * Y.l[q];  // x edges at y side q
+                            ey[q][side] = Y.kf[side] * X.l[q];  // y edges at x side q
+                        }
                 }
-                res += wijk * f;
+                const uint32_t ck = sCell[2][kk][lane];
+                const bool ok = ci != kOutside && cj != kOutside && ck != kOutside;
+                if (__any(ok && (ci != atI || cj != atJ || ck != atK))) {  // some lane's point has left its cell
+                    if (ok) {
+                        // pairs of consecutive nodes, an 8-byte load each (4-byte aligned)
+                        auto pair = [&](uint32_t at, float& a, float& b) {
+                            const NodePair q = *reinterpret_cast<const NodePair*>(nodes0 + at);
+                            a = q.a;
+                            b = q.b;
+                        };
+#pragma unroll
+                        for (uint32_t e = 0; e < 4; ++e) {
+                            pair((nx + 1) * (ny + 1) * (ck + (e >> 1)) + (nx + 1) * (cj + (e & 1u)) + ci, v[2 * e],
+                                 v[2 * e + 1]);
+                            pair(nv + 2 * (nx * (ny + 1) * (ck + (e & 1u)) + nx * (cj + (e >> 1)) + ci), v[8 + 2 * e],
+                                 v[9 + 2 * e]);
+                            pair(nv + 2 * nex + 2 * (ny * (nz + 1) * (ci + (e & 1u)) + ny * (ck + (e >> 1)) + cj),
+                                 v[16 + 2 * e], v[17 + 2 * e]);
+                            pair(nv + 2 * nex + 2 * ney + 2 * (nz * (nx + 1) * (cj + (e & 1u)) + nz * (ci + (e >> 1)) + ck),
+                                 v[24 + 2 * e], v[25 + 2 * e]);
+                        }
+                    }
+                    atI = ci;
+                    atJ = cj;
+                    atK = ck;
+                }
+                const AxisTerms Z = axis_terms(sXi[2][kk][lane]);
+                float phi = 0.0f;
+                const float t = 1.0f / 64.0f * (9.0f * (xy2 + Z.s2) - 19.0f);
+#pragma unroll
+                for (int c = 0; c < 8; ++c) phi += v[c] * (t * X.l[c & 1] * Y.l[(c >> 1) & 1] * Z.l[c >> 2]);
+#pragma unroll
+                for (int q = 0; q < 2; ++q)  // x edges: y side q, z side z
+#pragma unroll
+                    for (int z = 0; z < 2; ++z)
+#pragma unroll
+                        for (int side = 0; side < 2; ++side) phi += v[8 + 2 * (z + 2 * q) + side] * (ex[q][side] * Z.l[z]);
+#pragma unroll
+                for (int z = 0; z < 2; ++z)  // y edges: z side z, x side q
+#pragma unroll
+                    for (int q = 0; q < 2; ++q)
+#pragma unroll
+                        for (int side = 0; side < 2; ++side) phi += v[16 + 2 * (q + 2 * z) + side] * (ey[q][side] * Z.l[z]);
+#pragma unroll
+                for (int side = 0; side < 2; ++side) exy[2 * side] = Z.kf[side] * X.l[0], exy[2 * side + 1] = Z.kf[side] * X.l[1];
+#pragma unroll
+                for (int q = 0; q < 2; ++q)  // z edges: x side q, y side y
+#pragma unroll
+                    for (int y = 0; y < 2; ++y)
+#pragma unroll
+                        for (int side = 0; side < 2; ++side)
+                            phi += v[24 + 2 * (y + 2 * q) + side] * (exy[2 * side + q] * Y.l[y]);
+                float f = 0.0f;
+                if (ok) {
+                    if (phi <= 0.0f)
+                        f = 1.0f;
+                    else if (phi < R)
+                        f = getW_scalar(k, phi) / k.W0;
+                }
+                sTerm[s][lane] = wij * sW[kk] * f;
+            }
+            __syncthreads();
+            if (w == (s0 / kChunk) % kVolWaves) {
+                float res = sSum[lane];
+                for (uint32_t s = 0; s < count; ++s) res += sTerm[s][lane];
+                sSum[lane] = res;
+                if (s0 + kChunk >= points && n0 + lane < nearCount)
+                    nodes1[l] = 0.8f * (float)((double)res * (c0 * c0 * c0));
             }
         }
     }
-    res = (float)((double)res * (c0 * c0 * c0));
-    nodes1[l] = 0.8f * res;
 }
 
 void launch_map_field0(hipStream_t st, const ShapeDev& shape, const MapDev& map, float* nodes0) {
     hipLaunchKernelGGL(k_map_field0, dim3((map.nodeCount + 255) / 256), dim3(256), 0, st, shape, map, nodes0);
 }
 
+uint32_t map_scratch_words(const MapDev& map) { return map.nodeCount + 1; }
 void launch_map_field1(hipStream_t st, const MapDev& map, const float* nodes0, float* nodes1, const KTabHost& kt,
-                       const float* glx, const float* glw) {
-    hipLaunchKernelGGL(k_map_field1, dim3((map.nodeCount + 63) / 64), dim3(64), 0, st, map, nodes0, nodes1, kt, glx,
-                       glw);
+                       const float* glx, const float* glw, uint32_t* scratch, uint32_t numCU) {
+    launch_fill_u32(st, scratch, 0u, 1u);
+    hipLaunchKernelGGL(k_map_near, dim3((map.nodeCount + kTile - 1) / kTile), dim3(kTile), 0, st, map, nodes0, nodes1,
+                       kt.R, scratch);
+    hipLaunchKernelGGL(k_map_volume, dim3(std::min((map.nodeCount + kWave - 1) / kWave, 2 * numCU)), dim3(kVolThreads), 0,
+                       st, map, nodes0, nodes1, kt, glx, glw, (const uint32_t*)scratch);
 }
 
 // ---- triangle-mesh signed distance (MeshDistance::SignedDistance, Utility/SDF/MeshDistance.cpp:186-225) ----------
@@ -430,8 +622,7 @@ __device__ __forceinline__ float tri_d2(float4 r0, float4 r1, float4 r2, float4 
     return d2;
 }
 
-constexpr uint32_t kMeshTile = 256;
-static_assert(kMeshTile % kMeshCluster == 0 && kMeshCluster == 64, "a wave decides one cluster at a time");
+static_assert(kMeshCluster == kWave, "a wave tests a cluster's spheres a lane each");
 
 // The map's nodes as four grids (SDF.cu:45-139 numbering): vertices (nx+1, ny+1, nz+1), x-edge nodes (2nx, ny+1,
 // nz+1), y-edge nodes (2ny, nz+1, nx+1) and z-edge nodes (2nz, nx+1, ny+1), each linear with its first dimension
@@ -457,75 +648,151 @@ struct NodeBricks {
     __host__ __device__ uint32_t waves() const { return first[4]; }
     // node of lane `lane` of brick-wave w, or ~0u past the grid's edge
     __device__ uint32_t node(uint32_t w, uint32_t lane) const {
-        if (w >= first[4]) return ~0u;
-        int c = 0;
-        while (w >= first[c + 1]) ++c;
-        const uint32_t b = w - first[c];
-        const uint32_t i0 = (b % nb[c][0]) * 4 + (lane & 3u);
-        const uint32_t i1 = ((b / nb[c][0]) % nb[c][1]) * 4 + ((lane >> 2) & 3u);
-        const uint32_t i2 = (b / (nb[c][0] * nb[c][1])) * 4 + (lane >> 4);
-        if (i0 >= dim[c][0] || i1 >= dim[c][1] || i2 >= dim[c][2]) return ~0u;
-        return base[c] + (i2 * dim[c][1] + i1) * dim[c][0] + i0;
+        uint32_t n = ~0u;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {  // unrolled: the arrays stay in registers
+            if (w < first[c] || w >= first[c + 1]) continue;
+            const uint32_t b = w - first[c];
+            const uint32_t i0 = (b % nb[c][0]) * 4 + (lane & 3u);
+            const uint32_t i1 = ((b / nb[c][0]) % nb[c][1]) * 4 + ((lane >> 2) & 3u);
+            const uint32_t i2 = (b / (nb[c][0] * nb[c][1])) * 4 + (lane >> 4);
+            if (i0 < dim[c][0] && i1 < dim[c][1] && i2 < dim[c][2]) n = base[c] + (i2 * dim[c][1] + i1) * dim[c][0] + i0;
+        }
+        return n;
     }
 };
 
-// Field 0 of a mesh body: one thread per map node, a wave per brick of nodes (NodeBricks). A block stages
-// kMeshTile triangles at a time in LDS (read as broadcasts); each wave skips a cluster of kMeshCluster triangles when
-// every lane's node is provably farther from the cluster's bounding sphere than from a triangle already seen (or than
-// the farthest point of some cluster, the bound before any triangle is seen). The winner is the least squared distance, ties to the smaller mesh index - the
-// first minimum of the reference's order - so the skipped clusters cannot change it: the test keeps a margin of
-// 4e-5 (|p - c| + r)^2 over the rounding of the squared distances, which stays below 1e-6 of that scale. The
-// winner's closest point and feature give the sign: negative where (p - closest) points against the feature's normal.
-__global__ void __launch_bounds__(kMeshTile) k_mesh_field0(MeshDev mesh, MapDev map, float sign, float tol,
-                                                          float* nodes0) {
-    __shared__ float4 sTri[4 * kMeshTile];
+// Sphere about each triangle, its centre the vertices' mean, the vertices relative to it; the radius rounded up.
+__global__ void __launch_bounds__(kTile) k_mesh_spheres(MeshDev mesh, float4* out) {
+    const uint32_t t = blockIdx.x * kTile + threadIdx.x;
+    if (t >= mesh.triCount) return;
+    const float4* r = mesh.tri + 4 * (size_t)t;
+    const f3 x0 = ld3(r[0]), e0 = ld3(r[1]), e1 = ld3(r[2]);
+    const f3 c = x0 + (e0 + e1) * (1.0f / 3.0f);
+    const f3 a = x0 - c, b0 = a + e0, b1 = a + e1;
+    const float rad = sqrtf(fmaxf(gdot(a, a), fmaxf(gdot(b0, b0), gdot(b1, b1))));
+    out[t] = make_float4(c.x, c.y, c.z, rad * 1.00001f);
+}
+
+// Field 0 of a mesh body: a block per brick of 64 nodes (NodeBricks), a lane per node in each of its kWaves waves, which
+// share the triangles. The winner is the least squared distance, ties to the smaller mesh index - the first minimum of
+// the reference's order - so triangles that are provably farther may be left out: those in a sphere (c, r) with
+// |p - c| > r A + s B, s^2 the least squared distance seen (or the bound before any: no triangle of a cluster is farther
+// than u = |p - c| + r). With kFarA and kFarB that gives (|p - c| - r)^2 >= s^2 + 4e-5 u^2, and the rounding of the
+// squared distances stays below 1e-6 u^2.
+//   1. every node's bound over all clusters, and the triangles of the cluster nearest to the brick, so that s starts
+//      near the minimum;
+//   2. 64 triangles at a time, a lane per triangle: its sphere against the brick's with the largest s of the nodes;
+//   3. what is left, triangle by triangle: each node's sphere test, then the distance where some node needs it (40
+//      instructions and more, as the lanes fall into different regions).
+// The triangles are read at wave-uniform addresses (scalar loads). Most bricks test a few dozen triangles, but those
+// near the middle of a round body test them all, and a wave to itself took 2.7 ms for one of 5,120 triangles, the whole
+// kernel with it (0.36 ms of VALU work); 406k nodes now take 0.97 ms, 0.63 ms of it VALU work. The winner's closest point and feature give the sign: negative
+// where (p - closest) points against the feature's normal.
+constexpr float kFarA = 1.01289f, kFarB = 1.00646f;  // (1 + e) / (1 - e) and 1 / (1 - e), e = 6.4e-3, rounded up
+template <uint32_t kWaves>
+__global__ void __launch_bounds__(kWaves * kWave) k_mesh_field0(MeshDev mesh, const float4* __restrict__ spheres,
+                                                               MapDev map, float sign, float tol, float* nodes0) {
+    __shared__ float sBest[kWaves][kWave];
+    __shared__ uint32_t sIdx[kWaves][kWave], sPos[kWaves][kWave];
     const NodeBricks bricks(map);
-    const uint32_t t = blockIdx.x * kMeshTile + threadIdx.x;
-    const uint32_t l = bricks.node(t / 64u, t % 64u);
+    const uint32_t lane = threadIdx.x & (kWave - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const uint32_t l = bricks.node(blockIdx.x, lane);
     const bool live = l < map.nodeCount;
-    const f3 p = live ? node_position(map, l) : mk3(0.0f, 0.0f, 0.0f);
+    const unsigned long long lives = __ballot(live);  // (the same in every wave)
+    if (lives == 0ull) return;
+    const int lead = __ffsll((long long)lives) - 1;
+    f3 p = live ? node_position(map, l) : mk3(0.0f, 0.0f, 0.0f);
+    p = mk3(live ? p.x : __shfl(p.x, lead, kWave), live ? p.y : __shfl(p.y, lead, kWave),
+            live ? p.z : __shfl(p.z, lead, kWave));  // lanes without a node follow the first one that has one
+    // sphere about the brick's nodes
+    auto most = [](float v) { return wave_max(v); };
+    const f3 mid = mk3(0.5f * (most(p.x) - most(-p.x)), 0.5f * (most(p.y) - most(-p.y)), 0.5f * (most(p.z) - most(-p.z)));
+    const float brick = 1.00001f * sqrtf(most(length2(p - mid)));
     const uint32_t clusters = (mesh.triCount + kMeshCluster - 1) / kMeshCluster;
-    // |p - c| and the margin of one cluster
-    auto reach = [&](uint32_t c, float& dc, float& r) {
+    float best = INFINITY, s = INFINITY;  // s: kFarB times the root of the least squared distance or bound, rounded up
+    uint32_t bestIdx = 0xffffffffu, bestPos = mesh.firstPos;
+    auto reach_of = [](float d2) { return kFarB * 1.00001f * __builtin_amdgcn_sqrtf(d2); };
+    auto test = [&](uint32_t pos) {
+        const float4* r = mesh.tri + 4 * (size_t)pos;
+        const float4 r3 = r[3];
+        const float d2 = tri_d2<false>(r[0], r[1], r[2], r3, p, nullptr, nullptr);
+        const uint32_t idx = __float_as_uint(r3.w);
+        if (d2 < best || (d2 == best && idx < bestIdx)) {
+            best = d2;
+            bestIdx = idx;
+            bestPos = pos;
+            s = fminf(s, reach_of(d2));
+        }
+    };
+    // the least of the waves' values of `v`, lane by lane
+    auto least = [&](float v) {
+        if (kWaves == 1) return v;
+        sBest[w][lane] = v;
+        __syncthreads();
+#pragma unroll
+        for (uint32_t q = 0; q < kWaves; ++q) v = fminf(v, sBest[q][lane]);
+        __syncthreads();
+        return v;
+    };
+    float bound = INFINITY;
+    for (uint32_t c = w; c < clusters; c += kWaves) {
         const float4 sp = mesh.spheres[c];
         const f3 d = p - mk3(sp.x, sp.y, sp.z);
-        dc = sqrtf(gdot(d, d));
-        r = sp.w;
-    };
-    float bound = INFINITY;  // no triangle is farther than (|p - c| + r)^2 from p, for every cluster c
-    for (uint32_t c = 0; c < clusters; ++c) {
-        float dc, r;
-        reach(c, dc, r);
-        const float u = dc + r;
-        bound = fminf(bound, u * u);
+        bound = fminf(bound, __builtin_amdgcn_sqrtf(length2(d)) + sp.w);
     }
-    float best = INFINITY;
-    uint32_t bestIdx = 0xffffffffu, bestPos = mesh.firstPos;
-    for (uint32_t base = 0; base < mesh.triCount; base += kMeshTile) {
-        __syncthreads();
-        const uint32_t tl = base + threadIdx.x;
-        if (tl < mesh.triCount)
-            for (int q = 0; q < 4; ++q) sTri[4 * threadIdx.x + q] = mesh.tri[4 * (size_t)tl + q];
-        __syncthreads();
-        for (uint32_t cb = 0; cb < kMeshTile && base + cb < mesh.triCount; cb += kMeshCluster) {
-            float dc, r;
-            reach((base + cb) / kMeshCluster, dc, r);
-            const float lb = dc - r, u = dc + r;
-            const float lim = fminf(best, bound) + 4e-5f * (u * u);
-            const bool skip = !live || (lb > 0.0f && lb * lb > lim);
-            if (__all(skip)) continue;  // wave-uniform
-            const uint32_t n = min(kMeshCluster, mesh.triCount - (base + cb));
-            for (uint32_t k = cb; k < cb + n; ++k) {
-                const float4 r3 = sTri[4 * k + 3];
-                const float d2 = tri_d2<false>(sTri[4 * k], sTri[4 * k + 1], sTri[4 * k + 2], r3, p, nullptr, nullptr);
-                const uint32_t idx = __float_as_uint(r3.w);
-                if (d2 < best || (d2 == best && idx < bestIdx)) {
-                    best = d2;
-                    bestIdx = idx;
-                    bestPos = base + k;
-                }
+    bound = bound * bound * 1.00001f;
+    // the cluster nearest to the brick: lanes over clusters
+    float near = INFINITY;
+    uint32_t nearest = 0;
+    for (uint32_t c = lane; c < clusters; c += kWave) {
+        const float4 sp = mesh.spheres[c];
+        const float u = __builtin_amdgcn_sqrtf(length2(mid - mk3(sp.x, sp.y, sp.z))) + sp.w;
+        nearest = u < near ? c : nearest;
+        near = fminf(near, u);
+    }
+    const unsigned long long at = __ballot(near == -most(-near));
+    const uint32_t first = __builtin_amdgcn_readfirstlane((uint32_t)__shfl((int)nearest, at ? __ffsll((long long)at) - 1 : 0,
+                                                                           kWave));
+    s = reach_of(least(bound));
+    for (uint32_t q = w; q < kMeshCluster; q += kWaves)
+        if (first * kMeshCluster + q < mesh.triCount) test(first * kMeshCluster + q);
+    s = fminf(s, reach_of(least(best)));
+    float smax = most(s);
+    for (uint32_t c = w; c < clusters; c += kWaves) {
+        const uint32_t t = c * kMeshCluster + lane;
+        bool keep = false, tested = false;
+        if (t < mesh.triCount) {
+            const float4 sp = spheres[t];
+            const f3 d = mid - mk3(sp.x, sp.y, sp.z);
+            const float reach = 1.00001f * (kFarA * sp.w + smax + brick);
+            keep = !(length2(d) > reach * reach);  // (kept where the reach is not a number)
+        }
+        for (unsigned long long left = __ballot(keep); left; left &= left - 1ull) {
+            const uint32_t pos = __builtin_amdgcn_readfirstlane(c * kMeshCluster + (uint32_t)__ffsll((long long)left) - 1u);
+            const float4 sp = spheres[pos];
+            const f3 d = p - mk3(sp.x, sp.y, sp.z);
+            const float reach = kFarA * sp.w + s;
+            if (!__all(length2(d) > reach * reach)) {  // wave-uniform
+                test(pos);
+                tested = true;
             }
         }
+        if (tested) smax = most(s);
+    }
+    if (kWaves > 1) {
+        sBest[w][lane] = best;
+        sIdx[w][lane] = bestIdx;
+        sPos[w][lane] = bestPos;
+        __syncthreads();
+        if (w != 0) return;
+#pragma unroll
+        for (uint32_t q = 1; q < kWaves; ++q)
+            if (sBest[q][lane] < best || (sBest[q][lane] == best && sIdx[q][lane] < bestIdx)) {
+                best = sBest[q][lane];
+                bestIdx = sIdx[q][lane];
+                bestPos = sPos[q][lane];
+            }
     }
     if (!live) return;
     const float4* rp = mesh.tri + 4 * (size_t)bestPos;
@@ -537,10 +804,22 @@ __global__ void __launch_bounds__(kMeshTile) k_mesh_field0(MeshDev mesh, MapDev 
     nodes0[l] = sign * (d - tol);
 }
 
-void launch_mesh_field0(hipStream_t st, const MeshDev& mesh, const MapDev& map, float sign, float tol, float* nodes0) {
-    const uint32_t waves = NodeBricks(map).waves();
-    hipLaunchKernelGGL(k_mesh_field0, dim3((waves * 64u + kMeshTile - 1) / kMeshTile), dim3(kMeshTile), 0, st, mesh,
-                       map, sign, tol, nodes0);
+// A wave per cluster of the brick, up to eight: fewer triangles leave the further ones nothing to do.
+void launch_mesh_field0(hipStream_t st, const MeshDev& mesh, float4* triSpheres, const MapDev& map, float sign, float tol,
+                        float* nodes0) {
+    const uint32_t bricks = NodeBricks(map).waves(), clusters = (mesh.triCount + kMeshCluster - 1) / kMeshCluster;
+    if (mesh.triCount)
+        hipLaunchKernelGGL(k_mesh_spheres, dim3((mesh.triCount + kTile - 1) / kTile), dim3(kTile), 0, st, mesh, triSpheres);
+    const auto run = [&](auto kernel, uint32_t waves) {
+        hipLaunchKernelGGL(kernel, dim3(bricks), dim3(waves * kWave), 0, st, mesh, (const float4*)triSpheres, map, sign,
+                           tol, nodes0);
+    };
+    if (clusters >= 8)
+        run(k_mesh_field0<8>, 8);
+    else if (clusters >= 2)
+        run(k_mesh_field0<2>, 2);
+    else
+        run(k_mesh_field0<1>, 1);
 }
 
 // ---- ParticleSampler::SampleMeshVolume (Utility/Sampler/ParticleSampler.cpp:7-91) ---------------------------------

@@ -204,9 +204,12 @@ int static_scratch_address(int device, uint32_t** out);
 
 // ---- boundary.hip ---------------------------------------------------------------------------------------------
 void launch_map_field0(hipStream_t st, const ShapeDev& shape, const MapDev& map, float* nodes0);
-void launch_mesh_field0(hipStream_t st, const MeshDev& mesh, const MapDev& map, float sign, float tol, float* nodes0);
+// triSpheres: room for a sphere per triangle
+void launch_mesh_field0(hipStream_t st, const MeshDev& mesh, float4* triSpheres, const MapDev& map, float sign, float tol,
+                        float* nodes0);
+uint32_t map_scratch_words(const MapDev& map);
 void launch_map_field1(hipStream_t st, const MapDev& map, const float* nodes0, float* nodes1, const KTabHost& kt,
-                       const float* glx, const float* glw);
+                       const float* glx, const float* glw, uint32_t* scratch, uint32_t numCU);
 // flags[c] = 1 where candidate c of the lattice lies inside (field 0 < 0), c = (k * ny + j) * nx + i
 void launch_sample_flags(hipStream_t st, const SampleGrid& g, const MapDev& map, const float* nodes0, uint32_t* flags);
 void launch_sample_scatter(hipStream_t st, const SampleGrid& g, const uint32_t* flags, const uint32_t* offsets,

@@ -290,7 +290,7 @@ extern "C" int vfd_sample_mesh_volume(const vfd_mesh* mesh, const float* transfo
         ~DrainGuard() { (void)hipStreamSynchronize(s); }
     } drain{st};
     if ((e = dTri.alloc(prep.tri.size())) != hipSuccess || (e = dNrm.alloc(prep.normals.size())) != hipSuccess ||
-        (e = dSph.alloc(prep.spheres.size())) != hipSuccess ||
+        (e = dSph.alloc(prep.spheres.size() + 4 * (size_t)nt)) != hipSuccess ||
         (e = dNodes.alloc(map.nodeCount)) != hipSuccess || (e = dX.alloc(xs.size())) != hipSuccess ||
         (e = dY.alloc(ys.size())) != hipSuccess || (e = dZ.alloc(zs.size())) != hipSuccess ||
         (e = dFlags.alloc(n)) != hipSuccess || (e = dOffs.alloc(n)) != hipSuccess ||
@@ -307,7 +307,7 @@ extern "C" int vfd_sample_mesh_volume(const vfd_mesh* mesh, const float* transfo
         if ((e = hipMemcpyAsync(u.d, u.h, u.bytes, hipMemcpyHostToDevice, st)) != hipSuccess)
             return set_error(VFD_ERROR_HIP, std::string("sampler upload: ") + hipGetErrorString(e));
     const MeshDev md{(const float4*)dTri.p, dNrm.p, (const float4*)dSph.p, nt, prep.firstPos};
-    launch_mesh_field0(st, md, map, inverted ? -1.0f : 1.0f, 0.0f, dNodes.p);
+    launch_mesh_field0(st, md, (float4*)(dSph.p + prep.spheres.size()), map, inverted ? -1.0f : 1.0f, 0.0f, dNodes.p);
     map.nodes0 = dNodes.p;
     const SampleGrid g{dX.p, dY.p, dZ.p, (uint32_t)xs.size(), (uint32_t)ys.size(), (uint32_t)zs.size(), mode, radius,
                        diameter, shiftX};

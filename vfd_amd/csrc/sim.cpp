@@ -394,6 +394,7 @@ public:
     KernelTable kt;
     DevBuf<float2> dTab;
     DevBuf<float> dHalton, dGlx, dGlw;
+    DevBuf<uint32_t> mapScratch;  // nodes of the map being built that have a volume (kept for the next body)
     DevBuf<float> dMcTab;
     DevBuf<uint32_t> dMcOff;
     std::vector<float> mcTab;     // host copies of this step's tables (kept until the next step's upload)
@@ -894,7 +895,7 @@ public:
         DevBuf<float> tri, nrm, sph;
         VFD_TRY(tri.alloc(prep.tri.size()));
         VFD_TRY(nrm.alloc(prep.normals.size()));
-        VFD_TRY(sph.alloc(prep.spheres.size()));
+        VFD_TRY(sph.alloc(prep.spheres.size() + 4 * (size_t)mesh.TriangleCount));  // the clusters', the triangles'
         // destroyed before the buffers and `prep`: every return, early error ones included, drains the uploads and
         // the distance kernel that read them
         struct DrainGuard {
@@ -915,7 +916,9 @@ public:
         for (int a = 0; a < 3; ++a) d.CollisionMapResolution[a] = b.CollisionMapResolution[a];
         const float sign = b.Inverted ? -1.0f : 1.0f;
         return add_body(s, b.CollisionMapResolution, lo, hi, d,
-                        [&](const MapDev& m, float* n0) { launch_mesh_field0(stream, md, m, sign, tol, n0); });
+                        [&](const MapDev& m, float* n0) {
+                            launch_mesh_field0(stream, md, (float4*)(sph.p + prep.spheres.size()), m, sign, tol, n0);
+                        });
     }
 
     // Common tail of both: map geometry (SDF.cu:8-14), node storage, field 0 by `field0`, field 1 (the boundary
@@ -945,6 +948,7 @@ public:
                       2 * (nx * (ny + 1) * (nz + 1) + (nx + 1) * ny * (nz + 1) + (nx + 1) * (ny + 1) * nz);
         int rc = body->n0.alloc(m.nodeCount);
         if (rc == VFD_OK) rc = body->n1.alloc(m.nodeCount);
+        if (rc == VFD_OK) rc = mapScratch.alloc(map_scratch_words(m));
         if (rc != VFD_OK) {
             delete body;
             return rc;
@@ -952,7 +956,7 @@ public:
         m.nodes0 = body->n0.p;
         m.nodes1 = body->n1.p;
         field0(m, body->n0.p);
-        launch_map_field1(stream, m, body->n0.p, body->n1.p, ktab(), dGlx.p, dGlw.p);
+        launch_map_field1(stream, m, body->n0.p, body->n1.p, ktab(), dGlx.p, dGlw.p, mapScratch.p, numCU);
         hipError_t e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(stream);
         if (e != hipSuccess) {
