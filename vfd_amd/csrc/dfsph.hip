@@ -10,6 +10,8 @@
 //     host only polls every few iterations instead of copying a scalar back per iteration;
 //   - ClearAcceleration is fused into the divergence finaliser; the position update into the pressure finaliser.
 // Floating-point expressions keep the reference's association order (no implicit contraction; -ffp-contract=off).
+#include <algorithm>
+
 #include "terms.h"
 
 namespace vfd {
@@ -640,64 +642,108 @@ void launch_visc_apply(const Launch& L, const Fields& F) {
 }
 
 // ---- Monte-Carlo surface tension (SolveSurfaceTension, DFSPHImplementation.cu:810-839; Zorilla et al. 2020) -----
-// ComputeSurfaceTensionClassificationKernel (DFSPHKernels.cu:881-958) with ClassifyParticleConfigurable (:864-872)
+// ComputeSurfaceTensionClassificationKernel (DFSPHKernels.cu:881-958) with ClassifyParticleConfigurable (:864-872), in
+// two launches: every particle is classified (one thread each), and the surface candidates are sampled, a wave each, a
+// lane per Monte-Carlo sample. A thread that walked the samples of its candidate against its neighbours was one serial
+// chain of up to 50 x 40 distance tests while its wave's other lanes waited: 214 us for 990 particles and 132 us for
+// 250k; both launches together now take 14 and 95 us.
+// F.surface: [0] the number of candidates, [1 + k] their slots (any order: each is sampled by itself).
 __global__ void __launch_bounds__(kTile) k_st_classify(const SceneParams* __restrict__ P,
                                                        const uint32_t* __restrict__ tileScene, Fields F,
                                                        uint32_t cap) {
     const TileCtx c = tile_ctx(tileScene, P);
     const SceneParams& p = P[c.s];
-    if (!c.valid || !p.enableST) return;
-    const float R = p.R;
-    const f3 xi = ld3(F.pos[c.i]);
-    const uint32_t n = F.nbrCount[c.i];
-    F.nMC[c.i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (n == 0) {
-        F.kMC[c.i] = 1.0f / R;
-        return;
-    }
-    // neighbour positions are loaded kStBatch at a time so that their latencies overlap; sums stay in list order
-    constexpr uint32_t kStBatch = 8;
-    f3 com = mk3(0.0f, 0.0f, 0.0f);
-    for (uint32_t j0 = 0; j0 < n; j0 += kStBatch) {
-        f3 xb[kStBatch];
+    bool candidate = false;
+    if (c.valid && p.enableST) {
+        const float R = p.R;
+        const f3 xi = ld3(F.pos[c.i]);
+        const uint32_t n = F.nbrCount[c.i];
+        F.nMC[c.i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (n == 0) {
+            F.kMC[c.i] = 1.0f / R;
+        } else {
+            // neighbour positions are loaded kStBatch at a time so that their latencies overlap; sums in list order
+            constexpr uint32_t kStBatch = 8;
+            f3 com = mk3(0.0f, 0.0f, 0.0f);
+            for (uint32_t j0 = 0; j0 < n; j0 += kStBatch) {
+                f3 xb[kStBatch];
 #pragma unroll
-        for (uint32_t u = 0; u < kStBatch; ++u) xb[u] = ld3(F.pos[nbr(F, cap, c.i, min(j0 + u, n - 1u))]);
+                for (uint32_t u = 0; u < kStBatch; ++u) xb[u] = ld3(F.pos[nbr(F, cap, c.i, min(j0 + u, n - 1u))]);
 #pragma unroll
-        for (uint32_t u = 0; u < kStBatch; ++u)
-            if (j0 + u < n) com = com + (xb[u] - xi);
-    }
-    com = com / R;
-    const float ci = length(com) / (float)n;
-    if (!((float)n <= p.slope * ci + p.constant + 0.0f)) return;
-    const uint32_t S = F.state[c.s].S;
-    const uint32_t s = F.id[c.i] * S / 3u * 3u;
-    const float rr = p.NR / p.r;
-    const float lim = rr * rr * p.R2;
-    uint32_t count = 0;
-    f3 nsum = mk3(0.0f, 0.0f, 0.0f);
-    for (uint32_t q = 0; q < S; ++q) {
-        const uint32_t i3 = s + 3u * q;
-        const f3 pt = R * mk3(F.halton[i3 % kHaltonFloats], F.halton[(i3 + 1u) % kHaltonFloats],
-                              F.halton[(i3 + 2u) % kHaltonFloats]);
-        bool covered = false;
-        for (uint32_t j0 = 0; j0 < n && !covered; j0 += kStBatch) {
-            f3 xb[kStBatch];
-#pragma unroll
-            for (uint32_t u = 0; u < kStBatch; ++u) xb[u] = ld3(F.pos[nbr(F, cap, c.i, min(j0 + u, n - 1u))]);
-#pragma unroll
-            for (uint32_t u = 0; u < kStBatch; ++u)
-                if (j0 + u < n && length2(pt - (xb[u] - xi)) <= lim) covered = true;
+                for (uint32_t u = 0; u < kStBatch; ++u)
+                    if (j0 + u < n) com = com + (xb[u] - xi);
+            }
+            com = com / R;
+            const float ci = length(com) / (float)n;
+            candidate = (float)n <= p.slope * ci + p.constant + 0.0f;
         }
-        if (covered) continue;
-        nsum = nsum + pt;
-        ++count;
     }
-    if (count > 0) {
-        if (length2(nsum) > 0.0f) nsum = normalize(nsum);
-        F.nMC[c.i] = st4(nsum);
-        F.kMC[c.i] = 1.0f / R * -2.0f * sqrtf(1.0f - p.NR * p.NR / (p.r * p.r)) * F.mcTab[F.mcOff[c.s] + count];
-    } else {
-        F.kMC[c.i] = 0.0f;
+    const unsigned long long b = __ballot(candidate);
+    if (b == 0ull) return;
+    const int lane = threadIdx.x & (kWave - 1), first = __ffsll((long long)b) - 1;
+    uint32_t at = 0;
+    if (lane == first) at = atomicAdd(&F.surface[0], (uint32_t)__popcll(b));
+    at = (uint32_t)__shfl((int)at, first, kWave);
+    if (candidate) F.surface[1 + at + (uint32_t)__popcll(b & ((1ull << lane) - 1ull))] = c.i;
+}
+
+constexpr uint32_t kStWaves = kTile / kWave;
+__global__ void __launch_bounds__(kTile) k_st_sample(const SceneParams* __restrict__ P,
+                                                     const uint32_t* __restrict__ tileScene, Fields F, uint32_t cap) {
+    constexpr uint32_t kRows = (kMaxNeighbors + 7u) / 8u * 8u;
+    __shared__ float4 sRel[kStWaves][kRows];
+    const uint32_t lane = threadIdx.x & (kWave - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const uint32_t candidates = F.surface[0];
+    float4* rel = sRel[w];
+    for (uint32_t k = blockIdx.x * kStWaves + w; k < candidates; k += gridDim.x * kStWaves) {  // wave-uniform
+        const uint32_t i = __builtin_amdgcn_readfirstlane(F.surface[1 + k]);
+        const uint32_t scene = tileScene[i / kTile];
+        const SceneParams& p = P[scene];
+        const float R = p.R;
+        const f3 xi = ld3(F.pos[i]);
+        const uint32_t n = F.nbrCount[i];
+        const uint32_t S = F.state[scene].S;
+        const uint32_t s = F.id[i] * S / 3u * 3u;
+        const float rr = p.NR / p.r;
+        const float lim = rr * rr * p.R2;
+        // neighbours relative to the particle; past the list's end its last one again, which covers nothing new
+        for (uint32_t j = lane; j < kRows; j += kWave) rel[j] = st4(ld3(F.pos[nbr(F, cap, i, min(j, n - 1u))]) - xi);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        uint32_t count = 0;
+        f3 nsum = mk3(0.0f, 0.0f, 0.0f);
+        for (uint32_t q0 = 0; q0 < S; q0 += kWave) {
+            const bool in = q0 + lane < S;
+            const uint32_t i3 = s + 3u * (q0 + lane);
+            const f3 pt = R * mk3(F.halton[i3 % kHaltonFloats], F.halton[(i3 + 1u) % kHaltonFloats],
+                                  F.halton[(i3 + 2u) % kHaltonFloats]);
+            bool open = in;
+            for (uint32_t j0 = 0; j0 < n && __any(open); j0 += 8) {
+                f3 x[8];
+#pragma unroll
+                for (uint32_t u = 0; u < 8; ++u) x[u] = ld3(rel[j0 + u]);
+#pragma unroll
+                for (uint32_t u = 0; u < 8; ++u) open = open && !(length2(pt - x[u]) <= lim);
+            }
+            // the uncovered samples in their order
+            const unsigned long long left = __ballot(open);
+            count += (uint32_t)__popcll(left);
+            for (unsigned long long b = left; b; b &= b - 1ull) {
+                const int q = __ffsll((long long)b) - 1;
+                nsum = nsum + mk3(__shfl(pt.x, q, kWave), __shfl(pt.y, q, kWave), __shfl(pt.z, q, kWave));
+            }
+        }
+        if (lane == 0) {
+            if (count > 0) {
+                if (length2(nsum) > 0.0f) nsum = normalize(nsum);
+                F.nMC[i] = st4(nsum);
+                F.kMC[i] = 1.0f / R * -2.0f * sqrtf(1.0f - p.NR * p.NR / (p.r * p.r)) * F.mcTab[F.mcOff[scene] + count];
+            } else {
+                F.kMC[i] = 0.0f;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();  // the next candidate's positions follow this one's reads
     }
 }
 
@@ -715,15 +761,26 @@ __global__ void __launch_bounds__(kTile) k_st_normals(const SceneParams* __restr
     f3 nc = mk3(0.0f, 0.0f, 0.0f);
     float cc = 0.0f, cf = 0.0f;
     const uint32_t n = F.nbrCount[c.i];
-    for (uint32_t j = 0; j < n; ++j) {
-        const uint32_t t = nbr(F, cap, c.i, j);
-        const f3 nj = ld3(F.nMC[t]);
-        if (is_zero(nj)) continue;
-        const float dist = length(ld3(F.pos[t]) - xi);
-        const float num = 1.0f - dist / R;
-        nc = nc + nj * num;
-        cc += F.kMC[t] * num;
-        cf += num;
+    constexpr uint32_t kStBatch = 8;  // neighbours whose loads are in flight together; terms in list order
+    for (uint32_t j0 = 0; j0 < n; j0 += kStBatch) {
+        f3 nj[kStBatch], xj[kStBatch];
+        float kj[kStBatch];
+#pragma unroll
+        for (uint32_t u = 0; u < kStBatch; ++u) {
+            const uint32_t t = nbr(F, cap, c.i, min(j0 + u, n - 1u));
+            nj[u] = ld3(F.nMC[t]);
+            xj[u] = ld3(F.pos[t]);
+            kj[u] = F.kMC[t];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kStBatch; ++u) {
+            if (j0 + u >= n || is_zero(nj[u])) continue;
+            const float dist = length(xj[u] - xi);
+            const float num = 1.0f - dist / R;
+            nc = nc + nj[u] * num;
+            cc += kj[u] * num;
+            cf += num;
+        }
     }
     if (length2(nc) > 0.0f) nc = normalize(nc);
     f3 ns = (1.0f - sf) * ni + sf * nc;
@@ -761,7 +818,11 @@ __global__ void __launch_bounds__(kTile) k_st_blend(const SceneParams* __restric
 }
 
 void launch_surface_tension(const Launch& L, const Fields& F) {
+    launch_fill_u32(L.stream, F.surface, 0u, 1u);
     hipLaunchKernelGGL(k_st_classify, dim3(L.tiles), dim3(kTile), 0, L.stream, L.P, L.tileScene, F, L.capacity);
+    // enough waves for the chip (eight a SIMD); a tile has no more candidates than its 256 particles
+    hipLaunchKernelGGL(k_st_sample, dim3(std::min(L.tiles * kWave, 2048u)), dim3(kTile), 0, L.stream, L.P, L.tileScene, F,
+                       L.capacity);
     hipLaunchKernelGGL(k_st_normals, dim3(L.tiles), dim3(kTile), 0, L.stream, L.P, L.tileScene, F, L.capacity);
     hipLaunchKernelGGL(k_st_blend, dim3(L.tiles), dim3(kTile), 0, L.stream, L.P, L.tileScene, F);
 }

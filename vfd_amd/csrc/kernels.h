@@ -260,6 +260,7 @@ struct Fields {
     // curvature factor of the surface-tension classification, evaluated on the host for this step's S)
     const float* mcTab;
     const uint32_t* mcOff;
+    uint32_t* surface;  // [1 + capacity] surface tension: number of surface candidates, their slots
 };
 
 void launch_density_factor(const Launch& L, uint32_t groupTiles, const KTabHost& kt, const Fields& F);

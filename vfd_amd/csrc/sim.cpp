@@ -457,7 +457,7 @@ public:
     DevBuf<int> dMM, dMMPart;
     DevBuf<float4> pos, posNext, vel[2], dv[2], acc, ap, nMC, nS, xb, cgX, cgR, cgP, cgZ, cgAp;
     DevBuf<float> dk[2], density, factor, densAdv, kappa, kappaV, residuum, kMC, kS, vb, minv;
-    DevBuf<uint32_t> id[2], nbrCount, nbrList, cellOf, rank, tmpId, cellCount, cellStart, scanScratch, live;
+    DevBuf<uint32_t> id[2], nbrCount, nbrList, cellOf, rank, tmpId, surface, cellCount, cellStart, scanScratch, live;
     DevBuf<double> partials;
     DevBuf<float> partialsF;
     DevBuf<unsigned long long> nbStats;
@@ -1020,6 +1020,7 @@ public:
         for (auto* b : f1) VFD_TRY(b->alloc(c));
         DevBuf<uint32_t>* u1[] = {&id[0], &id[1], &nbrCount, &cellOf, &rank, &tmpId};
         for (auto* b : u1) VFD_TRY(b->alloc(c));
+        VFD_TRY(surface.alloc(c + 1));
         VFD_TRY(xb.alloc(c * kMaxBodies));
         VFD_TRY(vb.alloc(c * kMaxBodies));
         VFD_TRY(minv.alloc(c * 9));
@@ -1158,6 +1159,7 @@ public:
         F.haloIds = haloIds.p;
         F.state = dState.p;
         F.halton = dHalton.p;
+        F.surface = surface.p;
         return F;
     }
 
