@@ -116,8 +116,8 @@ typedef struct vfd_info {
 } vfd_info;
 
 /* Mirrors DFSPHDebugInfo (VFD/Source/Simulation/DFSPH/Structures/DFSPHDebugInfo.h:8-28). Phase timers are wall
- * milliseconds of the last step measured with HIP events (the reference uses steady_clock around synchronised
- * launches). The last four members are additions. */
+ * milliseconds of the last step between the starts of the phases' first kernels (the reference uses steady_clock around
+ * synchronised launches). The last four members are additions. */
 typedef struct vfd_debug_info {
     uint32_t IterationCount;
     uint32_t DivergenceSolverIterationCount;

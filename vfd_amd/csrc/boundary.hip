@@ -874,7 +874,9 @@ void launch_sample_scatter(hipStream_t st, const SampleGrid& g, const uint32_t* 
 __global__ void __launch_bounds__(kTile) k_boundary(const SceneParams* __restrict__ P,
                                                     const uint32_t* __restrict__ tileScene,
                                                     const MapDev* __restrict__ maps, float4* pos, float4* vel,
-                                                    float4* xbOut, float* vbOut, uint32_t capacity) {
+                                                    float4* xbOut, float* vbOut, uint32_t capacity,
+                                                    long long* stamps) {
+    note_time(stamps, kStampBase);
     const TileCtx c = tile_ctx(tileScene, P);
     if (!c.valid) return;
     const SceneParams& p = P[c.s];
@@ -937,7 +939,7 @@ __global__ void __launch_bounds__(kTile) k_boundary(const SceneParams* __restric
 
 void launch_boundary(const Launch& L, const MapDev* maps, float4* pos, float4* vel, float4* xb, float* vb) {
     hipLaunchKernelGGL(k_boundary, dim3(L.tiles), dim3(kTile), 0, L.stream, L.P, L.tileScene, maps, pos, vel, xb, vb,
-                       L.capacity);
+                       L.capacity, L.stamps);
 }
 
 // (I - n n^T) Hs / |g|: the derivative of the unit normal n = g / |g|, Hs = Hess(phi) as (xx, yy, zz, xy, xz, yz)

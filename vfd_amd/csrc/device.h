@@ -235,6 +235,11 @@ __device__ __forceinline__ void tile_loop(const TileGrid& tg, Body&& body) {
     }
 }
 
+// the time at which a phase's first kernel began (Launch::stamps)
+__device__ __forceinline__ void note_time(long long* stamps, int phase) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) stamps[phase] = wall_clock64();
+}
+
 // ---- neighbour groups (kGroupTiles tiles per kGroupSize-thread block) ---------------------------------------------
 // Thread group sub = threadIdx.x / kTile of a block works on tile kGroupTiles * g + sub of group g.
 __device__ __forceinline__ TileCtx tile_ctx4(uint32_t tile, bool ok, const uint32_t* tileScene,

@@ -94,7 +94,9 @@ constexpr int kFinishThreads = 1024;
 // One block; also counts the scenes that iterate into live[which] (and clears live[2], the viscosity count, at the
 // start of a step).
 __global__ void __launch_bounds__(kTile) k_jacobi_begin(const SceneParams* __restrict__ P, SceneState* state,
-                                                        uint32_t* live, uint32_t sceneCount, int which) {
+                                                        uint32_t* live, uint32_t sceneCount, int which,
+                                                        long long* stamps) {
+    if (which == 0) note_time(stamps, kStampDivergence);
     __shared__ uint32_t count;
     if (threadIdx.x == 0) count = 0;
     __syncthreads();
@@ -217,7 +219,8 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_div_final(const Sc
 }
 
 void launch_scene_init_div(const Launch& L, const Fields& F) {
-    hipLaunchKernelGGL(k_jacobi_begin, dim3(1), dim3(kTile), 0, L.stream, L.P, F.state, F.live, L.sceneCount, 0);
+    hipLaunchKernelGGL(k_jacobi_begin, dim3(1), dim3(kTile), 0, L.stream, L.P, F.state, F.live, L.sceneCount, 0,
+                       L.stamps);
 }
 void launch_div_init(const Launch& L, const KTabHost& kt, const Fields& F) {
     hipLaunchKernelGGL(k_div_init, dim3(L.gridGroups), dim3(kGroupSize), kLdsXV, L.stream, L.P, L.tileScene, kt, F, L.capacity,
@@ -323,7 +326,8 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_pres_final(const S
 }
 
 void launch_scene_init_pres(const Launch& L, const Fields& F) {
-    hipLaunchKernelGGL(k_jacobi_begin, dim3(1), dim3(kTile), 0, L.stream, L.P, F.state, F.live, L.sceneCount, 1);
+    hipLaunchKernelGGL(k_jacobi_begin, dim3(1), dim3(kTile), 0, L.stream, L.P, F.state, F.live, L.sceneCount, 1,
+                       L.stamps);
 }
 void launch_pres_init(const Launch& L, const KTabHost& kt, const Fields& F) {
     hipLaunchKernelGGL(k_pres_init, dim3(L.gridGroups), dim3(kGroupSize), kLdsXV, L.stream, L.P, L.tileScene, kt, F, L.capacity,
@@ -344,7 +348,9 @@ void launch_pres_final(const Launch& L, const KTabHost& kt, const Fields& F, int
 
 // ---- time step (ComputeTimeStepSize, DFSPHImplementation.cu:395-441) --------------------------------------------
 __global__ void __launch_bounds__(kTile) k_time_step(const SceneParams* __restrict__ P,
-                                                     const uint32_t* __restrict__ tileScene, Fields F, TileGrid tg) {
+                                                     const uint32_t* __restrict__ tileScene, Fields F, TileGrid tg,
+                                                     long long* stamps) {
+    note_time(stamps, kStampPressure);
     tile_loop(tg, [&](uint32_t tile) {
         const TileCtx c = tile_ctx(tile, tileScene, P);
         const SceneState& st = F.state[c.s];
@@ -402,6 +408,96 @@ void launch_frame_pack(hipStream_t s, uint32_t base, uint32_t count, const uint3
                                   x, v, a, out);
 }
 
+// ---- the step's report, restored particles, fields in the caller's order -------------------------------------------
+__global__ void __launch_bounds__(kTile) k_report(uint32_t sceneCount, const SceneState* __restrict__ state,
+                                                  const unsigned long long* __restrict__ nbStats,
+                                                  const uint32_t* __restrict__ haloStats,
+                                                  const uint32_t* __restrict__ words, const long long* stamps,
+                                                  StepReport* report, SceneReport* scenes) {
+    for (uint32_t s = threadIdx.x; s < sceneCount; s += kTile)
+        scenes[s] = SceneReport{state[s], nbStats[2 * s], nbStats[2 * s + 1]};
+    if (threadIdx.x == 0) {
+        StepReport r{words[kResidentAbortedAt], {haloStats[0], haloStats[1], haloStats[2]}, {}};
+        for (int k = 0; k < kStampEnd; ++k) r.stamps[k] = stamps[k];
+        r.stamps[kStampEnd] = wall_clock64();
+        *report = r;
+    }
+}
+void launch_report(const Launch& L, const SceneState* state, const unsigned long long* nbStats, const uint32_t* haloStats,
+                   const uint32_t* words, StepReport* report, SceneReport* scenes) {
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(kTile), 0, L.stream, L.sceneCount, state, nbStats, haloStats, words,
+                       (const long long*)L.stamps, report, scenes);
+}
+
+__global__ void __launch_bounds__(kTile) k_restore(const SceneParams* __restrict__ P,
+                                                   const uint32_t* __restrict__ tileScene, const float* __restrict__ x,
+                                                   const float* __restrict__ v, float4* pos, float4* posNext, float4* vel,
+                                                   float4* dv, float* dk, uint32_t* id) {
+    const TileCtx c = tile_ctx(tileScene, P);
+    const size_t k = 3 * (size_t)c.i;
+    const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const float4 xi = c.valid ? make_float4(x[k], x[k + 1], x[k + 2], 0.0f) : zero;
+    pos[c.i] = xi;
+    posNext[c.i] = xi;
+    vel[c.i] = c.valid ? make_float4(v[k], v[k + 1], v[k + 2], 0.0f) : zero;
+    dv[c.i] = zero;
+    dk[c.i] = 0.0f;
+    id[c.i] = c.valid ? c.i - P[c.s].base : 0u;
+}
+void launch_restore(const Launch& L, const float* x, const float* v, float4* pos, float4* posNext, float4* vel, float4* dv,
+                    float* dk, uint32_t* id) {
+    if (L.tiles)
+        hipLaunchKernelGGL(k_restore, dim3(L.tiles), dim3(kTile), 0, L.stream, L.P, L.tileScene, x, v, pos, posNext, vel,
+                           dv, dk, id);
+}
+
+__global__ void __launch_bounds__(kTile) k_gather4(uint32_t base, uint32_t count, const uint32_t* __restrict__ id,
+                                                   const float4* __restrict__ in, float* out) {
+    const uint32_t k = blockIdx.x * kTile + threadIdx.x;
+    if (k >= count) return;
+    const uint32_t j = id[base + k];
+    if (j >= count) return;  // ids of a scene are 0..count-1; anything else is not written
+    const float4 v = in[base + k];
+    float* o = out + 3 * (size_t)j;
+    o[0] = v.x, o[1] = v.y, o[2] = v.z;
+}
+__global__ void __launch_bounds__(kTile) k_gather1(uint32_t base, uint32_t count, const uint32_t* __restrict__ id,
+                                                   const float* __restrict__ in, uint32_t stride, float* out) {
+    const uint32_t k = blockIdx.x * kTile + threadIdx.x;
+    if (k >= count) return;
+    const uint32_t j = id[base + k];
+    if (j < count) out[(size_t)stride * j] = in[base + k];
+}
+__global__ void __launch_bounds__(kTile) k_scatter4(uint32_t base, uint32_t count, const uint32_t* __restrict__ id,
+                                                    const float* __restrict__ in, float4* out) {
+    const uint32_t k = blockIdx.x * kTile + threadIdx.x;
+    if (k >= count) return;
+    const uint32_t j = id[base + k];
+    if (j >= count) return;
+    out[base + k] = make_float4(in[3 * (size_t)j], in[3 * (size_t)j + 1], in[3 * (size_t)j + 2], 0.0f);
+}
+__global__ void __launch_bounds__(kTile) k_scatter1(uint32_t base, uint32_t count, const uint32_t* __restrict__ id,
+                                                    const float* __restrict__ in, float* out) {
+    const uint32_t k = blockIdx.x * kTile + threadIdx.x;
+    if (k >= count) return;
+    const uint32_t j = id[base + k];
+    if (j < count) out[base + k] = in[j];
+}
+static dim3 tiles_of(uint32_t count) { return dim3((count + kTile - 1) / kTile); }
+void launch_gather4(hipStream_t s, uint32_t base, uint32_t count, const uint32_t* id, const float4* in, float* out) {
+    if (count) hipLaunchKernelGGL(k_gather4, tiles_of(count), dim3(kTile), 0, s, base, count, id, in, out);
+}
+void launch_gather1(hipStream_t s, uint32_t base, uint32_t count, const uint32_t* id, const float* in, uint32_t stride,
+                    float* out) {
+    if (count) hipLaunchKernelGGL(k_gather1, tiles_of(count), dim3(kTile), 0, s, base, count, id, in, stride, out);
+}
+void launch_scatter4(hipStream_t s, uint32_t base, uint32_t count, const uint32_t* id, const float* in, float4* out) {
+    if (count) hipLaunchKernelGGL(k_scatter4, tiles_of(count), dim3(kTile), 0, s, base, count, id, in, out);
+}
+void launch_scatter1(hipStream_t s, uint32_t base, uint32_t count, const uint32_t* id, const float* in, float* out) {
+    if (count) hipLaunchKernelGGL(k_scatter1, tiles_of(count), dim3(kTile), 0, s, base, count, id, in, out);
+}
+
 // ComputeVelocityKernel (DFSPHKernels.cu:39-52)
 __global__ void __launch_bounds__(kTile) k_velocity(const SceneParams* __restrict__ P,
                                                     const uint32_t* __restrict__ tileScene, Fields F, TileGrid tg) {
@@ -413,7 +509,8 @@ __global__ void __launch_bounds__(kTile) k_velocity(const SceneParams* __restric
 }
 
 void launch_time_step(const Launch& L, const Fields& F) {
-    hipLaunchKernelGGL(k_time_step, dim3(L.gridAll), dim3(kTile), 0, L.stream, L.P, L.tileScene, F, TileGrid(L.tg));
+    hipLaunchKernelGGL(k_time_step, dim3(L.gridAll), dim3(kTile), 0, L.stream, L.P, L.tileScene, F, TileGrid(L.tg),
+                       L.stamps);
 }
 void launch_time_step_finish(const Launch& L, const Fields& F) {
     hipLaunchKernelGGL(k_time_step_finish, dim3(L.sceneCount), dim3(kTile), 0, L.stream, L.P, F);
@@ -427,7 +524,8 @@ void launch_velocity(const Launch& L, const Fields& F) {
 // block, right-hand side b = v (the boundary rhs term is dot(0, .) = 0) and initial guess x0 = v + dv.
 __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_visc_precond(const SceneParams* __restrict__ P,
                                                         const uint32_t* __restrict__ tileScene, KTabHost kh,
-                                                        Fields F, uint32_t cap, TileGrid tg) {
+                                                        Fields F, uint32_t cap, TileGrid tg, long long* stamps) {
+    note_time(stamps, kStampViscosity);
     VFD_HALO_KERNEL_PROLOGUE(kh)
     const LoadXQ load{F.pos, F.density, P[0].m};  // lo.w = m / rho_j
     group_loop<1>(tg, halo(F), rec, global_src(F, cap), load, [&](uint32_t tile, bool ok, const NbrSrc& src) {
@@ -612,7 +710,7 @@ __global__ void __launch_bounds__(kTile) k_visc_apply(const SceneParams* __restr
 
 void launch_visc_precond(const Launch& L, const KTabHost& kt, const Fields& F) {
     hipLaunchKernelGGL(k_visc_precond, dim3(L.gridGroups), dim3(kGroupSize), kLdsXS, L.stream, L.P, L.tileScene, kt, F,
-                       L.capacity, TileGrid(L.tg));
+                       L.capacity, TileGrid(L.tg), L.stamps);
 }
 void launch_cg_begin(const Launch& L, const KTabHost& kt, const Fields& F) {
     hipLaunchKernelGGL(k_cg_begin, dim3(L.gridGroups), dim3(kGroupSize), kLdsXSV, L.stream, L.P, L.tileScene, kt, F, L.capacity,
@@ -650,7 +748,8 @@ void launch_visc_apply(const Launch& L, const Fields& F) {
 // F.surface: [0] the number of candidates, [1 + k] their slots (any order: each is sampled by itself).
 __global__ void __launch_bounds__(kTile) k_st_classify(const SceneParams* __restrict__ P,
                                                        const uint32_t* __restrict__ tileScene, Fields F,
-                                                       uint32_t cap) {
+                                                       uint32_t cap, long long* stamps) {
+    note_time(stamps, kStampSurface);
     const TileCtx c = tile_ctx(tileScene, P);
     const SceneParams& p = P[c.s];
     bool candidate = false;
@@ -819,7 +918,7 @@ __global__ void __launch_bounds__(kTile) k_st_blend(const SceneParams* __restric
 
 void launch_surface_tension(const Launch& L, const Fields& F) {
     launch_fill_u32(L.stream, F.surface, 0u, 1u);
-    hipLaunchKernelGGL(k_st_classify, dim3(L.tiles), dim3(kTile), 0, L.stream, L.P, L.tileScene, F, L.capacity);
+    hipLaunchKernelGGL(k_st_classify, dim3(L.tiles), dim3(kTile), 0, L.stream, L.P, L.tileScene, F, L.capacity, L.stamps);
     // enough waves for the chip (eight a SIMD); a tile has no more candidates than its 256 particles
     hipLaunchKernelGGL(k_st_sample, dim3(std::min(L.tiles * kWave, 2048u)), dim3(kTile), 0, L.stream, L.P, L.tileScene, F,
                        L.capacity);

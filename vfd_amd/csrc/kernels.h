@@ -23,9 +23,29 @@ struct Launch {
     uint32_t grid2;              // persistent grid, 2 blocks per CU (80 KB LDS table)
     uint32_t gridGroups;         // persistent grid of kGroupSize-thread blocks (one group at a time), 1 per CU
     uint32_t groups;             // 8 * per / kGroupTiles
+    long long* stamps;           // device [kStampCount]: wall clock (100 MHz) at which each phase of the step began
     struct { uint32_t tiles, per; } tg;  // per = tiles of one XCD chunk, a multiple of 4
     // groups of `tiles` tiles, those of no particles in the chunks' ends included
     uint32_t group_count(uint32_t tiles) const { return 8u * (tg.per / tiles); }
+};
+
+// Phases whose first kernel notes the time: a step's phase timers without events on the stream (each costs it about
+// 5 us).
+enum { kStampStart = 0, kStampBase, kStampDivergence, kStampSurface, kStampViscosity, kStampPressure, kStampEnd,
+       kStampCount };
+// What the host reads at the end of a step, written by one kernel into pinned host memory.
+struct SceneReport {
+    SceneState state;
+    unsigned long long neighbors, maxNeighbors;
+};
+struct StepReport {
+    uint32_t aborted, halo[3];  // a resident solve was aborted; halo statistics
+    long long stamps[kStampCount];
+};
+// Up to this many scenes' grids travel to the device as a kernel argument.
+constexpr uint32_t kGridArgs = 4;
+struct GridArgs {
+    SceneGrid g[kGridArgs];
 };
 
 // ---- adjoint.hip -----------------------------------------------------------------------------------------------
@@ -172,7 +192,10 @@ struct KTabHost {
 uint32_t scan_scratch_words(uint32_t n);
 void exclusive_scan(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* scratch, hipStream_t st);
 void launch_fill_u32(hipStream_t st, uint32_t* p, uint32_t v, uint32_t n);
+// mm: 6 bounds per scene, in memory that the host reads
 void launch_minmax(const Launch& L, const float4* pos, int* part, int* mm);
+// clears the cell counts and, with args, writes the scenes' grids (at most kGridArgs) to G
+void launch_sort_begin(const Launch& L, const GridArgs* args, SceneGrid* G, uint32_t* cellCount, uint32_t totalCells);
 void launch_sort(const Launch& L, const SceneGrid* G, uint32_t totalCells, const float4* posIn, const float4* velIn,
                  const float4* dvIn, const float* dkIn, const uint32_t* idIn, float4* posOut, float4* velOut,
                  float4* dvOut, float* dkOut, uint32_t* idOut, uint32_t* cellOf, uint32_t* rank, uint32_t* tmpId,
@@ -309,6 +332,17 @@ void launch_pres_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt,
 void launch_visc_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt, const Fields& F, const Resident& r,
                        const uint32_t* haloStats);
 int configure_solve_kernels();
-void launch_scene_state_init(const Launch& L, SceneState* state, const float* dt0);
+// report and its scenes in pinned host memory
+void launch_report(const Launch& L, const SceneState* state, const unsigned long long* nbStats, const uint32_t* haloStats,
+                   const uint32_t* words, StepReport* report, SceneReport* scenes);
+// Baked particles (three floats each, scene by scene in slot order) into the state a simulation starts from
+void launch_restore(const Launch& L, const float* x, const float* v, float4* pos, float4* posNext, float4* vel, float4* dv,
+                    float* dk, uint32_t* id);
+// A field of the particles in slots [base, base + count) to the original order (out[comps * id + c]) and back
+void launch_gather4(hipStream_t s, uint32_t base, uint32_t count, const uint32_t* id, const float4* in, float* out);
+void launch_gather1(hipStream_t s, uint32_t base, uint32_t count, const uint32_t* id, const float* in, uint32_t stride,
+                    float* out);
+void launch_scatter4(hipStream_t s, uint32_t base, uint32_t count, const uint32_t* id, const float* in, float4* out);
+void launch_scatter1(hipStream_t s, uint32_t base, uint32_t count, const uint32_t* id, const float* in, float* out);
 
 }  // namespace vfd

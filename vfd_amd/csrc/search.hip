@@ -35,7 +35,9 @@ __device__ __forceinline__ uint32_t cell_key(const SceneGrid& g, uint32_t cx, ui
 // ComputeMinMaxKernel (ParticleSearchKernels.cu:40-62): integer cell bounds floor(x / R). Each tile writes its
 // bounds to part[tile * 6 + a]; k_minmax_finish reduces a scene's tiles (no atomics on a single address).
 __global__ void __launch_bounds__(kTile) k_minmax(const float4* __restrict__ pos, const SceneParams* __restrict__ P,
-                                                  const uint32_t* __restrict__ tileScene, int* part) {
+                                                  const uint32_t* __restrict__ tileScene, int* part,
+                                                  long long* stamps) {
+    note_time(stamps, kStampStart);
     __shared__ int sh[kTile / kWave][6];
     const TileCtx c = tile_ctx(tileScene, P);
     const float R = P[c.s].R;
@@ -534,15 +536,25 @@ void launch_fill_u32(hipStream_t st, uint32_t* p, uint32_t v, uint32_t n) {
 
 // ---- host launchers ---------------------------------------------------------------------------------------------
 void launch_minmax(const Launch& L, const float4* pos, int* part, int* mm) {
-    hipLaunchKernelGGL(k_minmax, dim3(L.tiles), dim3(kTile), 0, L.stream, pos, L.P, L.tileScene, part);
+    hipLaunchKernelGGL(k_minmax, dim3(L.tiles), dim3(kTile), 0, L.stream, pos, L.P, L.tileScene, part, L.stamps);
     hipLaunchKernelGGL(k_minmax_finish, dim3(L.sceneCount), dim3(kTile), 0, L.stream, L.P, (const int*)part, mm);
+}
+
+__global__ void __launch_bounds__(kTile) k_sort_begin(GridArgs args, SceneGrid* G, uint32_t scenes, uint32_t* cellCount,
+                                                      uint32_t totalCells) {
+    const uint32_t i = blockIdx.x * kTile + threadIdx.x;
+    if (i < scenes) G[i] = args.g[i];
+    for (uint32_t c = i; c < totalCells; c += gridDim.x * kTile) cellCount[c] = 0u;
+}
+void launch_sort_begin(const Launch& L, const GridArgs* args, SceneGrid* G, uint32_t* cellCount, uint32_t totalCells) {
+    hipLaunchKernelGGL(k_sort_begin, dim3(std::min((totalCells + kTile - 1) / kTile, 2048u)), dim3(kTile), 0, L.stream,
+                       args ? *args : GridArgs{}, G, args ? L.sceneCount : 0u, cellCount, totalCells);
 }
 
 void launch_sort(const Launch& L, const SceneGrid* G, uint32_t totalCells, const float4* posIn, const float4* velIn,
                  const float4* dvIn, const float* dkIn, const uint32_t* idIn, float4* posOut, float4* velOut,
                  float4* dvOut, float* dkOut, uint32_t* idOut, uint32_t* cellOf, uint32_t* rank, uint32_t* tmpId,
                  uint32_t* cellCount, uint32_t* cellStart, uint32_t* scanScratch) {
-    hipLaunchKernelGGL(k_fill_u32, dim3((totalCells + 255) / 256), dim3(256), 0, L.stream, cellCount, 0u, totalCells);
     hipLaunchKernelGGL(k_insert, dim3(L.tiles), dim3(kTile), 0, L.stream, posIn, L.P, G, L.tileScene, cellOf, rank,
                        cellCount);
     exclusive_scan(cellCount, cellStart, totalCells, scanScratch, L.stream);

@@ -454,7 +454,7 @@ public:
     DevBuf<SceneState> dState;
     DevBuf<SceneGrid> dGrid;
     DevBuf<MapDev> dMaps;
-    DevBuf<int> dMM, dMMPart;
+    DevBuf<int> dMMPart;
     DevBuf<float4> pos, posNext, vel[2], dv[2], acc, ap, nMC, nS, xb, cgX, cgR, cgP, cgZ, cgAp;
     DevBuf<float> dk[2], density, factor, densAdv, kappa, kappaV, residuum, kMC, kS, vb, minv;
     DevBuf<uint32_t> id[2], nbrCount, nbrList, cellOf, rank, tmpId, surface, cellCount, cellStart, scanScratch, live;
@@ -518,7 +518,6 @@ public:
     }
     uint32_t haloLimit = VFD_DEFAULT_HALO_LIMIT;  // largest halo staged in LDS (tuning)
     uint32_t cellCap = 0;
-    hipEvent_t ev[8] = {};
     bool eventsMade = false;
     // solver polling: live[which] is copied into one of two pinned slots after each chunk of iterations
     uint32_t* hostLive = nullptr;  // [2]
@@ -542,7 +541,15 @@ public:
     // an aborted one (other work held the CUs past the barrier's limit) the step is taken again with launched
     // iterations, and so are the next kResidentPause steps.
     DevBuf<uint32_t> residentWords;
-    uint32_t* hostAborted = nullptr;  // pinned
+    // Pinned memory that kernels write and the host reads (or the host writes and a copy reads) without a copy of its
+    // own in between: the step's report and its scenes', the grid bounds, the grids of many scenes.
+    StepReport* report = nullptr;
+    SceneReport* sceneReport = nullptr;
+    int* hostBounds = nullptr;
+    SceneGrid* hostGrids = nullptr;
+    DevBuf<long long> stamps;
+    DevBuf<float> bakedX, bakedV;  // the baked particles, three floats a slot (Simulate restores them)
+    DevBuf<float> fieldStage;      // a field in the caller's order, on its way to or from the caller
     uint32_t residentPause = 0;
     static constexpr uint32_t kResidentPause = 64;
     // longest wait at a resident solve's barrier: 100 ms, or VFD_RESIDENT_WAIT_US from the environment (the aborted
@@ -650,10 +657,10 @@ public:
     ~Simulation() {
         join_worker();
         if (eventsMade) {
-            for (auto& e : ev) (void)hipEventDestroy(e);
             for (auto& e : pollEv) (void)hipEventDestroy(e);
         }
         if (hostLive) (void)hipHostFree(hostLive);
+        if (report) (void)hipHostFree(report);
         drop_graphs();
         if (copyStream) (void)hipStreamSynchronize(copyStream);
         for (Scene* s : sc) release_frames(*s);
@@ -743,11 +750,22 @@ public:
             sc.push_back(s);
         }
         VFD_TRY(build_tables(descs[0].ParticleRadius));
-        for (auto& e : ev) VFD_HIP(hipEventCreate(&e));
         for (auto& e : pollEv) VFD_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         eventsMade = true;
-        VFD_HIP(hipHostMalloc((void**)&hostLive, 4 * sizeof(uint32_t), hipHostMallocDefault));
-        hostAborted = hostLive + 2;
+        VFD_HIP(hipHostMalloc((void**)&hostLive, 2 * sizeof(uint32_t), hipHostMallocDefault));
+        {
+            const size_t scenes = sizeof(StepReport), grids = scenes + n * sizeof(SceneReport);
+            const size_t bounds = grids + n * sizeof(SceneGrid);
+            static_assert(sizeof(StepReport) % 8 == 0 && sizeof(SceneReport) % 8 == 0 && sizeof(SceneGrid) % 8 == 0,
+                          "parts of the pinned block stay aligned");
+            char* p = nullptr;
+            VFD_HIP(hipHostMalloc((void**)&p, bounds + 6 * n * sizeof(int), hipHostMallocDefault));
+            report = reinterpret_cast<StepReport*>(p);
+            sceneReport = reinterpret_cast<SceneReport*>(p + scenes);
+            hostGrids = reinterpret_cast<SceneGrid*>(p + grids);
+            hostBounds = reinterpret_cast<int*>(p + bounds);
+            VFD_TRY(stamps.alloc(kStampCount));
+        }
         if (const char* us = std::getenv("VFD_RESIDENT_WAIT_US"))
             residentWait = (uint32_t)std::min(std::max(std::atol(us), 0L), 1000000L) * 100u;
         VFD_HIP(hipStreamCreateWithFlags(&ownStream, hipStreamNonBlocking));
@@ -1007,7 +1025,6 @@ public:
         VFD_TRY(dState.alloc(S));
         VFD_TRY(dGrid.alloc(S));
         VFD_TRY(dMaps.alloc((size_t)S * kMaxBodies));
-        VFD_TRY(dMM.alloc((size_t)S * 6));
         VFD_TRY(dMMPart.alloc((size_t)std::max<uint32_t>(tiles, 1) * 6));
         VFD_TRY(live.alloc(4));
         VFD_TRY(residentWords.alloc(kResidentWords));
@@ -1021,6 +1038,8 @@ public:
         DevBuf<uint32_t>* u1[] = {&id[0], &id[1], &nbrCount, &cellOf, &rank, &tmpId};
         for (auto* b : u1) VFD_TRY(b->alloc(c));
         VFD_TRY(surface.alloc(c + 1));
+        VFD_TRY(bakedX.alloc(3 * c));
+        VFD_TRY(bakedV.alloc(3 * c));
         VFD_TRY(xb.alloc(c * kMaxBodies));
         VFD_TRY(vb.alloc(c * kMaxBodies));
         VFD_TRY(minv.alloc(c * 9));
@@ -1053,33 +1072,27 @@ public:
         std::vector<SceneParams> prm(S);
         for (uint32_t k = 0; k < S; ++k) prm[k] = sc[k]->prm;
         VFD_HIP(hipMemcpy(dP.p, prm.data(), S * sizeof(SceneParams), hipMemcpyHostToDevice));
+        for (Scene* s : sc)
+            if (s->count) {
+                const size_t bytes = 3 * (size_t)s->count * sizeof(float);
+                VFD_HIP(hipMemcpy(bakedX.p + 3 * (size_t)s->base, s->x0.data(), bytes, hipMemcpyHostToDevice));
+                VFD_HIP(hipMemcpy(bakedV.p + 3 * (size_t)s->base, s->v0.data(), bytes, hipMemcpyHostToDevice));
+            }
         committed = true;
-        VFD_TRY(upload_baked());
+        VFD_TRY(restore_baked());
         return VFD_OK;
     }
 
     // Simulate() start (DFSPHImplementation.cu:36-45): baked particles, dv = dk = 0, dt = TimeStepSize.
-    int upload_baked() {
-        const size_t c = std::max<size_t>(cap, 1);
-        std::vector<float4> x(c, make_float4(0, 0, 0, 0)), v(c, make_float4(0, 0, 0, 0));
-        std::vector<uint32_t> ids(c, 0);
+    int restore_baked() {
         for (Scene* s : sc) {
-            for (uint32_t i = 0; i < s->count; ++i) {
-                x[s->base + i] = make_float4(s->x0[3 * i], s->x0[3 * i + 1], s->x0[3 * i + 2], 0.0f);
-                v[s->base + i] = make_float4(s->v0[3 * i], s->v0[3 * i + 1], s->v0[3 * i + 2], 0.0f);
-                ids[s->base + i] = i;
-            }
             std::lock_guard<std::mutex> lk(hostMu);
             s->dbg = vfd_debug_info{};
             release_frames(*s);
         }
         cur = 0;
-        VFD_HIP(hipMemcpy(posNext.p, x.data(), c * sizeof(float4), hipMemcpyHostToDevice));
-        VFD_HIP(hipMemcpy(pos.p, x.data(), c * sizeof(float4), hipMemcpyHostToDevice));
-        VFD_HIP(hipMemcpy(vel[0].p, v.data(), c * sizeof(float4), hipMemcpyHostToDevice));
-        VFD_HIP(hipMemcpy(id[0].p, ids.data(), c * sizeof(uint32_t), hipMemcpyHostToDevice));
-        VFD_HIP(hipMemset(dv[0].p, 0, c * sizeof(float4)));
-        VFD_HIP(hipMemset(dk[0].p, 0, c * sizeof(float)));
+        launch_restore(launch(), bakedX.p, bakedV.p, pos.p, posNext.p, vel[0].p, dv[0].p, dk[0].p, id[0].p);
+        VFD_HIP(hipGetLastError());
         for (Scene* s : sc) set_time_step(s->st, s->desc, s->desc.TimeStepSize);
         return push_state();
     }
@@ -1091,14 +1104,6 @@ public:
         VFD_HIP(hipStreamSynchronize(stream));
         return VFD_OK;
     }
-    int pull_state() {
-        std::vector<SceneState> st(sc.size());
-        VFD_HIP(hipMemcpyAsync(st.data(), dState.p, st.size() * sizeof(SceneState), hipMemcpyDeviceToHost, stream));
-        VFD_HIP(hipStreamSynchronize(stream));
-        for (size_t k = 0; k < sc.size(); ++k) sc[k]->st = st[k];
-        return VFD_OK;
-    }
-
     uint32_t numCU = 256;
 
     Launch launch() const {
@@ -1117,6 +1122,7 @@ public:
         L.grid2 = std::min(L.gridAll, p2);
         L.groups = 8 * (per / kGroupTiles);
         L.gridGroups = std::min(L.groups, std::max<uint32_t>(8, numCU * kGroupsPerCU / 8 * 8));
+        L.stamps = stamps.p;
         L.tg.tiles = tiles;
         L.tg.per = per;
         return L;
@@ -1167,12 +1173,11 @@ public:
     int search() {
         const Launch L = launch();
         const uint32_t S = (uint32_t)sc.size();
-        VFD_TRY(timed("minmax", [&] { launch_minmax(L, posNext.p, dMMPart.p, dMM.p); }));
-        std::vector<int> mm((size_t)S * 6);
-        VFD_HIP(hipMemcpyAsync(mm.data(), dMM.p, mm.size() * sizeof(int), hipMemcpyDeviceToHost, stream));
+        VFD_TRY(timed("minmax", [&] { launch_minmax(L, posNext.p, dMMPart.p, hostBounds); }));
+        VFD_HIP(hipGetLastError());
         VFD_HIP(hipStreamSynchronize(stream));
+        const int* mm = hostBounds;
         uint32_t cellTotal = 0, prefix = 0;
-        std::vector<SceneGrid> grids(S);
         for (uint32_t k = 0; k < S; ++k) {
             Scene& s = *sc[k];
             SceneGrid g{};
@@ -1188,7 +1193,7 @@ public:
             g.cellBase = cellTotal;
             g.startCorr = startCorr;
             cellTotal += g.cellCount;  // <= kMaxGridCells, checked by size_scene_grid
-            grids[k] = g;
+            hostGrids[k] = g;
             s.grid = g;
         }
         uint32_t *cCount = nullptr, *cStart = nullptr, *cScan = nullptr;
@@ -1212,9 +1217,14 @@ public:
             cStart = cellStart.p;
             cScan = scanScratch.p;
         }
-        VFD_HIP(hipMemcpyAsync(dGrid.p, grids.data(), S * sizeof(SceneGrid), hipMemcpyHostToDevice, stream));
+        GridArgs args{};
+        if (S <= kGridArgs)
+            std::copy(hostGrids, hostGrids + S, args.g);
+        else
+            VFD_HIP(hipMemcpyAsync(dGrid.p, hostGrids, S * sizeof(SceneGrid), hipMemcpyHostToDevice, stream));
         const int alt = cur ^ 1;
         VFD_TRY(timed("sort", [&] {
+            launch_sort_begin(L, S <= kGridArgs ? &args : nullptr, dGrid.p, cCount, cellTotal);
             launch_sort(L, dGrid.p, cellTotal, posNext.p, vel[cur].p, dv[cur].p, dk[cur].p, id[cur].p, pos.p,
                         vel[alt].p, dv[alt].p, dk[alt].p, id[alt].p, cellOf.p, rank.p, tmpId.p, cCount, cStart,
                         cScan);
@@ -1291,14 +1301,25 @@ public:
         return rc;
     }
     static constexpr int kStepAborted = -1;
-    // waits for the step's launches; kStepAborted when a resident solve was aborted
-    int drain(uint32_t resident) {
-        *hostAborted = 0;
-        if (resident)
-            VFD_HIP(hipMemcpyAsync(hostAborted, residentWords.p + kResidentAbortedAt, sizeof(uint32_t),
-                                   hipMemcpyDeviceToHost, stream));
+    // The step's report, written behind its launches, and the wait for it; kStepAborted when a resident solve was aborted
+    int drain() {
+        launch_report(launch(), dState.p, nbStats.p, haloStats.p, residentWords.p, report, sceneReport);
+        VFD_HIP(hipGetLastError());
         VFD_HIP(hipStreamSynchronize(stream));
-        return *hostAborted ? kStepAborted : VFD_OK;
+        return report->aborted ? kStepAborted : VFD_OK;
+    }
+    // the report into the host's copies of the scenes' state and statistics (hostMu held)
+    void take_report() {
+        for (size_t k = 0; k < sc.size(); ++k) {
+            sc[k]->st = sceneReport[k].state;
+            vfd_debug_info& d = sc[k]->dbg;
+            d.TotalNeighborCount = sceneReport[k].neighbors;
+            d.MaxNeighborCount = (uint32_t)sceneReport[k].maxNeighbors;
+            d.StagedGroupCount = report->halo[0];
+            d.GatheredGroupCount = report->halo[1];
+            d.MaxHaloSize = report->halo[2];
+        }
+        solver_debug();
     }
     // resident: tiles per group of the step's resident solves, 0: launched iterations
     int step_once(int last, uint32_t resident) {
@@ -1314,10 +1335,8 @@ public:
             minDiv = std::max(minDiv, s->desc.MinDivergenceSolverIterations);
             minPres = std::max(minPres, s->desc.MinPressureSolverIterations);
         }
-        VFD_HIP(hipEventRecord(ev[0], stream));
         VFD_TRY(search());
-        VFD_HIP(hipEventRecord(ev[1], stream));
-        if (last == VFD_PHASE_SEARCH) return finish_partial(resident);
+        if (last == VFD_PHASE_SEARCH) return finish_partial();
         Fields F = fields();
         if (taping) VFD_TRY(tape_copy(tapeXpre, pos.p, cap));
         VFD_TRY(timed("boundary", [&] { launch_boundary(L, dMaps.p, pos.p, vel[cur].p, xb.p, vb.p); }));
@@ -1327,7 +1346,7 @@ public:
             launch_build_halo(L, groupTiles, nbrCount.p, nbrList.p, haloLimit, haloCount.p, haloIds.p, nbrLocal.p, haloStats.p,
                               pos.p, K);
         }));
-        if (last == VFD_PHASE_BOUNDARY) return finish_partial(resident);
+        if (last == VFD_PHASE_BOUNDARY) return finish_partial();
         DevTape* tp = nullptr;
         if (taping) {
             if (tapeCount == tapes.size()) tapes.emplace_back(new DevTape());
@@ -1371,8 +1390,7 @@ public:
             VFD_TRY(tape_copy(tp->rho, density.p, tp->n));
             VFD_TRY(tape_copy(tp->alpha, factor.p, tp->n));
         }
-        VFD_HIP(hipEventRecord(ev[2], stream));
-        if (last == VFD_PHASE_DENSITY || last == VFD_PHASE_FACTOR) return finish_partial(resident);
+        if (last == VFD_PHASE_DENSITY || last == VFD_PHASE_FACTOR) return finish_partial();
         // divergence solve (ComputeDivergence :506-575)
         if (residentJacobi) {
             VFD_TRY(timed("div_solve", [&] { launch_div_solve(L, resident, K, F, resident_words()); }));
@@ -1393,8 +1411,7 @@ public:
             VFD_TRY(timed("div_final", [&] { launch_div_final(L, K, F); }));  // also ClearAccelerationKernel
         }
         if (tp) VFD_TRY(tape_copy(tp->v1, vel[cur].p, tp->n));
-        VFD_HIP(hipEventRecord(ev[3], stream));
-        if (last == VFD_PHASE_DIVERGENCE || last == VFD_PHASE_CLEAR_ACCELERATION) return finish_partial(resident);
+        if (last == VFD_PHASE_DIVERGENCE || last == VFD_PHASE_CLEAR_ACCELERATION) return finish_partial();
         if (anyST) {
             if (tp && tp->stTemporal) VFD_TRY(tape_copy(tp->dK0, dk[cur].p, tp->n));
             VFD_TRY(upload_mc_tables(F));
@@ -1404,8 +1421,7 @@ public:
             VFD_TRY(tape_copy(tp->nMC, nMC.p, tp->n));
             VFD_TRY(tape_copy(tp->kMC, kMC.p, tp->n));
         }
-        VFD_HIP(hipEventRecord(ev[4], stream));
-        if (last == VFD_PHASE_SURFACE_TENSION) return finish_partial(resident);
+        if (last == VFD_PHASE_SURFACE_TENSION) return finish_partial();
         if (anyVisc && resident) {
             VFD_TRY(timed("visc_solve", [&] { launch_visc_solve(L, resident, K, F, resident_words(), haloStats.p); }));
         } else if (anyVisc) {
@@ -1424,14 +1440,13 @@ public:
             VFD_TRY(timed("visc_apply", [&] { launch_visc_apply(L, F); }));
         }
         if (tp && anyVisc) VFD_TRY(tape_copy(tp->y, cgX.p, tp->n));
-        VFD_HIP(hipEventRecord(ev[5], stream));
-        if (last == VFD_PHASE_VISCOSITY) return finish_partial(resident);
+        if (last == VFD_PHASE_VISCOSITY) return finish_partial();
         VFD_TRY(timed("time_step", [&] { launch_time_step(L, F); }));
         VFD_TRY(timed("time_step_finish", [&] { launch_time_step_finish(L, F); }));
-        if (last == VFD_PHASE_TIME_STEP) return finish_partial(resident);
+        if (last == VFD_PHASE_TIME_STEP) return finish_partial();
         VFD_TRY(timed("velocity", [&] { launch_velocity(L, F); }));
         if (tp) VFD_TRY(tape_copy(tp->v2, vel[cur].p, tp->n));
-        if (last == VFD_PHASE_VELOCITY) return finish_partial(resident);
+        if (last == VFD_PHASE_VELOCITY) return finish_partial();
         if (residentJacobi) {
             VFD_TRY(timed("pres_solve", [&] {
                 launch_pres_solve(L, resident, K, F, resident_words(), last >= VFD_PHASE_POSITION ? 1 : 0);
@@ -1455,14 +1470,10 @@ public:
                                   resident ? residentWords.p + kResidentAbortedAt : nullptr);
             }));
         }
-        VFD_HIP(hipEventRecord(ev[6], stream));
-        if (last == VFD_PHASE_PRESSURE) return finish_partial(resident);
-        VFD_HIP(hipGetLastError());
-        VFD_TRY(drain(resident));
+        if (last == VFD_PHASE_PRESSURE) return finish_partial();
+        VFD_TRY(drain());
         std::unique_lock<std::mutex> lk(hostMu);  // the host bookkeeping that polling threads read
-        VFD_TRY(pull_state());
-        solver_debug();
-        VFD_TRY(neighbor_stats());
+        take_report();
         VFD_TRY(resolve_profile());
         int nonfiniteScene = -1;  // per-step non-finite check (no reference counterpart)
         for (size_t k = 0; k < sc.size() && nonfiniteScene < 0; ++k)
@@ -1475,13 +1486,13 @@ public:
                 r.Kp = sc[s]->st.pres.it;
                 r.atCap = sc[s]->count && sc[s]->dbg.MaxNeighborCount >= kMaxNeighbors;
             }
-        float t[6] = {0, 0, 0, 0, 0, 0};
-        VFD_HIP(hipEventElapsedTime(&t[0], ev[0], ev[1]));
-        VFD_HIP(hipEventElapsedTime(&t[1], ev[1], ev[2]));
-        VFD_HIP(hipEventElapsedTime(&t[2], ev[2], ev[3]));
-        VFD_HIP(hipEventElapsedTime(&t[3], ev[3], ev[4]));
-        VFD_HIP(hipEventElapsedTime(&t[4], ev[4], ev[5]));
-        VFD_HIP(hipEventElapsedTime(&t[5], ev[5], ev[6]));
+        // phase timers from the times at which the phases' first kernels began
+        const long long* at = report->stamps;
+        const long long visc = anyVisc ? at[kStampViscosity] : at[kStampPressure], surf = anyST ? at[kStampSurface] : visc;
+        const long long edges[7] = {at[kStampStart], at[kStampBase], at[kStampDivergence], surf, visc, at[kStampPressure],
+                                    at[kStampEnd]};
+        float t[6];
+        for (int k = 0; k < 6; ++k) t[k] = (float)(edges[k + 1] - edges[k]) * 1e-5f;  // 100 MHz ticks to ms
         for (Scene* s : sc) {
             if (s->count == 0) continue;
             vfd_debug_info& d = s->dbg;
@@ -1722,34 +1733,14 @@ public:
     }
 
     // after a partial step the working positions become the state the next step starts from
-    int finish_partial(uint32_t resident) {
-        VFD_TRY(drain(resident));
+    int finish_partial() {
+        VFD_TRY(drain());
         VFD_HIP(hipMemcpyAsync(posNext.p, pos.p, (size_t)cap * sizeof(float4), hipMemcpyDeviceToDevice, stream));
         VFD_HIP(hipGetLastError());
         VFD_HIP(hipStreamSynchronize(stream));
         std::lock_guard<std::mutex> lk(hostMu);
-        VFD_TRY(pull_state());
-        solver_debug();
-        VFD_TRY(neighbor_stats());
+        take_report();
         return resolve_profile();
-    }
-
-    int neighbor_stats() {
-        std::vector<unsigned long long> nb(2 * sc.size());
-        VFD_HIP(hipMemcpyAsync(nb.data(), nbStats.p, nb.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                               stream));
-        VFD_HIP(hipStreamSynchronize(stream));
-        uint32_t hs[3];
-        VFD_HIP(hipMemcpyAsync(hs, haloStats.p, sizeof(hs), hipMemcpyDeviceToHost, stream));
-        VFD_HIP(hipStreamSynchronize(stream));
-        for (size_t k = 0; k < sc.size(); ++k) {
-            sc[k]->dbg.TotalNeighborCount = nb[2 * k];
-            sc[k]->dbg.MaxNeighborCount = (uint32_t)nb[2 * k + 1];
-            sc[k]->dbg.StagedGroupCount = hs[0];
-            sc[k]->dbg.GatheredGroupCount = hs[1];
-            sc[k]->dbg.MaxHaloSize = hs[2];
-        }
-        return VFD_OK;
     }
 
     // solver iteration counts and errors of the last (possibly partial) step, DFSPHDebugInfo semantics
@@ -1786,60 +1777,65 @@ public:
     }
     int ids(uint32_t s, std::vector<uint32_t>& out) { return fetch(id[cur].p, s, out); }
 
+    // three floats per particle of a scene, or one, to the caller's order on the device and from there to `out`
+    int read4(const float4* d, uint32_t s, float* out) {
+        const Scene& S = *sc[s];
+        if (!S.count) return VFD_OK;
+        VFD_TRY(fieldStage.alloc(3 * (size_t)S.count));
+        launch_gather4(stream, S.base, S.count, id[cur].p, d, fieldStage.p);
+        VFD_HIP(hipGetLastError());
+        VFD_HIP(hipMemcpyAsync(out, fieldStage.p, 3 * (size_t)S.count * sizeof(float), hipMemcpyDeviceToHost, stream));
+        VFD_HIP(hipStreamSynchronize(stream));
+        return VFD_OK;
+    }
+    int read1(const float* d, uint32_t s, float* out) {
+        const Scene& S = *sc[s];
+        if (!S.count) return VFD_OK;
+        VFD_TRY(fieldStage.alloc((size_t)S.count));
+        launch_gather1(stream, S.base, S.count, id[cur].p, d, 1u, fieldStage.p);
+        VFD_HIP(hipGetLastError());
+        VFD_HIP(hipMemcpyAsync(out, fieldStage.p, S.count * sizeof(float), hipMemcpyDeviceToHost, stream));
+        VFD_HIP(hipStreamSynchronize(stream));
+        return VFD_OK;
+    }
     int get_field(uint32_t s, int field, uint32_t body, float* out) {
         if (!committed) VFD_TRY(commit());
         const Scene& S = *sc[s];
-        std::vector<uint32_t> idv;
-        VFD_TRY(ids(s, idv));
-        auto put4 = [&](const float4* d, int comps) -> int {
-            std::vector<float4> v;
-            VFD_TRY(fetch(d, s, v));
-            for (uint32_t k = 0; k < S.count; ++k) {
-                const uint32_t i = idv[k];
-                out[comps * i] = v[k].x;
-                if (comps > 1) {
-                    out[comps * i + 1] = v[k].y;
-                    out[comps * i + 2] = v[k].z;
-                }
-            }
-            return VFD_OK;
-        };
-        auto put1 = [&](const float* d) -> int {
-            std::vector<float> v;
-            VFD_TRY(fetch(d, s, v));
-            for (uint32_t k = 0; k < S.count; ++k) out[idv[k]] = v[k];
-            return VFD_OK;
-        };
+        auto put4 = [&](const float4* d) { return read4(d, s, out); };
+        auto put1 = [&](const float* d) { return read1(d, s, out); };
         switch (field) {
-            case VFD_FIELD_POSITION: return put4(posNext.p, 3);
-            case VFD_FIELD_VELOCITY: return put4(vel[cur].p, 3);
-            case VFD_FIELD_ACCELERATION: return put4(acc.p, 3);
-            case VFD_FIELD_PRESSURE_ACCELERATION: return put4(ap.p, 3);
+            case VFD_FIELD_POSITION: return put4(posNext.p);
+            case VFD_FIELD_VELOCITY: return put4(vel[cur].p);
+            case VFD_FIELD_ACCELERATION: return put4(acc.p);
+            case VFD_FIELD_PRESSURE_ACCELERATION: return put4(ap.p);
             case VFD_FIELD_PRESSURE_RESIDUUM: return put1(residuum.p);
             case VFD_FIELD_DENSITY: return put1(density.p);
             case VFD_FIELD_DENSITY_ADVECTION: return put1(densAdv.p);
             case VFD_FIELD_PRESSURE_RHO2: return put1(kappa.p);
             case VFD_FIELD_PRESSURE_RHO2_V: return put1(kappaV.p);
             case VFD_FIELD_FACTOR: return put1(factor.p);
-            case VFD_FIELD_VELOCITY_DIFFERENCE: return put4(dv[cur].p, 3);
-            case VFD_FIELD_MC_SURFACE_NORMAL: return put4(nMC.p, 3);
-            case VFD_FIELD_MC_SURFACE_NORMAL_SMOOTH: return put4(nS.p, 3);
+            case VFD_FIELD_VELOCITY_DIFFERENCE: return put4(dv[cur].p);
+            case VFD_FIELD_MC_SURFACE_NORMAL: return put4(nMC.p);
+            case VFD_FIELD_MC_SURFACE_NORMAL_SMOOTH: return put4(nS.p);
             case VFD_FIELD_MC_SURFACE_CURVATURE: return put1(kMC.p);
             case VFD_FIELD_MC_SURFACE_CURVATURE_SMOOTH: return put1(kS.p);
             case VFD_FIELD_DELTA_FINAL_CURVATURE: return put1(dk[cur].p);
             case VFD_FIELD_BOUNDARY_XJ:
                 if (body >= kMaxBodies) return fail(VFD_ERROR_INVALID_ARGUMENT, "body out of range");
-                return put4(xb.p + (size_t)body * cap, 3);
+                return put4(xb.p + (size_t)body * cap);
             case VFD_FIELD_BOUNDARY_VOLUME:
                 if (body >= kMaxBodies) return fail(VFD_ERROR_INVALID_ARGUMENT, "body out of range");
                 return put1(vb.p + (size_t)body * cap);
-            case VFD_FIELD_VISCOSITY_SOLUTION: return put4(cgX.p, 3);
+            case VFD_FIELD_VISCOSITY_SOLUTION: return put4(cgX.p);
             case VFD_FIELD_VISCOSITY_PRECONDITIONER: {
-                for (int e = 0; e < 9; ++e) {
-                    std::vector<float> v;
-                    VFD_TRY(fetch(minv.p + (size_t)e * cap, s, v));
-                    for (uint32_t k = 0; k < S.count; ++k) out[9 * idv[k] + e] = v[k];
-                }
+                if (!S.count) return VFD_OK;
+                VFD_TRY(fieldStage.alloc(9 * (size_t)S.count));
+                for (uint32_t e = 0; e < 9; ++e)
+                    launch_gather1(stream, S.base, S.count, id[cur].p, minv.p + (size_t)e * cap, 9u, fieldStage.p + e);
+                VFD_HIP(hipGetLastError());
+                VFD_HIP(hipMemcpyAsync(out, fieldStage.p, 9 * (size_t)S.count * sizeof(float), hipMemcpyDeviceToHost,
+                                       stream));
+                VFD_HIP(hipStreamSynchronize(stream));
                 return VFD_OK;
             }
         }
@@ -1849,32 +1845,26 @@ public:
     int set_field(uint32_t s, int field, const float* in) {
         if (!committed) VFD_TRY(commit());
         const Scene& S = *sc[s];
-        std::vector<uint32_t> idv;
-        VFD_TRY(ids(s, idv));
-        auto write4 = [&](float4* d) -> int {
-            std::vector<float4> v(S.count);
-            for (uint32_t k = 0; k < S.count; ++k) {
-                const uint32_t i = idv[k];
-                v[k] = make_float4(in[3 * i], in[3 * i + 1], in[3 * i + 2], 0.0f);
-            }
-            if (S.count) VFD_HIP(hipMemcpy(d + S.base, v.data(), S.count * sizeof(float4), hipMemcpyHostToDevice));
-            return VFD_OK;
-        };
+        if (field != VFD_FIELD_POSITION && field != VFD_FIELD_VELOCITY && field != VFD_FIELD_VELOCITY_DIFFERENCE &&
+            field != VFD_FIELD_DELTA_FINAL_CURVATURE)
+            return fail(VFD_ERROR_INVALID_ARGUMENT, "field is not writable");
+        if (!S.count) return VFD_OK;
+        const size_t floats = (field == VFD_FIELD_DELTA_FINAL_CURVATURE ? 1 : 3) * (size_t)S.count;
+        VFD_TRY(fieldStage.alloc(floats));
+        VFD_HIP(hipMemcpyAsync(fieldStage.p, in, floats * sizeof(float), hipMemcpyHostToDevice, stream));
+        auto write4 = [&](float4* d) { launch_scatter4(stream, S.base, S.count, id[cur].p, fieldStage.p, d); };
         switch (field) {
             case VFD_FIELD_POSITION:
-                VFD_TRY(write4(posNext.p));
-                return write4(pos.p);
-            case VFD_FIELD_VELOCITY: return write4(vel[cur].p);
-            case VFD_FIELD_VELOCITY_DIFFERENCE: return write4(dv[cur].p);
-            case VFD_FIELD_DELTA_FINAL_CURVATURE: {
-                std::vector<float> v(S.count);
-                for (uint32_t k = 0; k < S.count; ++k) v[k] = in[idv[k]];
-                if (S.count)
-                    VFD_HIP(hipMemcpy(dk[cur].p + S.base, v.data(), S.count * sizeof(float), hipMemcpyHostToDevice));
-                return VFD_OK;
-            }
+                write4(posNext.p);
+                write4(pos.p);
+                break;
+            case VFD_FIELD_VELOCITY: write4(vel[cur].p); break;
+            case VFD_FIELD_VELOCITY_DIFFERENCE: write4(dv[cur].p); break;
+            default: launch_scatter1(stream, S.base, S.count, id[cur].p, fieldStage.p, dk[cur].p);
         }
-        return fail(VFD_ERROR_INVALID_ARGUMENT, "field is not writable");
+        VFD_HIP(hipGetLastError());
+        VFD_HIP(hipStreamSynchronize(stream));  // the caller's array and the stage are free again
+        return VFD_OK;
     }
 
     int get_neighbors(uint32_t s, uint32_t* counts, uint32_t* offsets, uint32_t* out, uint64_t* total) {
@@ -2163,7 +2153,7 @@ int vfd_step_until(vfd_sim* sim, int32_t phase) {
 int vfd_simulate(vfd_sim* sim) {
     DRIVE(sim);
     Simulation& S = sim->impl;
-    const int rc = S.committed ? S.upload_baked() : S.commit();
+    const int rc = S.committed ? S.restore_baked() : S.commit();
     if (rc != VFD_OK) return rc;
     return S.simulate_frames();
 }
@@ -2175,7 +2165,7 @@ int vfd_simulate_async(vfd_sim* sim) {
         return fail(VFD_ERROR_STATE, "the simulation is running on another thread");
     S.join_worker();  // a finished worker nobody waited for
     // baked particles restored and earlier frames released here, before any poll can read them
-    const int rc = S.committed ? S.upload_baked() : S.commit();
+    const int rc = S.committed ? S.restore_baked() : S.commit();
     if (rc != VFD_OK) {
         S.busy = false;
         return rc;

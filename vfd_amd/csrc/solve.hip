@@ -705,7 +705,8 @@ __global__ void __launch_bounds__(kTiles * kTile, 1) k_jacobi_solve(const SceneP
                                                                     const uint32_t* __restrict__ tileScene, KTabHost kh,
                                                                     Fields F, uint32_t cap, TileGrid tg,
                                                                     uint32_t sceneCount, uint32_t* words,
-                                                                    uint32_t waitTicks, int writeNext) {
+                                                                    uint32_t waitTicks, int writeNext, long long* stamps) {
+    if (!kPressure) note_time(stamps, kStampDivergence);
     extern __shared__ float4 lds[];
     __shared__ SceneCtl ctl[kResidentScenes];
     if (words[kResidentAbortedAt]) return;  // an earlier solve of this step was aborted
@@ -737,7 +738,9 @@ __global__ void __launch_bounds__(kTiles * kTile, 1) k_visc_solve(const ScenePar
                                                                          KTabHost kh, Fields F, uint32_t cap,
                                                                          TileGrid tg, uint32_t sceneCount,
                                                                          uint32_t* words, uint32_t waitTicks,
-                                                                         const uint32_t* __restrict__ haloStats) {
+                                                                         const uint32_t* __restrict__ haloStats,
+                                                                         long long* stamps) {
+    note_time(stamps, kStampViscosity);
     __shared__ SceneCtl ctl[kResidentScenes];
     if (words[kResidentAbortedAt]) return;  // an earlier solve of this step was aborted
     VFD_HALO_KERNEL_PROLOGUE(kh)
@@ -943,7 +946,7 @@ void launch_div_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt, 
     with_tiles(groupTiles, [&](auto t) {
         hipLaunchKernelGGL((k_jacobi_solve<t(), false>), dim3(L.group_count(t())), dim3(t() * kTile), kLdsJacobi,
                            L.stream, L.P, L.tileScene, kt, F, L.capacity, TileGrid(L.tg), L.sceneCount, r.words,
-                           r.waitTicks, 0);
+                           r.waitTicks, 0, L.stamps);
     });
 }
 void launch_pres_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt, const Fields& F, const Resident& r,
@@ -951,7 +954,7 @@ void launch_pres_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt,
     with_tiles(groupTiles, [&](auto t) {
         hipLaunchKernelGGL((k_jacobi_solve<t(), true>), dim3(L.group_count(t())), dim3(t() * kTile), kLdsJacobi,
                            L.stream, L.P, L.tileScene, kt, F, L.capacity, TileGrid(L.tg), L.sceneCount, r.words,
-                           r.waitTicks, writeNext);
+                           r.waitTicks, writeNext, L.stamps);
     });
 }
 void launch_visc_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt, const Fields& F, const Resident& r,
@@ -959,7 +962,7 @@ void launch_visc_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt,
     with_tiles(groupTiles, [&](auto t) {
         hipLaunchKernelGGL((k_visc_solve<t()>), dim3(L.group_count(t())), dim3(t() * kTile), kLdsVisc, L.stream, L.P,
                            L.tileScene, kt, F, L.capacity, TileGrid(L.tg), L.sceneCount, r.words, r.waitTicks,
-                           haloStats);
+                           haloStats, L.stamps);
     });
 }
 int configure_solve_kernels() {

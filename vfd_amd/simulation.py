@@ -322,7 +322,7 @@ class DFSPHSimulation:
     def field(self, name, body=0):
         fid, comps = _abi.FIELDS[name]
         n = self.GetParticleCount()
-        out = np.zeros((n, comps), np.float32)
+        out = np.empty((n, comps), np.float32)
         check(self._lib.vfd_get_field(self._h, self._scene, fid, body, ptr(out)), "vfd_get_field(%s)" % name)
         return out if comps > 1 else out[:, 0]
 
@@ -333,9 +333,7 @@ class DFSPHSimulation:
 
     def particles(self):
         n = self.GetParticleCount()
-        x = np.zeros((n, 3), np.float32)
-        v = np.zeros((n, 3), np.float32)
-        a = np.zeros((n, 3), np.float32)
+        x, v, a = (np.empty((n, 3), np.float32) for _ in range(3))
         check(self._lib.vfd_batch_get_particles(self._h, self._scene, ptr(x), ptr(v), ptr(a)), "vfd_get_particles")
         return x, v, a
 
@@ -355,7 +353,7 @@ class DFSPHSimulation:
         cnt = _abi.ctypes.c_uint32()
         check(self._lib.vfd_get_boundary_map(self._h, self._scene, body, field, None, _abi.ctypes.byref(cnt)),
               "vfd_get_boundary_map")
-        out = np.zeros(cnt.value, np.float32)
+        out = np.empty(cnt.value, np.float32)
         check(self._lib.vfd_get_boundary_map(self._h, self._scene, body, field, ptr(out), _abi.ctypes.byref(cnt)),
               "vfd_get_boundary_map")
         return out
@@ -407,7 +405,7 @@ class DFSPHSimulation:
         n = self.GetParticleCount()
         lx = np.ascontiguousarray(lx_out, np.float32).reshape(n, 3)
         lv = None if lv_out is None else np.ascontiguousarray(lv_out, np.float32).reshape(n, 3)
-        ox, ov = np.zeros((n, 3), np.float32), np.zeros((n, 3), np.float32)
+        ox, ov = np.empty((n, 3), np.float32), np.empty((n, 3), np.float32)
         mu = _abi.ctypes.c_double()
         args = (ptr(lx), None if lv is None else ptr(lv), ptr(ox), ptr(ov), _abi.ctypes.byref(mu))
         if self._scene == 0:
@@ -433,7 +431,7 @@ class DFSPHSimulation:
         n = self.GetParticleCount()
         frames = []
         for k in range(cnt.value):
-            xva = np.zeros((n, 9), np.float32)
+            xva = np.empty((n, 9), np.float32)
             mv = _abi.ctypes.c_float()
             dt = _abi.ctypes.c_float()
             check(self._lib.vfd_get_frame(self._h, self._scene, k, ptr(xva), _abi.ctypes.byref(mv),
