@@ -76,7 +76,7 @@ __device__ __forceinline__ f3 vjp_grad(const AdjK& a, f3 r, float rl, float g, f
     return o;
 }
 __device__ __forceinline__ uint32_t adj_nbr(const AdjK& a, uint32_t i, uint32_t j) {
-    return a.list[(size_t)j * a.cap + i];
+    return a.list[list_at(i, j)];
 }
 __device__ __forceinline__ uint32_t pid() { return blockIdx.x * blockDim.x + threadIdx.x; }
 // The neighbour-loop kernels run over the scene's slots [base, base + n) (one thread each) and index every array by

@@ -4,9 +4,12 @@
 // kTile, slots in Morton cell order and re-sorted every step):
 //   positions / velocities / vectors: float4 per particle (w unused), one 16-byte load per neighbour gather
 //   scalars: float per particle
-//   neighbour lists: uint32 slot indices, transposed list[j * capacity + i] so that the j-th neighbour of 64
-//   consecutive particles is one coalesced 256-byte read; at most kMaxNeighbors per particle; for the particles of a
-//   staged group also as uint16 halo slots and uint16 kernel-table codes of the pairs, in the same transposed layout;
+//   neighbour lists: uint32 slot indices, at most kMaxNeighbors per particle, tile by tile and transposed inside a tile
+//   ([tile][j][kTile], list_at) so that the j-th neighbour of 64 consecutive particles is one coalesced 256-byte access
+//   and a tile's lists are one stretch of 70 KB; for the particles of a staged group also as uint16 halo slots and
+//   uint16 kernel-table codes of the pairs, rows in pairs ([tile][j / 2][kTile][2], local_at). With rows as long as the
+//   state instead ([j][capacity]) a wave's stores of its lists went to 40 rows megabytes apart: k_build_lists took
+//   659 us instead of 597 on 2 million particles, 198 instead of 178 on 500,000;
 //   halos: per group, haloCount[g] and the halo's particle slots haloIds[g * kHaloMax + k].
 //
 // All HIP sources are compiled with -ffp-contract=off: every fused multiply-add is an explicit fmaf, so the
@@ -26,6 +29,14 @@ namespace vfd {
 
 constexpr unsigned kTile = 256;              // particles per tile = threads per block
 constexpr unsigned kMaxNeighbors = 70;       // ParticleSearchKernels.cuh:7
+constexpr unsigned kTileList = kMaxNeighbors * kTile;  // list entries of a tile
+// entry j of the list of slot i, and the pair of staged entries 2k, 2k + 1 (in pairs)
+__host__ __device__ inline size_t list_at(uint32_t i, uint32_t j) {
+    return (size_t)(i / kTile) * kTileList + (j * kTile + i % kTile);
+}
+__host__ __device__ inline size_t local_at(uint32_t i, uint32_t k) {
+    return (size_t)(i / kTile) * (kTileList / 2) + (k * kTile + i % kTile);
+}
 constexpr unsigned kMetaGroup = 8;           // ParticleSearchKernels.cuh:8
 constexpr unsigned kMetaBlock = 512;         // ParticleSearchKernels.cuh:9
 constexpr unsigned kTableResolution = 10000; // Kernel/DFSPHKernels.h:143

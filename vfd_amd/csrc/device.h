@@ -274,23 +274,6 @@ __device__ __forceinline__ void tile_partials4(double (&v)[NV], double* partials
     __syncthreads();
 }
 
-// Neighbour j of particle i in the transposed lists; f(t) is called in list order, four list entries fetched per
-// trip so that their gathers can be in flight together.
-template <class Fn>
-__device__ __forceinline__ void each_neighbor(const uint32_t* __restrict__ list, uint32_t cap, uint32_t i, uint32_t n,
-                                              Fn&& f) {
-    uint32_t j = 0;
-    for (; j + 4 <= n; j += 4) {
-        const uint32_t t0 = list[(size_t)j * cap + i], t1 = list[(size_t)(j + 1) * cap + i];
-        const uint32_t t2 = list[(size_t)(j + 2) * cap + i], t3 = list[(size_t)(j + 3) * cap + i];
-        f(t0);
-        f(t1);
-        f(t2);
-        f(t3);
-    }
-    for (; j < n; ++j) f(list[(size_t)j * cap + i]);
-}
-
 // Kernel table staged in LDS: tab[p] (float2 {W, G}) or G only, loaded once per block. The sizes are rounded up to
 // 16 bytes so that the halo records can follow the table.
 // both LDS tables hold one entry past the kernel table, for code kGCodeZero (see gcode)
@@ -395,8 +378,8 @@ __device__ __forceinline__ f3 gradW(const KLds& k, f3 r) {
 // list entry. Both paths hand the same values to the same arithmetic in the same list order.
 struct NbrSrc {
     const float* rec;                      // LDS records of the halo (layout: HaloRec); nullptr: global gathers
-    const uint32_t* __restrict__ local;    // [j * cap + i] halo slot | table code << 16 (staged groups)
-    const uint32_t* __restrict__ list;     // [j * cap + i] particle slots
+    const uint32_t* __restrict__ local;    // halo slot | table code << 16 (staged groups; local_at)
+    const uint32_t* __restrict__ list;     // particle slots (list_at)
     const uint32_t* __restrict__ count;    // [i]
     uint32_t cap;
 };
@@ -574,15 +557,30 @@ template <class Load> struct HaloRec {
 constexpr int kRawBufferWord3 = 0x00020000;
 // An offset at or past a raw buffer's num_records reads 0 without touching memory; adding this to a lane's offset
 // keeps the load in the instruction stream (so the compiler still counts it in flight) but takes it off the memory
-// path. Valid offsets stay below 2^31 bytes (a simulation holds at most 2^28 slots: 8-byte row-pair entries).
+// path (a tile's lists are 70 KB).
 constexpr uint32_t kBufferOutOfRange = 0x80000000u;
+// The staged lists of the tile of slot i (the same tile in every lane) as one buffer
+struct TileLists {
+    __amdgpu_buffer_rsrc_t rows;
+    uint32_t at;
+    __device__ __forceinline__ TileLists(const uint32_t* local, uint32_t i)
+        : rows(__builtin_amdgcn_make_buffer_rsrc(
+              const_cast<uint32_t*>(local + (size_t)__builtin_amdgcn_readfirstlane(i / kTile) * kTileList), (short)0,
+              (int)(kTileList * sizeof(uint32_t)), kRawBufferWord3)),
+          at(i % kTile * 8u) {}
+    // entries 2k, 2k + 1 (k the same in every lane); 0 without a memory access where !in
+    template <int kCache> __device__ __forceinline__ uint2 pair(uint32_t k, bool in) const {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b64(rows, (int)(at + (in ? 0u : kBufferOutOfRange)),
+                                                            (int)(k * kTile * 8u), kCache);
+        return make_uint2(v[0], v[1]);
+    }
+};
 
 template <int R, class TV, class Load, class Fn>
 __device__ __forceinline__ void each_neighbor_rec(const NbrSrc& src, uint32_t i, float cutR, float invStep, f3 xi,
                                                   const TV* tab, const Load& load, Fn&& f) {
     constexpr uint32_t C = Load::template Shape<R>::chunk;
     const uint32_t n = src.count[i];
-    const size_t cap = src.cap;
     uint32_t j = 0;
     if (src.rec) {
         if (n == 0) return;
@@ -590,22 +588,19 @@ __device__ __forceinline__ void each_neighbor_rec(const NbrSrc& src, uint32_t i,
         using HR = HaloRec<Load>;
         const uint32_t last = n - 1u;
         // the list is read once per launch: non-temporal loads keep it from displacing the halo records, which
-        // neighbouring groups gather again, from the caches. The staged lists hold rows in pairs ([j/2][cap][2]):
-        // rows r, r + 1 of the wave (r even, the same in every lane) are one buffer of cap 8-byte entries, read with
-        // one load per lane; a lane whose list ended before row r reads past the buffer's end, which returns 0
-        // without a memory access, so the rows past a short list cost the memory path nothing.
+        // neighbouring groups gather again, from the caches. The staged lists hold rows in pairs: rows r, r + 1 of
+        // the wave (r even, the same in every lane) are read with one 8-byte load per lane from the buffer that holds
+        // the tile's lists; a lane whose list ended before row r reads past the buffer's end, which returns 0 without
+        // a memory access, so the rows past a short list cost the memory path nothing.
         static_assert(C % 2 == 0, "list chunks cover whole row pairs");
+        const TileLists lists(src.local, i);
         auto fetch = [&](uint32_t (&e)[C], uint32_t b) {
 #pragma unroll
             for (uint32_t u = 0; u < C / 2; ++u) {
                 const uint32_t r = b + 2 * u;
-                const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
-                    const_cast<uint32_t*>(src.local + (size_t)(r >> 1) * cap * 2), (short)0, (int)(cap * 8),
-                    kRawBufferWord3);
-                const uint32_t off = i * 8u + (r <= last ? 0u : kBufferOutOfRange);
-                const auto v = __builtin_amdgcn_raw_buffer_load_b64(rows, (int)off, 0, Load::kListCache);
-                e[2 * u] = v[0];
-                e[2 * u + 1] = v[1];
+                const uint2 v = lists.template pair<Load::kListCache>(r >> 1, r <= last);
+                e[2 * u] = v.x;
+                e[2 * u + 1] = v.y;
             }
         };
         auto consume = [&](const uint32_t (&e)[C], uint32_t b) {
@@ -648,7 +643,7 @@ __device__ __forceinline__ void each_neighbor_rec(const NbrSrc& src, uint32_t i,
         for (; j + 4 <= n; j += 4) {
             uint32_t t[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) t[u] = src.list[(j + u) * cap + i];
+            for (int u = 0; u < 4; ++u) t[u] = src.list[list_at(i, j + u)];
             float4 lo[4], hi[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) load(t[u], lo[u], hi[u]);
@@ -657,7 +652,7 @@ __device__ __forceinline__ void each_neighbor_rec(const NbrSrc& src, uint32_t i,
         }
         for (; j < n; ++j) {
             float4 lo, hi;
-            load(src.list[j * cap + i], lo, hi);
+            load(src.list[list_at(i, j)], lo, hi);
             f(lo, hi, tab[gcode<Load::kShortSqrt>(cutR, invStep, xi - ld3(lo))]);
         }
     }

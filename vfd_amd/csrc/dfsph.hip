@@ -409,24 +409,49 @@ void launch_frame_pack(hipStream_t s, uint32_t base, uint32_t count, const uint3
 }
 
 // ---- the step's report, restored particles, fields in the caller's order -------------------------------------------
-__global__ void __launch_bounds__(kTile) k_report(uint32_t sceneCount, const SceneState* __restrict__ state,
-                                                  const unsigned long long* __restrict__ nbStats,
-                                                  const uint32_t* __restrict__ haloStats,
-                                                  const uint32_t* __restrict__ words, const long long* stamps,
-                                                  StepReport* report, SceneReport* scenes) {
-    for (uint32_t s = threadIdx.x; s < sceneCount; s += kTile)
-        scenes[s] = SceneReport{state[s], nbStats[2 * s], nbStats[2 * s + 1]};
+// a block per scene
+__global__ void __launch_bounds__(kFinishThreads) k_report(const SceneParams* __restrict__ P,
+                                                           const SceneState* __restrict__ state,
+                                                           const uint2* __restrict__ tileStats,
+                                                           const uint32_t* __restrict__ haloStats,
+                                                           const uint32_t* __restrict__ words, const long long* stamps,
+                                                           StepReport* report, SceneReport* scenes) {
+    __shared__ unsigned long long total[kFinishThreads / kWave], longest[kFinishThreads / kWave];
+    const uint32_t s = blockIdx.x;
+    unsigned long long tot = 0, mx = 0;
+    for (uint32_t t = P[s].tileBegin + threadIdx.x; t < P[s].tileEnd; t += kFinishThreads) {
+        const uint2 v = tileStats[t];
+        tot += v.x;
+        mx = max(mx, (unsigned long long)v.y);
+    }
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        tot += __shfl_xor(tot, o, kWave);
+        mx = max(mx, __shfl_xor(mx, o, kWave));
+    }
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        total[threadIdx.x / kWave] = tot;
+        longest[threadIdx.x / kWave] = mx;
+    }
+    __syncthreads();
     if (threadIdx.x == 0) {
-        StepReport r{words[kResidentAbortedAt], {haloStats[0], haloStats[1], haloStats[2]}, {}};
-        for (int k = 0; k < kStampEnd; ++k) r.stamps[k] = stamps[k];
-        r.stamps[kStampEnd] = wall_clock64();
-        *report = r;
+        for (uint32_t w = 1; w < kFinishThreads / kWave; ++w) {
+            tot += total[w];
+            mx = max(mx, longest[w]);
+        }
+        scenes[s] = SceneReport{state[s], tot, mx};
+        if (s == 0) {
+            StepReport r{words[kResidentAbortedAt], {haloStats[0], haloStats[1], haloStats[2]}, {}};
+            for (int k = 0; k < kStampEnd; ++k) r.stamps[k] = stamps[k];
+            r.stamps[kStampEnd] = wall_clock64();
+            *report = r;
+        }
     }
 }
-void launch_report(const Launch& L, const SceneState* state, const unsigned long long* nbStats, const uint32_t* haloStats,
+void launch_report(const Launch& L, const SceneState* state, const uint2* tileStats, const uint32_t* haloStats,
                    const uint32_t* words, StepReport* report, SceneReport* scenes) {
-    hipLaunchKernelGGL(k_report, dim3(1), dim3(kTile), 0, L.stream, L.sceneCount, state, nbStats, haloStats, words,
-                       (const long long*)L.stamps, report, scenes);
+    hipLaunchKernelGGL(k_report, dim3(L.sceneCount), dim3(kFinishThreads), 0, L.stream, L.P, state, tileStats, haloStats,
+                       words, (const long long*)L.stamps, report, scenes);
 }
 
 __global__ void __launch_bounds__(kTile) k_restore(const SceneParams* __restrict__ P,

@@ -205,7 +205,7 @@ void launch_build_halo(const Launch& L, uint32_t groupTiles, const uint32_t* nbr
                        const float4* pos, const KTabHost& kt);
 void launch_build_lists(const Launch& L, const SceneGrid* G, const float4* pos, const uint32_t* cellStart,
                         const uint32_t* cellCount, uint32_t* nbrCount, uint32_t* nbrList,
-                        unsigned long long* nbStats);
+                        uint2* tileStats);
 
 // Static scratch of the allocation-free step, in 32-bit words: the grid's cell counts and cell starts (kStaticCells
 // each), the scan's chunk sums, the surface-tension curvature tables (kStaticMcFloats floats) and their per-scene
@@ -263,7 +263,7 @@ struct Fields {
     float* vb;        // [kMaxBodies][capacity]
     const uint32_t* nbrCount;
     const uint32_t* nbrList;
-    const uint32_t* nbrLocal;    // [j][capacity] halo slot | table code << 16 (staged groups)
+    const uint32_t* nbrLocal;    // [tile][j / 2][kTile][2] halo slot | table code << 16 (staged groups)
     const uint32_t* haloCount;   // [groups] kHaloNone: global gathers
     const uint32_t* haloIds;     // [groups][kHaloMax]
     // viscosity solver
@@ -333,7 +333,7 @@ void launch_visc_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt,
                        const uint32_t* haloStats);
 int configure_solve_kernels();
 // report and its scenes in pinned host memory
-void launch_report(const Launch& L, const SceneState* state, const unsigned long long* nbStats, const uint32_t* haloStats,
+void launch_report(const Launch& L, const SceneState* state, const uint2* tileStats, const uint32_t* haloStats,
                    const uint32_t* words, StepReport* report, SceneReport* scenes);
 // Baked particles (three floats each, scene by scene in slot order) into the state a simulation starts from
 void launch_restore(const Launch& L, const float* x, const float* v, float4* pos, float4* posNext, float4* vel, float4* dv,

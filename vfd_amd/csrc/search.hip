@@ -7,7 +7,7 @@
 //   - particles are physically reordered by (cell, original id) every step, so every later neighbour loop reads
 //     contiguous cells; the reference keeps particles in input order and only sorts index arrays;
 //   - the order inside a cell is ascending original id (deterministic) instead of atomicAdd order;
-//   - lists hold slot indices in a transposed [j][i] layout with a fixed capacity of 70 per particle.
+//   - lists hold slot indices, tile by tile in a transposed [j][i] layout with a fixed capacity of 70 per particle.
 #include <algorithm>
 #include <mutex>
 
@@ -162,10 +162,27 @@ __global__ void __launch_bounds__(kTile) k_reorder(const SceneParams* __restrict
 #ifndef VFD_SEARCH_UNROLL
 #define VFD_SEARCH_UNROLL 8
 #endif
-#ifndef VFD_STAGE_LISTS
-#define VFD_STAGE_LISTS 0
-#endif
 constexpr uint32_t kSearchUnroll = VFD_SEARCH_UNROLL;
+
+// The tile's neighbour total and longest list to tileStats[tile], which the step's report sums up. (A 64-bit atomic add
+// and maximum per wave on the scene's two counters were what the kernel waited for, about 14 ns a wave whatever the
+// search did: 866 -> 659 us on 2 million particles, 92 -> 65 us on 123,000.)
+__device__ __forceinline__ void note_neighbors(uint32_t cnt, uint32_t tile, uint2* tileStats) {
+    __shared__ uint2 sh[kTile / kWave];
+    uint32_t tot = cnt, mx = cnt;
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        tot += (uint32_t)__shfl_xor((int)tot, o, kWave);
+        mx = max(mx, (uint32_t)__shfl_xor((int)mx, o, kWave));
+    }
+    if ((threadIdx.x & (kWave - 1)) == 0) sh[threadIdx.x / kWave] = make_uint2(tot, mx);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint2 t = sh[0];
+        for (uint32_t w = 1; w < kTile / kWave; ++w) t = make_uint2(t.x + sh[w].x, max(t.y, sh[w].y));
+        tileStats[tile] = t;
+    }
+}
 
 // FindNeighbors (ParticleSearch.cu:95-195; kernels ParticleSearchKernels.cu:93-193) in one traversal per particle:
 // the 27 cells in z, y, x order, each cell's particles in slot order (= ascending original id), strict
@@ -232,225 +249,21 @@ __device__ __forceinline__ uint32_t neighbor_list(const TileCtx& c, const SceneP
     return cnt;
 }
 
-// With VFD_STAGE_LISTS the lists are staged in LDS ([kMaxNeighbors][kTile] per block) while the traversals run,
-// then written row by row, so every global store of a row is one coalesced 1 KB write of the tile; otherwise each
-// entry is stored as it is found.
-constexpr unsigned kLdsListStage = VFD_STAGE_LISTS ? kMaxNeighbors * kTile * sizeof(uint32_t) : 0u;
+// One thread per particle, each entry stored as it is found; a tile's lists are one stretch of memory (list_at).
 __global__ void __launch_bounds__(kTile) k_build_lists(const float4* __restrict__ pos, const SceneParams* __restrict__ P,
                                                        const SceneGrid* __restrict__ G,
                                                        const uint32_t* __restrict__ tileScene,
                                                        const uint32_t* __restrict__ cellStart,
                                                        const uint32_t* __restrict__ cellCount, uint32_t* nbrCount,
-                                                       uint32_t* nbrList, uint32_t capacity,
-                                                       unsigned long long* nbStats) {
-    extern __shared__ uint32_t stage[];  // [kMaxNeighbors][kTile]
-    __shared__ uint32_t rows;
+                                                       uint32_t* nbrList, uint2* tileStats) {
     const TileCtx c = tile_ctx(tileScene, P);
-    if (threadIdx.x == 0) rows = 0;
-    __syncthreads();
     uint32_t cnt = 0;
     if (c.valid) {
-        cnt = neighbor_list(c, P, G, pos, cellStart, cellCount, [&](uint32_t j, uint32_t t) {
-            if (VFD_STAGE_LISTS)
-                stage[j * kTile + threadIdx.x] = t;
-            else
-                nbrList[(size_t)j * capacity + c.i] = t;
-        });
+        uint32_t* out = nbrList + list_at(c.i, 0);
+        cnt = neighbor_list(c, P, G, pos, cellStart, cellCount, [&](uint32_t j, uint32_t t) { out[j * kTile] = t; });
         nbrCount[c.i] = cnt;
-        if (cnt) atomicMax(&rows, cnt);
     }
-    if (VFD_STAGE_LISTS) {
-        __syncthreads();
-        const uint32_t nr = rows;
-        for (uint32_t j = 0; j < nr; ++j)
-            if (j < cnt) nbrList[(size_t)j * capacity + c.i] = stage[j * kTile + threadIdx.x];
-    }
-    // per-scene total and maximum neighbour count (debug statistics)
-    int tot = (int)cnt, mx = (int)cnt;
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) {
-        tot += __shfl_xor(tot, o, kWave);
-        mx = max(mx, __shfl_xor(mx, o, kWave));
-    }
-    if ((threadIdx.x & (kWave - 1)) == 0 && tot > 0) {
-        atomicAdd(&nbStats[2 * c.s], (unsigned long long)tot);
-        atomicMax(&nbStats[2 * c.s + 1], (unsigned long long)mx);
-    }
-}
-
-// ---- cell-parallel list build (VFD_SEARCH_CELLS) ---------------------------------------------------------------------
-#ifndef VFD_SEARCH_CELLS
-#define VFD_SEARCH_CELLS 0
-#endif
-constexpr uint32_t kCellWaves = kTile / kWave;
-
-__device__ __forceinline__ uint32_t slot_cell(const SceneGrid& g, const float4& x) {  // k_insert's key
-    const float fx = (x.x - g.gridMin[0]) * g.gridDelta[0];
-    const float fy = (x.y - g.gridMin[1]) * g.gridDelta[1];
-    const float fz = (x.z - g.gridMin[2]) * g.gridDelta[2];
-    return cell_key(g, clampu((int)fx, g.dims[0]), clampu((int)fy, g.dims[1]), clampu((int)fz, g.dims[2]));
-}
-
-// Every wave owns the 64 slots of its window and builds exactly their lists. The window's particles fall into runs of
-// one grid cell (segments: a cell may begin before the window or end after it; only the window's own particles are
-// handled). A segment's particles share the 27 candidate ranges, so the wave loads the candidates once, 64 per chunk
-// with a lane per candidate (consecutive slots of a range are consecutive lanes: few, coalesced loads instead of one
-// load per particle and candidate), and tests them against each of the segment's particles in turn; a ballot gives
-// each accepted candidate its rank in that particle's list (candidates are visited in list order: ranges in z, y, x
-// order, slots ascending), so the first kMaxNeighbors are kept exactly as the per-particle traversal keeps them.
-// Entries are staged in LDS as 16-bit {range, offset} codes in [row][lane] (rows padded so that the ranks of one
-// particle fall into different banks), decoded with the segment's range starts and written at the end as whole
-// 256-byte rows of 64 consecutive slots. A segment that does not fit the codes (a range of 2048 or more particles,
-// or a window of more than kWinSegs cells) stores its entries directly instead.
-constexpr uint32_t kWinPitch = kWave + 2;  // u16 entries per staged row
-constexpr uint32_t kWinSegs = 16;          // segments per window with staged entries
-constexpr uint32_t kWinDirect = 0xFFu;     // segment index of a lane whose entries went straight to HBM
-// lane q's value (q wave-uniform), read into a scalar register
-__device__ __forceinline__ float rdlane(float v, uint32_t q) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), (int)q));
-}
-__device__ __forceinline__ uint32_t rdlane(uint32_t v, uint32_t q) {
-    return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)q);
-}
-__global__ void __launch_bounds__(kTile) k_build_lists_cells(const float4* __restrict__ pos,
-                                                           const SceneParams* __restrict__ P,
-                                                           const SceneGrid* __restrict__ G,
-                                                           const uint32_t* __restrict__ tileScene, uint32_t tiles,
-                                                           uint32_t per, const uint32_t* __restrict__ cellStart,
-                                                           const uint32_t* __restrict__ cellCount, uint32_t* nbrCount,
-                                                           uint32_t* nbrList, uint32_t capacity,
-                                                           unsigned long long* nbStats) {
-    __shared__ uint16_t stage[kCellWaves][kMaxNeighbors * kWinPitch];
-    __shared__ uint32_t tabStart[kCellWaves][kWinSegs][28];  // range starts of the staged segments
-    __shared__ uint32_t pre[kCellWaves][32];  // exclusive prefix of the 27 range lengths of the current segment
-    __shared__ uint32_t cst[kCellWaves][32];  // first slot of each range of the current segment
-    const uint32_t tile = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
-    if (tile >= tiles) return;  // block-uniform
-    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
-    const uint32_t s = tileScene[tile];
-    const SceneParams& p = P[s];
-    const SceneGrid& g = G[s];
-    const uint32_t end = p.base + p.count;
-    const uint32_t win0 = tile * kTile + w * kWave;  // first slot of the window
-    const uint32_t i = win0 + lane;
-    const bool valid = i < end;
-    const float4 x = valid ? pos[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    const uint32_t key = valid ? slot_cell(g, x) : 0xFFFFFFFFu;
-    const uint32_t prevKey = __shfl_up(key, 1, kWave);
-    unsigned long long segs = __ballot(valid && (lane == 0 || key != prevKey));  // first lane of each segment
-    const uint32_t nvalid = (uint32_t)__popcll(__ballot(valid));  // the valid lanes are the first nvalid
-    const float R2 = p.R * p.R;
-    uint16_t* st = stage[w];
-    uint32_t cnt = 0;            // accepted neighbours of this lane's particle (only the first kMaxNeighbors are kept)
-    uint32_t mySeg = kWinDirect;  // this lane's staged segment
-    for (uint32_t seg = 0; segs; ++seg) {
-        const uint32_t b = (uint32_t)__ffsll(segs) - 1u;
-        segs &= segs - 1ull;
-        const uint32_t e = segs ? (uint32_t)__ffsll(segs) - 1u : nvalid;  // segment lanes [b, e)
-        const float xlx = rdlane(x.x, b), xly = rdlane(x.y, b), xlz = rdlane(x.z, b);
-        // the cell of the key (k_insert's clamped cell; for a particle inside the grid the cell the per-particle
-        // traversal takes with floorf)
-        const int gx = (int)clampu((int)((xlx - g.gridMin[0]) * g.gridDelta[0]), g.dims[0]);
-        const int gy = (int)clampu((int)((xly - g.gridMin[1]) * g.gridDelta[1]), g.dims[1]);
-        const int gz = (int)clampu((int)((xlz - g.gridMin[2]) * g.gridDelta[2]), g.dims[2]);
-        uint32_t cn = 0, cs = 0;
-        if (lane < 27) {
-            const int cx = gx + (int)(lane % 3) - 1, cy = gy + (int)((lane / 3) % 3) - 1, cz = gz + (int)(lane / 9) - 1;
-            if (cx >= 0 && cx < (int)g.dims[0] && cy >= 0 && cy < (int)g.dims[1] && cz >= 0 && cz < (int)g.dims[2]) {
-                const uint32_t k = cell_key(g, (uint32_t)cx, (uint32_t)cy, (uint32_t)cz);
-                cn = cellCount[k];
-                cs = (uint32_t)((int32_t)cellStart[k] + g.startCorr);
-            }
-        }
-        const bool staged = seg < kWinSegs && __ballot(cn >= 2048u) == 0ull;  // wave-uniform
-        uint32_t incl = cn;
-#pragma unroll
-        for (int o = 1; o < 32; o <<= 1) {
-            const uint32_t t = __shfl_up(incl, o, kWave);
-            if ((int)lane >= o) incl += t;
-        }
-        const uint32_t T = rdlane(incl, 26);  // candidates in the 27 ranges
-        if (lane < 27) {
-            pre[w][lane] = incl - cn;
-            cst[w][lane] = cs;
-            if (staged) tabStart[w][seg][lane] = cs;
-        }
-        if (lane >= b && lane < e) mySeg = staged ? seg : kWinDirect;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        // candidate t of the segment's stream: its range (the last one whose prefix is <= t) and offset in it
-        auto locate = [&](uint32_t t, uint32_t& off) {
-            uint32_t r = 0;
-#pragma unroll
-            for (uint32_t step = 16; step > 0; step >>= 1)
-                if (r + step < 27 && pre[w][r + step] <= t) r += step;
-            off = t - pre[w][r];
-            return r;
-        };
-        uint32_t offN = 0, rN = lane < T ? locate(lane, offN) : 0u;
-        uint32_t slotN = lane < T ? cst[w][rN] + offN : 0u;
-        float4 xjN = lane < T ? pos[slotN] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        for (uint32_t c0 = 0; c0 < T; c0 += kWave) {
-            const uint32_t slot = slotN, code = (rN << 11) | offN;
-            const float4 xj = xjN;
-            const bool has = c0 + lane < T;
-            if (c0 + kWave < T) {  // the next chunk's candidates are requested before this chunk is tested
-                const uint32_t tn = c0 + kWave + lane;
-                rN = tn < T ? locate(tn, offN) : 0u;
-                slotN = tn < T ? cst[w][rN] + offN : 0u;
-                xjN = tn < T ? pos[slotN] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            }
-            for (uint32_t q = b; q < e; ++q) {  // wave-uniform: the segment's particles in slot order
-                const float xqx = rdlane(x.x, q), xqy = rdlane(x.y, q), xqz = rdlane(x.z, q);
-                const float ddx = xj.x - xqx, ddy = xj.y - xqy, ddz = xj.z - xqz;
-                const float d2 = fmaf(ddz, ddz, fmaf(ddy, ddy, ddx * ddx));
-                const bool acc = has && d2 < R2 && d2 > 0.0f;
-                const unsigned long long bal = __ballot(acc);
-                const uint32_t cq = rdlane(cnt, q);
-                if (acc) {
-                    const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
-                                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-                    const uint32_t rank = cq + below;  // accepted lanes before this one
-                    if (rank < kMaxNeighbors) {
-                        if (staged)
-                            st[rank * kWinPitch + q] = (uint16_t)code;
-                        else
-                            nbrList[(size_t)rank * capacity + win0 + q] = slot;
-                    }
-                }
-                if (lane == q) cnt += (uint32_t)__popcll(bal);
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    // the window's rows, whole: row r holds entry r of each of the 64 slots
-    const uint32_t n = valid ? min(cnt, kMaxNeighbors) : 0u;
-    uint32_t rows = n;
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) rows = max(rows, (uint32_t)__shfl_xor(rows, o, kWave));
-    const uint32_t* ts = tabStart[w][mySeg < kWinSegs ? mySeg : 0u];
-    for (uint32_t r = 0; r < rows; ++r) {
-        if (r < n && mySeg != kWinDirect) {
-            const uint32_t code = st[r * kWinPitch + lane];
-            nbrList[(size_t)r * capacity + i] = ts[code >> 11] + (code & 2047u);
-        }
-    }
-    if (valid) nbrCount[i] = n;
-    // per-scene total and maximum neighbour count (debug statistics)
-    unsigned long long t = n;
-    uint32_t mx = n;
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) {
-        t += __shfl_xor(t, o, kWave);
-        mx = max(mx, (uint32_t)__shfl_xor(mx, o, kWave));
-    }
-    if (lane == 0 && t > 0) {
-        atomicAdd(&nbStats[2 * s], t);
-        atomicMax(&nbStats[2 * s + 1], (unsigned long long)mx);
-    }
+    note_neighbors(cnt, blockIdx.x, tileStats);
 }
 
 // ---- exclusive scan of uint32 (cell counts) --------------------------------------------------------------------
@@ -565,11 +378,6 @@ void launch_sort(const Launch& L, const SceneGrid* G, uint32_t totalCells, const
                        (const uint32_t*)tmpId, posIn, velIn, dvIn, dkIn, idIn, posOut, velOut, dvOut, dkOut, idOut);
 }
 
-__global__ void k_fill_u64(unsigned long long* p, uint32_t n) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0ull;
-}
-
 // ---- halos of the neighbour groups ------------------------------------------------------------------------------
 // One block per group of kTiles tiles. The distinct particle slots among the lists of its particles are collected in an
 // LDS hash set of 32-slot buckets (bucket = slot >> 5, Fibonacci-hashed, linear probing) with a presence mask each;
@@ -592,8 +400,7 @@ template <unsigned kTiles>
 __global__ void __launch_bounds__(kTiles * kTile) k_build_halo(const SceneParams* __restrict__ P,
                                                            const uint32_t* __restrict__ tileScene, uint32_t tiles,
                                                            const uint32_t* __restrict__ nbrCount,
-                                                           const uint32_t* __restrict__ nbrList, uint32_t cap,
-                                                           uint32_t limit, uint32_t* haloCount, uint32_t* haloIds,
+                                                           const uint32_t* __restrict__ nbrList, uint32_t limit, uint32_t* haloCount, uint32_t* haloIds,
                                                            uint32_t* nbrLocal, uint32_t* haloStats,
                                                            const float4* __restrict__ pos, float R, float invStep) {
     constexpr uint32_t kThreads = kTiles * kTile, kFill = halo_fill(kTiles);
@@ -631,7 +438,7 @@ __global__ void __launch_bounds__(kTiles * kTile) k_build_halo(const SceneParams
     for (uint32_t j0 = 0; j0 < nr; j0 += kHaloBatch) {
         uint32_t tb[kHaloBatch];
 #pragma unroll
-        for (uint32_t u = 0; u < kHaloBatch; ++u) tb[u] = j0 + u < n ? nbrList[(size_t)(j0 + u) * cap + i] : 0u;
+        for (uint32_t u = 0; u < kHaloBatch; ++u) tb[u] = j0 + u < n ? nbrList[list_at(i, j0 + u)] : 0u;
 #pragma unroll
         for (uint32_t u = 0; u < kHaloBatch; ++u) {
             if (j0 + u >= n || *vused > kBucketLimit) continue;
@@ -720,7 +527,7 @@ __global__ void __launch_bounds__(kTiles * kTile) k_build_halo(const SceneParams
     }
     __syncthreads();
     // staged entries: the halo number of each neighbour | its table code << 16, in list order (the neighbour's
-    // position from the halo's copy in LDS), rows in pairs ([j/2][cap][2]: one 8-byte store per row pair; the entry
+    // position from the halo's copy in LDS), rows in pairs (one 8-byte store per row pair; the entry
     // after a list's last one is 0 and never read)
     static_assert(kHaloBatch % 2 == 0 && kMaxNeighbors % 2 == 0, "staged rows are stored in pairs");
     const f3 xi = n ? ld3(pos[i]) : mk3(0.0f, 0.0f, 0.0f);
@@ -729,7 +536,7 @@ __global__ void __launch_bounds__(kTiles * kTile) k_build_halo(const SceneParams
         // the list's last read in the step: non-temporal loads (it would only displace cached positions)
 #pragma unroll
         for (uint32_t u = 0; u < kHaloBatch; ++u)
-            tb[u] = j0 + u < n ? __builtin_nontemporal_load(nbrList + (size_t)(j0 + u) * cap + i) : 0u;
+            tb[u] = j0 + u < n ? __builtin_nontemporal_load(nbrList + list_at(i, j0 + u)) : 0u;
         uint32_t en[kHaloBatch];
 #pragma unroll
         for (uint32_t u = 0; u < kHaloBatch; ++u) {
@@ -743,10 +550,10 @@ __global__ void __launch_bounds__(kTiles * kTile) k_build_halo(const SceneParams
             const uint32_t code = gcode<false>(R, invStep, xi - mk3(hpos[3 * s], hpos[3 * s + 1], hpos[3 * s + 2]));
             en[u] = s | (code << 16);
         }
-        uint2* out = reinterpret_cast<uint2*>(nbrLocal) + (size_t)(j0 >> 1) * cap + i;
+        uint2* out = reinterpret_cast<uint2*>(nbrLocal) + local_at(i, j0 >> 1);
 #pragma unroll
         for (uint32_t u = 0; u < kHaloBatch; u += 2)
-            if (j0 + u < n) out[(size_t)(u >> 1) * cap] = make_uint2(en[u], en[u + 1]);
+            if (j0 + u < n) out[(u >> 1) * kTile] = make_uint2(en[u], en[u + 1]);
     }
 }
 
@@ -756,7 +563,7 @@ void launch_build_halo(const Launch& L, uint32_t groupTiles, const uint32_t* nbr
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, L.stream, haloStats, 0u, 3u);
     const auto run = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(L.group_count(groupTiles)), dim3(groupTiles * kTile), kLdsHaloPos, L.stream,
-                           L.P, L.tileScene, L.tiles, nbrCount, nbrList, L.capacity,
+                           L.P, L.tileScene, L.tiles, nbrCount, nbrList,
                            std::min<uint32_t>(haloLimit, halo_cap(groupTiles)), haloCount, haloIds, nbrLocal,
                            haloStats, pos, kt.R, kt.invStep);
     };
@@ -770,24 +577,16 @@ void launch_build_halo(const Launch& L, uint32_t groupTiles, const uint32_t* nbr
 
 void launch_build_lists(const Launch& L, const SceneGrid* G, const float4* pos, const uint32_t* cellStart,
                         const uint32_t* cellCount, uint32_t* nbrCount, uint32_t* nbrList,
-                        unsigned long long* nbStats) {
-    hipLaunchKernelGGL(k_fill_u64, dim3((2 * L.sceneCount + 63) / 64), dim3(64), 0, L.stream, nbStats,
-                       2 * L.sceneCount);
-    if (VFD_SEARCH_CELLS)
-        hipLaunchKernelGGL(k_build_lists_cells, dim3(L.gridAll), dim3(kTile), 0, L.stream, pos, L.P, G, L.tileScene,
-                           L.tiles, L.tg.per, cellStart, cellCount, nbrCount, nbrList, L.capacity, nbStats);
-    else
-        hipLaunchKernelGGL(k_build_lists, dim3(L.tiles), dim3(kTile), kLdsListStage, L.stream, pos, L.P, G,
-                           L.tileScene, cellStart, cellCount, nbrCount, nbrList, L.capacity, nbStats);
+                        uint2* tileStats) {
+    hipLaunchKernelGGL(k_build_lists, dim3(L.tiles), dim3(kTile), 0, L.stream, pos, L.P, G, L.tileScene, cellStart,
+                       cellCount, nbrCount, nbrList, tileStats);
 }
 
 int configure_search_kernels() {
     for (const void* fn : {(const void*)k_build_halo<1>, (const void*)k_build_halo<2>, (const void*)k_build_halo<4>})
         if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsHaloPos) != hipSuccess)
             return 1;
-    if (kLdsListStage == 0) return 0;
-    return hipFuncSetAttribute((const void*)k_build_lists, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)kLdsListStage) == hipSuccess ? 0 : 1;
+    return 0;
 }
 
 // ---- static scratch of the allocation-free step -------------------------------------------------------------------

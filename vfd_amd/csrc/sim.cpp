@@ -460,7 +460,7 @@ public:
     DevBuf<uint32_t> id[2], nbrCount, nbrList, cellOf, rank, tmpId, surface, cellCount, cellStart, scanScratch, live;
     DevBuf<double> partials;
     DevBuf<float> partialsF;
-    DevBuf<unsigned long long> nbStats;
+    DevBuf<uint2> tileStats;  // each tile's neighbour total and longest list
     DevBuf<uint32_t> haloCount, haloIds, haloStats;
     DevBuf<uint32_t> nbrLocal;
 
@@ -1013,7 +1013,7 @@ public:
             s->prm.bodyCount = (uint32_t)s->bodies.size();
         }
         cap = tiles * kTile;
-        // a pair of staged-list rows (cap 8-byte entries) is read as one buffer whose byte offsets stay below 2^31
+        // 32-bit slot arithmetic (8 bytes a slot stay below 2^31)
         if ((uint64_t)cap * 2 * sizeof(uint32_t) >= (1ull << 31))
             return fail(VFD_ERROR_NOT_SUPPORTED, "at most 2^28 particle slots in one simulation");
         const uint32_t S = (uint32_t)sc.size();
@@ -1046,7 +1046,7 @@ public:
         VFD_TRY(nbrList.alloc(c * kMaxNeighbors));
         VFD_TRY(partials.alloc((size_t)std::max<uint32_t>(tiles, 1) * kPartialSlots));
         VFD_TRY(partialsF.alloc(std::max<uint32_t>(tiles, 1)));
-        VFD_TRY(nbStats.alloc((size_t)2 * S));
+        VFD_TRY(tileStats.alloc(std::max<uint32_t>(tiles, 1)));
         {
             const Launch L = launch();
             const uint32_t rt = resident_group_tiles(L, numCU);
@@ -1231,7 +1231,7 @@ public:
         }));
         cur = alt;
         VFD_TRY(timed("build_lists", [&] {
-            launch_build_lists(L, dGrid.p, pos.p, cStart, cCount, nbrCount.p, nbrList.p, nbStats.p);
+            launch_build_lists(L, dGrid.p, pos.p, cStart, cCount, nbrCount.p, nbrList.p, tileStats.p);
         }));
         VFD_HIP(hipGetLastError());
         return VFD_OK;
@@ -1303,7 +1303,7 @@ public:
     static constexpr int kStepAborted = -1;
     // The step's report, written behind its launches, and the wait for it; kStepAborted when a resident solve was aborted
     int drain() {
-        launch_report(launch(), dState.p, nbStats.p, haloStats.p, residentWords.p, report, sceneReport);
+        launch_report(launch(), dState.p, tileStats.p, haloStats.p, residentWords.p, report, sceneReport);
         VFD_HIP(hipGetLastError());
         VFD_HIP(hipStreamSynchronize(stream));
         return report->aborted ? kStepAborted : VFD_OK;
@@ -1884,16 +1884,15 @@ public:
         if (counts) std::memcpy(counts, cOrig.data(), S.count * sizeof(uint32_t));
         if (offsets) std::memcpy(offsets, off.data(), S.count * sizeof(uint32_t));
         if (!out) return VFD_OK;
-        std::vector<uint32_t> rows((size_t)kMaxNeighbors * S.count);
-        for (uint32_t j = 0; j < kMaxNeighbors; ++j)
-            if (S.count)
-                VFD_HIP(hipMemcpyAsync(&rows[(size_t)j * S.count], nbrList.p + (size_t)j * cap + S.base,
-                                       S.count * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
+        std::vector<uint32_t> lists((size_t)((S.count + kTile - 1) / kTile) * kTileList);  // the scene's tiles
+        if (S.count)
+            VFD_HIP(hipMemcpyAsync(lists.data(), nbrList.p + list_at(S.base, 0), lists.size() * sizeof(uint32_t),
+                                   hipMemcpyDeviceToHost, stream));
         VFD_HIP(hipStreamSynchronize(stream));
         for (uint32_t k = 0; k < S.count; ++k) {
             const uint32_t i = idv[k];
             for (uint32_t j = 0; j < cnt[k]; ++j) {
-                const uint32_t t = rows[(size_t)j * S.count + k];
+                const uint32_t t = lists[list_at(k, j)];
                 if (t < S.base || t >= S.base + S.count) return fail(VFD_ERROR_STATE, "neighbour outside its scene");
                 out[off[i] + j] = idv[t - S.base];
             }

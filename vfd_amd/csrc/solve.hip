@@ -450,12 +450,7 @@ template <unsigned kTiles> struct PairSums {
     }
     // staged entries 2j, 2j + 1 (0 past the list's end, without a memory access; see each_neighbor_rec)
     __device__ __forceinline__ uint2 entries(uint32_t j) const {
-        const __amdgpu_buffer_rsrc_t row = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint32_t*>(r.src.local + (size_t)j * r.src.cap * 2), (short)0, (int)(r.src.cap * 8),
-            kRawBufferWord3);
-        const uint32_t off = r.c.i * 8u + (2 * j < n ? 0u : kBufferOutOfRange);
-        const auto v = __builtin_amdgcn_raw_buffer_load_b64(row, (int)off, 0, 0);
-        return make_uint2(v[0], v[1]);
+        return TileLists(r.src.local, r.c.i).pair<0>(j, 2 * j < n);
     }
     __device__ __forceinline__ void begin() {
         fill_halo(r, [&](uint32_t t) { return PosVec{ld3(F.pos[t]), ld3(F.vel[t])}; },

@@ -10,7 +10,7 @@ namespace vfd {
 
 __device__ __forceinline__ KTab ktab(const KTabHost& h) { return KTab{h.tab, h.R, h.R2, h.invStep, h.W0}; }
 __device__ __forceinline__ uint32_t nbr(const Fields& F, uint32_t cap, uint32_t i, uint32_t j) {
-    return F.nbrList[(size_t)j * cap + i];
+    return F.nbrList[list_at(i, j)];
 }
 __device__ __forceinline__ HaloView halo(const Fields& F) { return HaloView{F.haloCount, F.haloIds}; }
 __device__ __forceinline__ NbrSrc global_src(const Fields& F, uint32_t cap) {
