@@ -638,7 +638,7 @@ __global__ void __launch_bounds__(kGroupSize, kGroupsPerCU) k_cg_matvec(const Sc
             v[0] = (double)dot3(ld3(F.cgP[c.i]), ap);
         }
         tile_partials4<1>(v, F.partials, tile, act);
-    });
+    }, [&](uint32_t tile) { return F.state[tileScene[tile]].cg.active != 0u; });
 }
 
 __global__ void __launch_bounds__(kFinishThreads) k_cg_alpha(const SceneParams* __restrict__ P, Fields F) {
