@@ -7,9 +7,9 @@
 //   neighbour lists: uint32 slot indices, at most kMaxNeighbors per particle, tile by tile and transposed inside a tile
 //   ([tile][j][kTile], list_at) so that the j-th neighbour of 64 consecutive particles is one coalesced 256-byte access
 //   and a tile's lists are one stretch of 70 KB; for the particles of a staged group also as uint16 halo slots and
-//   uint16 kernel-table codes of the pairs, rows in pairs ([tile][j / 2][kTile][2], local_at). With rows as long as the
-//   state instead ([j][capacity]) a wave's stores of its lists went to 40 rows megabytes apart: k_build_lists took
-//   659 us instead of 597 on 2 million particles, 198 instead of 178 on 500,000;
+//   uint16 kernel-table codes of the pairs, rows in pairs ([tile][j / 2][kTile][2], local_at) (one buffer
+//   for the staged loops' loads; rows as long as the state instead, [j][capacity], spread a wave's stores over 40 rows
+//   megabytes apart: 659 -> 652 us of k_build_lists on 2 million particles);
 //   halos: per group, haloCount[g] and the halo's particle slots haloIds[g * kHaloMax + k].
 //
 // All HIP sources are compiled with -ffp-contract=off: every fused multiply-add is an explicit fmaf, so the
