@@ -942,7 +942,6 @@ __global__ void __launch_bounds__(kTile) k_st_blend(const SceneParams* __restric
 }
 
 void launch_surface_tension(const Launch& L, const Fields& F) {
-    launch_fill_u32(L.stream, F.surface, 0u, 1u);
     hipLaunchKernelGGL(k_st_classify, dim3(L.tiles), dim3(kTile), 0, L.stream, L.P, L.tileScene, F, L.capacity, L.stamps);
     // enough waves for the chip (eight a SIMD); a tile has no more candidates than its 256 particles
     hipLaunchKernelGGL(k_st_sample, dim3(std::min(L.tiles * kWave, 2048u)), dim3(kTile), 0, L.stream, L.P, L.tileScene, F,

@@ -194,8 +194,10 @@ void exclusive_scan(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* scr
 void launch_fill_u32(hipStream_t st, uint32_t* p, uint32_t v, uint32_t n);
 // mm: 6 bounds per scene, in memory that the host reads
 void launch_minmax(const Launch& L, const float4* pos, int* part, int* mm);
-// clears the cell counts and, with args, writes the scenes' grids (at most kGridArgs) to G
-void launch_sort_begin(const Launch& L, const GridArgs* args, SceneGrid* G, uint32_t* cellCount, uint32_t totalCells);
+// clears the cell counts, the halo statistics and the count of surface candidates (Fields::surface) and, with args,
+// writes the scenes' grids (at most kGridArgs) to G
+void launch_sort_begin(const Launch& L, const GridArgs* args, SceneGrid* G, uint32_t* cellCount, uint32_t totalCells,
+                       uint32_t* haloStats, uint32_t* surface);
 void launch_sort(const Launch& L, const SceneGrid* G, uint32_t totalCells, const float4* posIn, const float4* velIn,
                  const float4* dvIn, const float* dkIn, const uint32_t* idIn, float4* posOut, float4* velOut,
                  float4* dvOut, float* dkOut, uint32_t* idOut, uint32_t* cellOf, uint32_t* rank, uint32_t* tmpId,

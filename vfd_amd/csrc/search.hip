@@ -358,14 +358,17 @@ void launch_minmax(const Launch& L, const float4* pos, int* part, int* mm) {
 }
 
 __global__ void __launch_bounds__(kTile) k_sort_begin(GridArgs args, SceneGrid* G, uint32_t scenes, uint32_t* cellCount,
-                                                      uint32_t totalCells) {
+                                                      uint32_t totalCells, uint32_t* haloStats, uint32_t* surface) {
     const uint32_t i = blockIdx.x * kTile + threadIdx.x;
     if (i < scenes) G[i] = args.g[i];
+    if (i < 3u) haloStats[i] = 0u;
+    if (i == 0u) surface[0] = 0u;
     for (uint32_t c = i; c < totalCells; c += gridDim.x * kTile) cellCount[c] = 0u;
 }
-void launch_sort_begin(const Launch& L, const GridArgs* args, SceneGrid* G, uint32_t* cellCount, uint32_t totalCells) {
+void launch_sort_begin(const Launch& L, const GridArgs* args, SceneGrid* G, uint32_t* cellCount, uint32_t totalCells,
+                       uint32_t* haloStats, uint32_t* surface) {
     hipLaunchKernelGGL(k_sort_begin, dim3(std::min((totalCells + kTile - 1) / kTile, 2048u)), dim3(kTile), 0, L.stream,
-                       args ? *args : GridArgs{}, G, args ? L.sceneCount : 0u, cellCount, totalCells);
+                       args ? *args : GridArgs{}, G, args ? L.sceneCount : 0u, cellCount, totalCells, haloStats, surface);
 }
 
 void launch_sort(const Launch& L, const SceneGrid* G, uint32_t totalCells, const float4* posIn, const float4* velIn,
@@ -400,14 +403,19 @@ static_assert(kBucketLimit + 4 * kTile < kBucketSlots, "bucket table must never 
 __device__ __forceinline__ uint32_t bucket_hash(uint32_t b) { return (b * 0x9E3779B1u) >> 21; }  // 11 bits
 constexpr size_t kLdsHaloPos = (size_t)kHaloMax * 3 * sizeof(float);  // halo positions of k_build_halo
 
-template <unsigned kTiles>
-__global__ void __launch_bounds__(kTiles * kTile) k_build_halo(const SceneParams* __restrict__ P,
+//
+// Smaller groups (the resident solves') have fewer threads than a CU runs, and each entry is a chain of LDS reads: there
+// kSplit threads share a particle's list, a batch of entries each in turn: 30.5 -> 15.4 us on 990 particles (groups of
+// 256), 46.8 -> 34.9 us on 123,000 (groups of 512).
+template <unsigned kTiles, unsigned kSplit = (kTiles < kGroupTiles ? kGroupTiles / kTiles : 1u)>
+__global__ void __launch_bounds__(kTiles * kTile * kSplit) k_build_halo(const SceneParams* __restrict__ P,
                                                            const uint32_t* __restrict__ tileScene, uint32_t tiles,
                                                            const uint32_t* __restrict__ nbrCount,
                                                            const uint32_t* __restrict__ nbrList, uint32_t limit, uint32_t* haloCount, uint32_t* haloIds,
                                                            uint32_t* nbrLocal, uint32_t* haloStats,
                                                            const float4* __restrict__ pos, float R, float invStep) {
-    constexpr uint32_t kThreads = kTiles * kTile, kFill = halo_fill(kTiles);
+    constexpr uint32_t kOwn = kTiles * kTile, kThreads = kOwn * kSplit;
+    constexpr uint32_t kFill = (halo_cap(kTiles) + kThreads - 1) / kThreads;
     __shared__ uint32_t bkey[kBucketSlots];
     __shared__ uint32_t bmask[kBucketSlots];
     __shared__ uint16_t bbase[kBucketSlots];
@@ -415,8 +423,8 @@ __global__ void __launch_bounds__(kTiles * kTile) k_build_halo(const SceneParams
     __shared__ uint32_t used, rows;
     extern __shared__ float hpos[];  // [kHaloMax * 3]: positions of the halo, by halo number
     const uint32_t g = blockIdx.x;
-    const uint32_t tile = g * kTiles + threadIdx.x / kTile;
-    const uint32_t i = g * kThreads + threadIdx.x;
+    const uint32_t i = g * kOwn + threadIdx.x % kOwn, tile = i / kTile;
+    const uint32_t share = threadIdx.x / kOwn;  // which of the list's batches are this thread's
     uint32_t n = 0;
     if (tile < tiles) {
         const SceneParams& p = P[tileScene[tile]];
@@ -439,7 +447,7 @@ __global__ void __launch_bounds__(kTiles * kTile) k_build_halo(const SceneParams
     volatile uint32_t* vused = &used;
     // the list entries are loaded kHaloBatch at a time (their latencies overlap), then inserted in list order
     constexpr uint32_t kHaloBatch = 8;
-    for (uint32_t j0 = 0; j0 < nr; j0 += kHaloBatch) {
+    for (uint32_t j0 = share * kHaloBatch; j0 < nr; j0 += kSplit * kHaloBatch) {
         uint32_t tb[kHaloBatch];
 #pragma unroll
         for (uint32_t u = 0; u < kHaloBatch; ++u) tb[u] = j0 + u < n ? nbrList[list_at(i, j0 + u)] : 0u;
@@ -467,7 +475,7 @@ __global__ void __launch_bounds__(kTiles * kTile) k_build_halo(const SceneParams
         }
     }
     __syncthreads();
-    // halo numbers: thread t owns bucket slots [2t, 2t + 2)
+    // halo numbers: thread t owns bucket slots [kPer * t, kPer * (t + 1))
     constexpr uint32_t kPer = kBucketSlots / kThreads;
     uint32_t own = 0;
 #pragma unroll
@@ -535,7 +543,7 @@ __global__ void __launch_bounds__(kTiles * kTile) k_build_halo(const SceneParams
     // after a list's last one is 0 and never read)
     static_assert(kHaloBatch % 2 == 0 && kMaxNeighbors % 2 == 0, "staged rows are stored in pairs");
     const f3 xi = n ? ld3(pos[i]) : mk3(0.0f, 0.0f, 0.0f);
-    for (uint32_t j0 = 0; j0 < nr; j0 += kHaloBatch) {
+    for (uint32_t j0 = share * kHaloBatch; j0 < nr; j0 += kSplit * kHaloBatch) {
         uint32_t tb[kHaloBatch];
         // the list's last read in the step: non-temporal loads (it would only displace cached positions)
 #pragma unroll
@@ -564,10 +572,9 @@ __global__ void __launch_bounds__(kTiles * kTile) k_build_halo(const SceneParams
 void launch_build_halo(const Launch& L, uint32_t groupTiles, const uint32_t* nbrCount, const uint32_t* nbrList,
                        uint32_t haloLimit, uint32_t* haloCount, uint32_t* haloIds, uint32_t* nbrLocal,
                        uint32_t* haloStats, const float4* pos, const KTabHost& kt) {
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, L.stream, haloStats, 0u, 3u);
     const auto run = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(L.group_count(groupTiles)), dim3(groupTiles * kTile), kLdsHaloPos, L.stream,
-                           L.P, L.tileScene, L.tiles, nbrCount, nbrList,
+        hipLaunchKernelGGL(kernel, dim3(L.group_count(groupTiles)), dim3(std::max(groupTiles, kGroupTiles) * kTile),
+                           kLdsHaloPos, L.stream, L.P, L.tileScene, L.tiles, nbrCount, nbrList,
                            std::min<uint32_t>(haloLimit, halo_cap(groupTiles)), haloCount, haloIds, nbrLocal,
                            haloStats, pos, kt.R, kt.invStep);
     };

@@ -1224,7 +1224,8 @@ public:
             VFD_HIP(hipMemcpyAsync(dGrid.p, hostGrids, S * sizeof(SceneGrid), hipMemcpyHostToDevice, stream));
         const int alt = cur ^ 1;
         VFD_TRY(timed("sort", [&] {
-            launch_sort_begin(L, S <= kGridArgs ? &args : nullptr, dGrid.p, cCount, cellTotal);
+            launch_sort_begin(L, S <= kGridArgs ? &args : nullptr, dGrid.p, cCount, cellTotal, haloStats.p,
+                              surface.p);
             launch_sort(L, dGrid.p, cellTotal, posNext.p, vel[cur].p, dv[cur].p, dk[cur].p, id[cur].p, pos.p,
                         vel[alt].p, dv[alt].p, dk[alt].p, id[alt].p, cellOf.p, rank.p, tmpId.p, cCount, cStart,
                         cScan);
@@ -1597,6 +1598,7 @@ public:
             VFD_TRY(aHaloIds.alloc((size_t)std::max<uint32_t>(L.groups, 1) * kHaloMax));
             VFD_TRY(aNbrLocal.alloc((size_t)cap * kMaxNeighbors));
             VFD_TRY(aHaloStats.alloc(3));
+            launch_fill_u32(stream, aHaloStats.p, 0u, 3u);
             launch_build_halo(L, kGroupTiles, t.count.p, t.list.p, haloLimit, aHaloCount.p, aHaloIds.p, aNbrLocal.p, aHaloStats.p,
                               t.x.p, ktab());
             A.groups.grid = L.gridGroups;
