@@ -415,11 +415,11 @@ __global__ void __launch_bounds__(kFinishThreads) k_report(const SceneParams* __
                                                            const uint2* __restrict__ tileStats,
                                                            const uint32_t* __restrict__ haloStats,
                                                            const uint32_t* __restrict__ words, const long long* stamps,
-                                                           StepReport* report, SceneReport* scenes) {
+                                                           StepReport* report, SceneReport* scenes, uint32_t perTile) {
     __shared__ unsigned long long total[kFinishThreads / kWave], longest[kFinishThreads / kWave];
     const uint32_t s = blockIdx.x;
     unsigned long long tot = 0, mx = 0;
-    for (uint32_t t = P[s].tileBegin + threadIdx.x; t < P[s].tileEnd; t += kFinishThreads) {
+    for (uint32_t t = P[s].tileBegin * perTile + threadIdx.x; t < P[s].tileEnd * perTile; t += kFinishThreads) {
         const uint2 v = tileStats[t];
         tot += v.x;
         mx = max(mx, (unsigned long long)v.y);
@@ -451,7 +451,7 @@ __global__ void __launch_bounds__(kFinishThreads) k_report(const SceneParams* __
 void launch_report(const Launch& L, const SceneState* state, const uint2* tileStats, const uint32_t* haloStats,
                    const uint32_t* words, StepReport* report, SceneReport* scenes) {
     hipLaunchKernelGGL(k_report, dim3(L.sceneCount), dim3(kFinishThreads), 0, L.stream, L.P, state, tileStats, haloStats,
-                       words, (const long long*)L.stamps, report, scenes);
+                       words, (const long long*)L.stamps, report, scenes, list_stats_per_tile(L.tiles));
 }
 
 __global__ void __launch_bounds__(kTile) k_restore(const SceneParams* __restrict__ P,

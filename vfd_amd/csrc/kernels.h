@@ -205,6 +205,8 @@ void launch_sort(const Launch& L, const SceneGrid* G, uint32_t totalCells, const
 void launch_build_halo(const Launch& L, uint32_t groupTiles, const uint32_t* nbrCount, const uint32_t* nbrList,
                        uint32_t haloLimit, uint32_t* haloCount, uint32_t* haloIds, uint32_t* nbrLocal, uint32_t* haloStats,
                        const float4* pos, const KTabHost& kt);
+// tileStats: {neighbour total, longest list} of each block of the list build, list_stats_per_tile(tiles) of them a tile
+uint32_t list_stats_per_tile(uint32_t tiles);
 void launch_build_lists(const Launch& L, const SceneGrid* G, const float4* pos, const uint32_t* cellStart,
                         const uint32_t* cellCount, uint32_t* nbrCount, uint32_t* nbrList,
                         uint2* tileStats);

@@ -460,7 +460,7 @@ public:
     DevBuf<uint32_t> id[2], nbrCount, nbrList, cellOf, rank, tmpId, surface, cellCount, cellStart, scanScratch, live;
     DevBuf<double> partials;
     DevBuf<float> partialsF;
-    DevBuf<uint2> tileStats;  // each tile's neighbour total and longest list
+    DevBuf<uint2> tileStats;  // neighbour total and longest list of the list build's blocks
     DevBuf<uint32_t> haloCount, haloIds, haloStats;
     DevBuf<uint32_t> nbrLocal;
 
@@ -1046,7 +1046,7 @@ public:
         VFD_TRY(nbrList.alloc(c * kMaxNeighbors));
         VFD_TRY(partials.alloc((size_t)std::max<uint32_t>(tiles, 1) * kPartialSlots));
         VFD_TRY(partialsF.alloc(std::max<uint32_t>(tiles, 1)));
-        VFD_TRY(tileStats.alloc(std::max<uint32_t>(tiles, 1)));
+        VFD_TRY(tileStats.alloc((size_t)std::max<uint32_t>(tiles, 1) * list_stats_per_tile(tiles)));
         {
             const Launch L = launch();
             const uint32_t rt = resident_group_tiles(L, numCU);
