@@ -685,42 +685,21 @@ __global__ void __launch_bounds__(kTile) k_adj_push(uint32_t n, uint32_t stride,
 // one BicgState, every kernel returns at once when `done` is set, and the host reads `done` only every few
 // iterations. Dots are FP64 per-block partials summed in a fixed order, scalar updates are in double and the vector
 // updates round the scalars to float.
-__global__ void __launch_bounds__(kTile) k_bicg_dot(uint32_t n, const float4* __restrict__ p,
-                                                    const float4* __restrict__ q, const float4* __restrict__ p2,
-                                                    const float4* __restrict__ q2, double* part,
-                                                    const BicgState* __restrict__ st) {
-    if (st->done) return;
-    const uint32_t i = pid();
-    double v[2] = {i < n ? (double)dot3(ld3(p[i]), ld3(q[i])) : 0.0,
-                   (p2 && i < n) ? (double)dot3(ld3(p2[i]), ld3(q2[i])) : 0.0};
-    block_sum<2>(v);
-    if (threadIdx.x == 0) {
-        part[blockIdx.x] = v[0];
-        part[gridDim.x + blockIdx.x] = v[1];
-    }
-}
-// the dots' block partials summed by the block in a fixed order (strided per thread, then block_sum's tree), then
-// the scalar update of stage `which`
-__global__ void __launch_bounds__(kTile) k_bicg_scalars(const double* __restrict__ part, uint32_t blocks,
-                                                        BicgState* st, int which) {
-    if (st->done) return;  // block-uniform
-    double v[2] = {0.0, 0.0};
-    for (uint32_t k = threadIdx.x; k < blocks; k += blockDim.x) {
-        v[0] += part[k];
-        if (which == kBicgTsTt || which == kBicgBegin) v[1] += part[blocks + k];
-    }
-    block_sum<2>(v);
-    if (threadIdx.x != 0) return;
-    const double a = v[0], b = v[1];
+//
+// Launches are what an iteration of a small system costs (4 to 6 us each, whatever they do): the residual's two dots are
+// taken where it is formed, and up to kBicgFinishBlocks blocks the last block of a dot to arrive sums the partials and
+// updates the scalars itself, 13 -> 7 launches an iteration. Arrivals at one counter take about 7 ns each, one after the
+// other, which from some 700 blocks on costs what the launch did: there the scalars keep a launch of their own (10).
+constexpr uint32_t kBicgFinishBlocks = 512;
+// the scalar update of stage `which` from the dots a and b
+__device__ __forceinline__ void bicg_scalars(BicgState* st, int which, double a, double b) {
     switch (which) {
-        case kBicgBegin:  // a = |b|^2, b = |r0|^2
+        case kBicgBegin:  // a = |b|^2, b = |r0|^2 (= rh.r0: the shadow residual is r0)
             st->rr = b;
             st->tol2 = 1e-12 * a;
             if (a == 0.0 || !(b > st->tol2)) st->done = 1u;
-            break;
-        case kBicgRho:
-            st->rhoNew = a;
-            st->beta = (a / st->rhoOld) * (st->alpha / st->omega);
+            st->rhoNew = b;
+            st->beta = (b / st->rhoOld) * (st->alpha / st->omega);
             break;
         case kBicgRv:
             st->alpha = st->rhoNew / a;
@@ -728,13 +707,68 @@ __global__ void __launch_bounds__(kTile) k_bicg_scalars(const double* __restrict
         case kBicgTsTt:
             st->omega = b > 0.0 ? a / b : 0.0;
             break;
-        default: {  // kBicgRr: end of an iteration
+        default: {  // kBicgEnd: end of an iteration, a = |r|^2; and the next one's rho, b = rh.r
             st->rr = a;
             st->rhoOld = st->rhoNew;
             st->it += 1;
-            if (st->omega == 0.0 || !(st->it < st->maxIt && a > st->tol2)) st->done = 1u;
+            if (st->omega == 0.0 || !(st->it < st->maxIt && a > st->tol2)) {
+                st->done = 1u;
+                return;
+            }
+            st->rhoNew = b;
+            st->beta = (b / st->rhoOld) * (st->alpha / st->omega);
         }
     }
+}
+// the dots' block partials summed by the block in a fixed order (strided per thread, then block_sum's tree), then
+// the scalar update of stage `which`; the partials were written by other blocks of this launch (kLive) or by an earlier one
+template <bool kLive>
+__device__ __forceinline__ void bicg_finish(const double* part, uint32_t blocks, BicgState* st, int which) {
+    double v[2] = {0.0, 0.0};
+    for (uint32_t k = threadIdx.x; k < blocks; k += blockDim.x)
+        for (int d = 0; d < 2; ++d)
+            v[d] += kLive ? __hip_atomic_load(part + d * blocks + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                          : part[d * blocks + k];
+    block_sum<2>(v);
+    if (threadIdx.x == 0) bicg_scalars(st, which, v[0], v[1]);
+}
+__global__ void __launch_bounds__(kTile) k_bicg_scalars(const double* __restrict__ part, uint32_t blocks,
+                                                        BicgState* st, int which) {
+    if (st->done) return;  // block-uniform
+    bicg_finish<false>(part, blocks, st, which);
+}
+// a block's partials of two dots; called by every thread of every block
+__device__ __forceinline__ void bicg_dots(double (&v)[2], double* part, BicgState* st, int which) {
+    const uint32_t blocks = gridDim.x;
+    block_sum<2>(v);
+    if (blocks > kBicgFinishBlocks) {
+        if (threadIdx.x == 0) {
+            part[blockIdx.x] = v[0];
+            part[blocks + blockIdx.x] = v[1];
+        }
+        return;
+    }
+    __shared__ uint32_t last;
+    if (threadIdx.x == 0) {
+        for (int d = 0; d < 2; ++d)
+            __hip_atomic_store(part + d * blocks + blockIdx.x, v[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the partials are out before the arrival counts
+        last = __hip_atomic_fetch_add(&st->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == blocks;
+    }
+    __syncthreads();
+    if (!last) return;  // block-uniform
+    if (threadIdx.x == 0) __hip_atomic_store(&st->arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    bicg_finish<true>(part, blocks, st, which);
+}
+__global__ void __launch_bounds__(kTile) k_bicg_dot(uint32_t n, const float4* __restrict__ p,
+                                                    const float4* __restrict__ q, const float4* __restrict__ p2,
+                                                    const float4* __restrict__ q2, double* part, BicgState* st,
+                                                    int which) {
+    if (st->done) return;
+    const uint32_t i = pid();
+    double v[2] = {i < n ? (double)dot3(ld3(p[i]), ld3(q[i])) : 0.0,
+                   (p2 && i < n) ? (double)dot3(ld3(p2[i]), ld3(q2[i])) : 0.0};
+    bicg_dots(v, part, st, which);
 }
 __global__ void k_bicg_reset(BicgState* st, uint32_t maxIt) {
     if (threadIdx.x == 0) *st = BicgState{1.0, 0.0, 1.0, 1.0, 0.0, 0.0, 0.0, 0u, maxIt, 0u, 0u};
@@ -762,17 +796,23 @@ __global__ void k_bicg_s(uint32_t n, const float4* __restrict__ r, const float4*
     const float na = (float)-st->alpha;
     if (i < n) s[i] = st4(ld3(r[i]) + na * ld3(v[i]));
 }
-// x += alpha p, then x += omega s; r = s - omega t
-__global__ void k_bicg_xr(uint32_t n, const float4* __restrict__ p, const float4* __restrict__ s,
-                          const float4* __restrict__ t, float4* x, float4* r, const BicgState* __restrict__ st) {
+// x += alpha p, then x += omega s; r = s - omega t; and the dots r.r and rh.r that end the iteration
+__global__ void __launch_bounds__(kTile) k_bicg_xr(uint32_t n, const float4* __restrict__ p, const float4* __restrict__ s,
+                                                   const float4* __restrict__ t, const float4* __restrict__ rh,
+                                                   float4* x, float4* r, double* part, BicgState* st) {
     if (st->done) return;
     const uint32_t i = pid();
     const float alpha = (float)st->alpha, omega = (float)st->omega, no = (float)-st->omega;
+    double v[2] = {0.0, 0.0};
     if (i < n) {
         const f3 si = ld3(s[i]);
         x[i] = st4((ld3(x[i]) + alpha * ld3(p[i])) + omega * si);
-        r[i] = st4(si + no * ld3(t[i]));
+        const f3 ri = si + no * ld3(t[i]);
+        r[i] = st4(ri);
+        v[0] = (double)dot3(ri, ri);
+        v[1] = (double)dot3(ld3(rh[i]), ri);
     }
+    bicg_dots(v, part, st, kBicgEnd);
 }
 
 // three copies in one launch (a recorded Jacobi iteration)
@@ -930,12 +970,21 @@ void adj_launch_push(hipStream_t s, uint32_t n, uint32_t stride, const float4* p
     if (n) hipLaunchKernelGGL(k_adj_push, grid_of(n), dim3(kTile), 0, s, n, stride, push, lx, lv);
 }
 
+// the scalars of stage `which` from the partials of a dot of n rows, where the dot's last block did not update them
+static void launch_bicg_scalars(hipStream_t s, uint32_t n, double* part, BicgState* st, int which) {
+    if (grid_of(n).x > kBicgFinishBlocks)
+        hipLaunchKernelGGL(k_bicg_scalars, dim3(1), dim3(kTile), 0, s, part, grid_of(n).x, st, which);
+}
+static void launch_bicg_dot(hipStream_t s, uint32_t n, const float4* p, const float4* q, const float4* p2,
+                            const float4* q2, double* part, BicgState* st, int which) {
+    hipLaunchKernelGGL(k_bicg_dot, grid_of(n), dim3(kTile), 0, s, n, p, q, p2, q2, part, st, which);
+    launch_bicg_scalars(s, n, part, st, which);
+}
 void adj_launch_bicg_begin(hipStream_t s, const AdjKHost& h, const float4* b, const float4* r, double* part,
                            BicgState* st, uint32_t maxIt) {
     const uint32_t n = h.n, o = h.base;
     hipLaunchKernelGGL(k_bicg_reset, dim3(1), dim3(kWave), 0, s, st, maxIt);
-    hipLaunchKernelGGL(k_bicg_dot, grid_of(n), dim3(kTile), 0, s, n, b + o, b + o, r + o, r + o, part, st);
-    hipLaunchKernelGGL(k_bicg_scalars, dim3(1), dim3(kTile), 0, s, part, grid_of(n).x, st, (int)kBicgBegin);
+    launch_bicg_dot(s, n, b + o, b + o, r + o, r + o, part, st, kBicgBegin);
 }
 void adj_launch_mu_acc(hipStream_t s, const double* part, uint32_t blocks, double* acc) {
     hipLaunchKernelGGL(k_adj_mu_acc, dim3(1), dim3(kTile), 0, s, part, blocks, acc);
@@ -945,20 +994,15 @@ void adj_launch_bicg_iteration(hipStream_t s, const AdjKHost& h, float dt, const
     // the vectors are slot-indexed arrays: the operator takes them whole, the pointwise kernels from the scene's
     // first slot
     const uint32_t n = h.n, b = h.base;
-    const uint32_t blocks = grid_of(n).x;
-    hipLaunchKernelGGL(k_bicg_dot, grid_of(n), dim3(kTile), 0, s, n, v.rh + b, v.r + b, nullptr, nullptr, part, st);
-    hipLaunchKernelGGL(k_bicg_scalars, dim3(1), dim3(kTile), 0, s, part, blocks, st, (int)kBicgRho);
     hipLaunchKernelGGL(k_bicg_p, grid_of(n), dim3(kTile), 0, s, n, v.r + b, v.v + b, v.p + b, st);
     adj_launch_visc_T(s, h, dt, rho, v.p, v.v, st);
-    hipLaunchKernelGGL(k_bicg_dot, grid_of(n), dim3(kTile), 0, s, n, v.rh + b, v.v + b, nullptr, nullptr, part, st);
-    hipLaunchKernelGGL(k_bicg_scalars, dim3(1), dim3(kTile), 0, s, part, blocks, st, (int)kBicgRv);
+    launch_bicg_dot(s, n, v.rh + b, v.v + b, nullptr, nullptr, part, st, kBicgRv);
     hipLaunchKernelGGL(k_bicg_s, grid_of(n), dim3(kTile), 0, s, n, v.r + b, v.v + b, v.s + b, st);
     adj_launch_visc_T(s, h, dt, rho, v.s, v.t, st);
-    hipLaunchKernelGGL(k_bicg_dot, grid_of(n), dim3(kTile), 0, s, n, v.t + b, v.s + b, v.t + b, v.t + b, part, st);
-    hipLaunchKernelGGL(k_bicg_scalars, dim3(1), dim3(kTile), 0, s, part, blocks, st, (int)kBicgTsTt);
-    hipLaunchKernelGGL(k_bicg_xr, grid_of(n), dim3(kTile), 0, s, n, v.p + b, v.s + b, v.t + b, v.x + b, v.r + b, st);
-    hipLaunchKernelGGL(k_bicg_dot, grid_of(n), dim3(kTile), 0, s, n, v.r + b, v.r + b, nullptr, nullptr, part, st);
-    hipLaunchKernelGGL(k_bicg_scalars, dim3(1), dim3(kTile), 0, s, part, blocks, st, (int)kBicgRr);
+    launch_bicg_dot(s, n, v.t + b, v.s + b, v.t + b, v.t + b, part, st, kBicgTsTt);
+    hipLaunchKernelGGL(k_bicg_xr, grid_of(n), dim3(kTile), 0, s, n, v.p + b, v.s + b, v.t + b, v.rh + b, v.x + b, v.r + b,
+                       part, st);
+    launch_bicg_scalars(s, n, part, st, kBicgEnd);
 }
 
 }  // namespace vfd

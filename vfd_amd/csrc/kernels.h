@@ -91,16 +91,17 @@ void adj_launch_fill(hipStream_t s, float* p, float v, uint32_t n);
 // scalars of a device-driven BiCGSTAB (adjoint viscosity solve); kernels given a state return at once once `done`
 struct BicgState {
     double rhoOld, rhoNew, alpha, omega, beta, rr, tol2;  // tol2: continue while rr > tol2
-    uint32_t it, maxIt, done, pad;
+    uint32_t it, maxIt, done, arrived;  // arrived: blocks of the current dot that have stored their partials
 };
-enum { kBicgRho = 0, kBicgRv = 1, kBicgTsTt = 2, kBicgRr = 3, kBicgBegin = 4 };
+enum { kBicgRv = 0, kBicgTsTt = 1, kBicgEnd = 2, kBicgBegin = 3 };
 struct BicgVectors {
     float4 *x, *r, *rh, *p, *v, *s, *t;
 };
 void adj_launch_visc_T(hipStream_t s, const AdjKHost& h, float dt, const float* rho, const float4* w, float4* out,
                        const BicgState* st = nullptr);
 // the solve's start on the device: state reset, |b|^2 and |r0|^2, the stopping threshold 1e-12 |b|^2, and done
-// when b = 0 or r0 already meets it (b, r0 slot-indexed; part holds 2 * ceil(n / kTile) doubles)
+// when b = 0 or r0 already meets it (b, r0 slot-indexed; the shadow residual is r0; part holds 2 * ceil(n / kTile)
+// doubles)
 void adj_launch_bicg_begin(hipStream_t s, const AdjKHost& h, const float4* b, const float4* r, double* part,
                            BicgState* st, uint32_t maxIt);
 // acc[0] += the sum of part[0, blocks) (per-block d/dmu partials of one step), in a fixed order
