@@ -29,7 +29,7 @@ struct AdjK {
     uint32_t n, cap;                    // particles of the scene being reversed, list capacity
     uint32_t base, stride;              // the scene's first slot; slots per record of the step (contact records)
     const uint32_t* __restrict__ count;
-    const uint32_t* __restrict__ list;  // [j * cap + i]
+    const uint32_t* __restrict__ list;  // particle slots (list_at)
     const float4* __restrict__ x;
     const float4* __restrict__ con;  // contact records [(kContactRecs b + q) stride + i] (k_adj_boundary_tape)
     uint32_t bodies;                 // 0: no contact records
@@ -334,7 +334,7 @@ __global__ void __launch_bounds__(kTile) k_adj_div_T(AdjK a, const float* __rest
 struct AdjStage {
     TileGrid tg;
     HaloView H;
-    const uint32_t* __restrict__ local;  // [j * cap + i] halo slot | table code << 16
+    const uint32_t* __restrict__ local;  // halo slot | table code << 16 (local_at)
 };
 constexpr size_t kLdsAdjStage = kLdsG + HaloRec<LoadXSV>::kBytes;
 template <class Make, class Fin>
