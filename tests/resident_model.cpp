@@ -1,0 +1,241 @@
+// The blocks of a resident solve (vfd_amd/csrc/resident.h) as threads of a host program: a thread per wave, the barrier
+// words in one lock-protected array. argv[1] names a scenario; the program prints "ok" or what was wrong.
+#include <atomic>
+#include <chrono>
+#include <condition_variable>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "resident.h"
+
+using namespace vfd;
+
+static std::mutex mu;
+static uint32_t words[kResidentWords];
+static std::atomic<long long> now{0};
+
+[[noreturn]] static void wrong(const char* what) {
+    std::printf("wrong: %s\n", what);
+    std::fflush(stdout);
+    std::_Exit(1);
+}
+
+// A block: the waves still in the launch, their barrier, and the value its leader hands to all (at first what the
+// memory happens to hold).
+struct Block {
+    std::mutex m;
+    std::condition_variable cv;
+    uint32_t waves = 0, waiting = 0, generation = 0, shared = 0xDEADBEEFu;
+    void meet() {
+        std::unique_lock<std::mutex> lk(m);
+        const uint32_t g = generation;
+        if (++waiting == waves) {
+            next();
+            return;
+        }
+        if (!cv.wait_for(lk, std::chrono::seconds(30), [&] { return generation != g; })) wrong("a wave never left");
+    }
+    void next() {
+        waiting = 0;
+        ++generation;
+        cv.notify_all();
+    }
+    void wave_ends() {  // as on the device, a wave that has ended is not waited for
+        std::lock_guard<std::mutex> lk(m);
+        --waves;
+        if (waves && waiting == waves) next();
+    }
+};
+
+struct Wave {
+    Block* block = nullptr;
+    uint32_t wave = 0;
+    std::function<void()> afterMark;  // called between a read of the abort mark and its use
+};
+static thread_local Wave self;
+
+struct Ops {
+    static uint32_t load(const uint32_t* p) {
+        uint32_t v;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            v = *p;
+        }
+        if (p == words + kResidentAbortedAt && self.afterMark) self.afterMark();
+        std::this_thread::yield();
+        return v;
+    }
+    static void store(uint32_t* p, uint32_t v) {
+        std::lock_guard<std::mutex> lk(mu);
+        *p = v;
+    }
+    static uint32_t add(uint32_t* p, uint32_t v) {
+        std::lock_guard<std::mutex> lk(mu);
+        return *p += v;
+    }
+    static bool swap(uint32_t* p, uint32_t& seen, uint32_t v) {
+        std::lock_guard<std::mutex> lk(mu);
+        if (*p != seen) {
+            seen = *p;
+            return false;
+        }
+        *p = v;
+        return true;
+    }
+    static long long ticks() { return ++now; }
+    static bool leader() { return self.wave == 0; }
+    static void settle() {}
+    static void meet() { self.block->meet(); }
+    template <class Fn> static uint32_t one(Fn&& f) {
+        if (leader()) self.block->shared = f();
+        meet();
+        return self.block->shared;
+    }
+};
+
+static GridSync grid_of(uint32_t block, uint32_t blocks, uint32_t limit) {  // as resident_group lays the blocks out
+    const uint32_t per = (blocks + 7) / 8, chunk = block / per;
+    return GridSync{words, blocks, chunk, std::min(per, blocks - chunk * per), (blocks + per - 1) / per, 0u, limit};
+}
+
+struct Outcome {
+    bool open = false;
+    uint32_t passed = 0;
+};
+// a wave of a solve with `barriers` barriers; `arrived` counts the blocks that have come to each
+static void solve(GridSync g, uint32_t barriers, std::atomic<uint32_t>* arrived, Outcome& out) {
+    out.open = solve_open<Ops>(words);
+    if (!out.open) return;
+    for (uint32_t k = 0; k < barriers; ++k) {
+        if (arrived && Ops::leader()) ++arrived[k];
+        if (!grid_sync<Ops>(g)) {
+            grid_leave<Ops>(g, true);
+            return;
+        }
+        if (arrived && arrived[k] != g.blocks) wrong("a barrier was passed before every block had come to it");
+        ++out.passed;
+    }
+    grid_leave<Ops>(g, false);
+}
+
+static void run(Block& b, uint32_t waves, std::vector<std::thread>& threads, const std::function<void(uint32_t)>& body) {
+    b.waves = waves;
+    for (uint32_t w = 0; w < waves; ++w)
+        threads.emplace_back([&b, w, body] {
+            self = Wave{&b, w, nullptr};
+            body(w);
+            b.wave_ends();
+        });
+}
+static void join(std::vector<std::thread>& threads) {
+    for (auto& t : threads) t.join();
+    threads.clear();
+}
+
+// Every block there: all barriers are passed, and the words are zero again.
+static void all_pass(uint32_t blocks) {
+    constexpr uint32_t kBarriers = 4, kWaves = 2;
+    std::vector<Block> b(blocks);
+    std::vector<Outcome> out(blocks * kWaves);
+    std::vector<std::thread> threads;
+    std::atomic<uint32_t> arrived[kBarriers] = {};
+    for (uint32_t k = 0; k < blocks; ++k)
+        run(b[k], kWaves, threads, [&, k](uint32_t w) {
+            solve(grid_of(k, blocks, 0xFFFFFFFFu), kBarriers, arrived, out[k * kWaves + w]);
+        });
+    join(threads);
+    for (const Outcome& o : out)
+        if (!o.open || o.passed != kBarriers) wrong("a block did not pass every barrier");
+    for (uint32_t w : words)
+        if (w) wrong("a word was left behind");
+}
+// No time to wait: blocks give up at barriers that are still open; every wave leaves.
+static void no_time(uint32_t blocks) {
+    constexpr uint32_t kBarriers = 3, kWaves = 2;
+    std::vector<Block> b(blocks);
+    std::vector<Outcome> out(blocks * kWaves);
+    std::vector<std::thread> threads;
+    std::atomic<uint32_t> arrived[kBarriers] = {};
+    for (uint32_t k = 0; k < blocks; ++k)
+        run(b[k], kWaves, threads, [&, k](uint32_t w) {
+            solve(grid_of(k, blocks, 0u), kBarriers, arrived, out[k * kWaves + w]);
+        });
+    join(threads);
+    uint32_t all = 0;
+    for (uint32_t k = 0; k < blocks; ++k) {
+        if (out[2 * k].open != out[2 * k + 1].open || out[2 * k].passed != out[2 * k + 1].passed)
+            wrong("waves of a block went different ways");
+        all += out[2 * k].passed == kBarriers;
+    }
+    if (all && all != blocks) wrong("some blocks passed the last barrier and some did not");
+    if ((all == 0) != (words[kResidentAbortedAt] != 0)) wrong("the mark and the outcome differ");
+}
+// The last block starts when the others have given up: its first look at the mark falls before they set it, every later
+// one after.
+static void late(uint32_t blocks) {
+    constexpr uint32_t kWaves = 4;
+    std::vector<Block> b(blocks);
+    std::vector<Outcome> out(blocks * kWaves);
+    std::vector<std::thread> punctual, last;
+    std::mutex m;
+    std::condition_variable cv;
+    int looks = 0;
+    bool others = false;
+    const uint32_t k = blocks - 1;
+    run(b[k], kWaves, last, [&](uint32_t w) {
+        self.afterMark = [&] {
+            std::unique_lock<std::mutex> lk(m);
+            if (looks++ == 0) {
+                cv.notify_all();
+                cv.wait(lk, [&] { return others; });
+            }
+        };
+        if (w != 0) {  // another wave looks after wave 0 at the earliest (if it looks at all)
+            std::unique_lock<std::mutex> lk(m);
+            cv.wait(lk, [&] { return looks > 0; });
+        }
+        if (w > 1) {
+            std::unique_lock<std::mutex> lk(m);
+            cv.wait(lk, [&] { return others; });
+        }
+        solve(grid_of(k, blocks, 2000u), 2, nullptr, out[k * kWaves + w]);
+    });
+    {
+        std::unique_lock<std::mutex> lk(m);
+        cv.wait(lk, [&] { return looks > 0; });
+    }
+    for (uint32_t q = 0; q < k; ++q)
+        run(b[q], 1, punctual, [&, q](uint32_t) { solve(grid_of(q, blocks, 2000u), 2, nullptr, out[q * kWaves]); });
+    join(punctual);
+    {
+        std::lock_guard<std::mutex> lk(m);
+        others = true;
+    }
+    cv.notify_all();
+    join(last);
+    if (!words[kResidentAbortedAt]) wrong("the solve was not marked as aborted");
+    for (uint32_t w = 0; w < kWaves; ++w) {
+        if (out[k * kWaves + w].open != out[k * kWaves].open) wrong("waves of a block went different ways");
+        if (out[k * kWaves + w].passed) wrong("a barrier was passed that nobody had completed");
+    }
+}
+
+int main(int argc, char** argv) {
+    const char* what = argc > 1 ? argv[1] : "";
+    const uint32_t blocks = argc > 2 ? (uint32_t)std::atoi(argv[2]) : 1u;
+    if (!std::strcmp(what, "all_pass"))
+        all_pass(blocks);
+    else if (!std::strcmp(what, "no_time"))
+        no_time(blocks);
+    else if (!std::strcmp(what, "late"))
+        late(blocks);
+    else
+        wrong("unknown scenario");
+    std::printf("ok\n");
+    return 0;
+}

@@ -1,0 +1,35 @@
+"""The meeting of a resident solve's blocks (vfd_amd/csrc/resident.h), run on the host with a thread for each wave."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "vfd_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def model(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("resident") / "model")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-pthread", "-I", CSRC,
+                           os.path.join(HERE, "resident_model.cpp"), "-o", exe])
+
+    def run(*args):
+        p = subprocess.run([exe] + [str(a) for a in args], stdout=subprocess.PIPE, text=True, timeout=100)
+        assert p.stdout.strip() == "ok", p.stdout
+    return run
+
+
+@pytest.mark.parametrize("blocks", [1, 2, 64, 65, 100])  # one polled word up to 64 blocks, a word per chunk beyond
+def test_every_block_passes_every_barrier(model, blocks):
+    model("all_pass", blocks)
+
+
+@pytest.mark.parametrize("blocks", [2, 64, 65, 100])
+def test_blocks_that_may_not_wait_all_leave(model, blocks):
+    model("no_time", blocks)
+
+
+@pytest.mark.parametrize("blocks", [3, 70])
+def test_a_block_that_starts_after_the_others_gave_up_leaves_as_a_whole(model, blocks):
+    model("late", blocks)

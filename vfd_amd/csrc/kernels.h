@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "common.h"
+#include "resident.h"
 
 namespace vfd {
 
@@ -321,9 +322,6 @@ void launch_pres_iter(const Launch& L, const KTabHost& kt, const Fields& F);
 void launch_pres_final(const Launch& L, const KTabHost& kt, const Fields& F, int writeNext, const uint32_t* aborted);
 // ---- solve.hip: whole solves as one launch ----------------------------------------------------------------------
 constexpr uint32_t kResidentScenes = 256;        // scenes of a resident solve (their scalars live in LDS)
-// Barrier words (32-bit), zero between launches; words[kResidentAbortedAt] is set when a solve was aborted, and then
-// the host clears all of them.
-constexpr uint32_t kResidentWords = 1024, kResidentAbortedAt = 18 * 32;
 struct Resident {
     uint32_t* words;
     uint32_t waitTicks;  // longest wait at a barrier, in ticks of the 100 MHz wall clock

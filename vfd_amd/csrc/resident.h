@@ -1,0 +1,116 @@
+// resident.h - how the blocks of a resident solve (solve.hip) enter it, meet and leave it: the bounded grid barrier,
+// written over the few operations that a block needs (Ops below), so that the same code runs on the device and, with
+// threads for waves, in a program on the host.
+//
+// Ops:  load(p), store(p, v), add(p, v) (the new value), swap(p, seen, v) (compare-and-exchange, seen = what was there):
+//       relaxed atomics that every block sees; ticks(): a clock, the same for all blocks; one(f): called by every thread
+//       of the block, f() by one of them, its value to all; leader(): true in one thread of the block; settle(): waits
+//       for the calling thread's own stores; meet(): the block's barrier.
+#pragma once
+
+#include <cstdint>
+
+#ifdef __HIPCC__
+#define VFD_RESIDENT __device__ __forceinline__
+#else
+#define VFD_RESIDENT inline
+#endif
+
+namespace vfd {
+
+// Barrier words (32-bit), zero between launches; words[kResidentAbortedAt] is set when a solve was aborted, and then
+// the host clears all of them.
+constexpr uint32_t kResidentWords = 1024, kResidentAbortedAt = 18 * 32;
+// A 128-byte line each: arrivals (2 per block or chunk, bit 0 = aborted), arrivals per XCD chunk, release words, blocks
+// that have left.
+constexpr uint32_t kLine = 32;
+constexpr uint32_t kWordArrive = 0, kWordChunk = kLine, kWordRelease = 9 * kLine, kWordLeft = 17 * kLine;
+static_assert(kWordLeft + kLine <= kResidentAbortedAt && kResidentAbortedAt < kResidentWords, "barrier words");
+constexpr uint32_t kAbortBit = 1u, kReleaseAbort = 0xFFFFFFFFu;
+// Up to this many blocks poll the arrival word itself (1.5 us at 8 blocks, 2.1 at 64); more arrive through their XCD
+// chunk's word and poll a release word per chunk (2.5 us at 121 blocks, 2.9 at 248, where one polled word takes 5.8).
+constexpr uint32_t kFlatBlocks = 64;
+
+struct GridSync {
+    uint32_t* w;
+    uint32_t blocks, chunk, chunkBlocks, chunks, epoch;
+    uint32_t waitTicks;  // of the 100 MHz wall clock
+};
+
+// Whether no solve of this step has been aborted, the same answer in every thread of the block: the mark is read once,
+// since blocks of this very launch may set it (a block that starts after the others' limit), and a block of which only
+// some waves went on would pass barriers that nobody has completed.
+template <class Ops> VFD_RESIDENT bool solve_open(const uint32_t* words) {
+    return Ops::one([&] { return Ops::load(words + kResidentAbortedAt); }) == 0u;
+}
+template <class Ops> VFD_RESIDENT void release_chunks(const GridSync& g, uint32_t v) {
+    for (uint32_t c = 0; c < g.chunks; ++c) Ops::store(g.w + kWordRelease + kLine * c, v);
+}
+// the wait of one thread; target = arrivals (times 2) that complete the barrier
+template <class Ops> VFD_RESIDENT bool sync_thread(const GridSync& g) {
+    const long long t0 = Ops::ticks();
+    uint32_t* arrive = g.w + kWordArrive;
+    if (g.blocks <= kFlatBlocks) {
+        const uint32_t target = 2u * g.blocks * g.epoch;
+        uint32_t v = Ops::add(arrive, 2u);
+        while (!(v & kAbortBit) && v < target) {
+            if ((uint64_t)(Ops::ticks() - t0) > g.waitTicks) {  // only a barrier that is still open can be aborted
+                uint32_t seen = v;
+                if (Ops::swap(arrive, seen, v | kAbortBit)) return false;
+                v = seen;
+            } else {
+                v = Ops::load(arrive);
+            }
+        }
+        return !(v & kAbortBit);
+    }
+    const uint32_t target = 2u * g.chunks * g.epoch;
+    uint32_t* mine = g.w + kWordRelease + kLine * g.chunk;
+    if (Ops::add(g.w + kWordChunk + kLine * g.chunk, 1u) == g.chunkBlocks * g.epoch) {
+        const uint32_t v = Ops::add(arrive, 2u);
+        if (v & kAbortBit) {
+            release_chunks<Ops>(g, kReleaseAbort);
+            return false;
+        }
+        if (v == target) {
+            release_chunks<Ops>(g, g.epoch);
+            return true;
+        }
+    }
+    for (;;) {
+        const uint32_t r = Ops::load(mine);
+        if (r == kReleaseAbort) return false;
+        if (r >= g.epoch) return true;
+        if ((uint64_t)(Ops::ticks() - t0) > g.waitTicks) {
+            uint32_t v = Ops::load(arrive);
+            if (v & kAbortBit) return false;
+            if (v >= target) continue;  // complete: its release is being written
+            if (Ops::swap(arrive, v, v | kAbortBit)) {
+                release_chunks<Ops>(g, kReleaseAbort);
+                return false;
+            }
+        }
+    }
+}
+// Barrier over the launch's blocks, called by every thread; false: the solve is aborted (the same answer in every
+// block). Every wave waits for its own stores before its block arrives.
+template <class Ops> VFD_RESIDENT bool grid_sync(GridSync& g) {
+    Ops::settle();
+    Ops::meet();
+    g.epoch += 1;
+    return Ops::one([&] { return sync_thread<Ops>(g) ? 1u : 0u; }) != 0u;
+}
+// The last block to leave clears the words for the next launch; an aborted solve leaves its mark.
+template <class Ops> VFD_RESIDENT void grid_leave(const GridSync& g, bool aborted) {
+    if (!Ops::leader()) return;
+    if (aborted) Ops::store(g.w + kResidentAbortedAt, 1u);
+    if (Ops::add(g.w + kWordLeft, 1u) != g.blocks) return;
+    Ops::store(g.w + kWordArrive, 0u);
+    for (uint32_t c = 0; c < 8; ++c) {
+        Ops::store(g.w + kWordChunk + kLine * c, 0u);
+        Ops::store(g.w + kWordRelease + kLine * c, 0u);
+    }
+    Ops::store(g.w + kWordLeft, 0u);
+}
+
+}  // namespace vfd

@@ -17,10 +17,11 @@
 // take no stale copy from an XCD's L2; everything else is read-only during the solve or private to its thread. A
 // value is overwritten only after a barrier that follows its last read.
 //
-// Barriers are bounded. A block that waits longer than waitTicks - other work holds CUs that this launch needs - sets
-// the abort bit in the arrival word, atomically with the arrivals, so that either every block passes a barrier or none
-// does; an aborted solve writes neither velocities nor positions, every later resident solve of the step returns at
-// once, and the host takes the step again with launched iterations. Every wave leaves every launch.
+// Barriers (resident.h) are bounded. A block that waits longer than waitTicks - other work holds CUs that this launch
+// needs - sets the abort bit in the arrival word, atomically with the arrivals and only while the barrier is open, so that
+// either every block passes the solve's last barrier or none does; an aborted solve writes neither velocities nor
+// positions, every later resident solve of the step returns at once, and the host takes the step again with launched
+// iterations. Whether to return is decided by a block as a whole, so every wave leaves every launch.
 //
 // Results are the launched kernels' bits: the same sums in the same list order (terms.h), the same per-tile and
 // per-scene FP64 trees, the same loop conditions.
@@ -59,106 +60,32 @@ __device__ __forceinline__ f3 get_agent(const float4* p) {
     return mk3(__uint_as_float((uint32_t)a), __uint_as_float((uint32_t)(a >> 32)), __uint_as_float((uint32_t)b));
 }
 
-// ---- bounded grid barrier -----------------------------------------------------------------------------------------
-// Words of a solve's barrier (all zero between launches; kResidentWords in kernels.h), a 128-byte line each: arrivals
-// (2 per block or chunk, bit 0 = aborted), arrivals per XCD chunk, release words, blocks that have left.
-constexpr uint32_t kLine = 32;
-constexpr uint32_t kWordArrive = 0, kWordChunk = kLine, kWordRelease = 9 * kLine, kWordLeft = 17 * kLine;
-static_assert(kWordLeft + kLine <= kResidentAbortedAt && kResidentAbortedAt < kResidentWords, "barrier words");
-constexpr uint32_t kAbortBit = 1u, kReleaseAbort = 0xFFFFFFFFu;
-// Up to this many blocks poll the arrival word itself (1.5 us at 8 blocks, 2.1 at 64); more arrive through their XCD
-// chunk's word and poll a release word per chunk (2.5 us at 121 blocks, 2.9 at 248, where one polled word takes 5.8).
-constexpr uint32_t kFlatBlocks = 64;
-
-struct GridSync {
-    uint32_t* w;
-    uint32_t blocks, chunk, chunkBlocks, chunks, epoch;
-    uint32_t waitTicks;  // of the 100 MHz wall clock
+// ---- the blocks' meeting (resident.h) on the device -----------------------------------------------------------------
+struct DeviceOps {
+    static __device__ __forceinline__ uint32_t load(const uint32_t* p) {
+        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    static __device__ __forceinline__ void store(uint32_t* p, uint32_t v) {
+        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    static __device__ __forceinline__ uint32_t add(uint32_t* p, uint32_t v) {
+        return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + v;
+    }
+    static __device__ __forceinline__ bool swap(uint32_t* p, uint32_t& seen, uint32_t v) {
+        return __hip_atomic_compare_exchange_strong(p, &seen, v, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT);
+    }
+    static __device__ __forceinline__ long long ticks() { return wall_clock64(); }
+    static __device__ __forceinline__ bool leader() { return threadIdx.x == 0; }
+    static __device__ __forceinline__ void settle() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+    static __device__ __forceinline__ void meet() { __syncthreads(); }
+    template <class Fn> static __device__ __forceinline__ uint32_t one(Fn&& f) {
+        __shared__ uint32_t v;
+        if (threadIdx.x == 0) v = f();
+        __syncthreads();
+        return v;
+    }
 };
-__device__ __forceinline__ uint32_t word(const uint32_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void set_word(uint32_t* p, uint32_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ uint32_t add_word(uint32_t* p, uint32_t v) {
-    return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + v;
-}
-__device__ __forceinline__ void release_chunks(const GridSync& g, uint32_t v) {
-    for (uint32_t c = 0; c < g.chunks; ++c) set_word(g.w + kWordRelease + kLine * c, v);
-}
-// the wait of one thread; target = arrivals (times 2) that complete the barrier
-__device__ __forceinline__ bool sync_thread(const GridSync& g) {
-    const long long t0 = wall_clock64();
-    uint32_t* arrive = g.w + kWordArrive;
-    if (g.blocks <= kFlatBlocks) {
-        const uint32_t target = 2u * g.blocks * g.epoch;
-        uint32_t v = add_word(arrive, 2u);
-        while (!(v & kAbortBit) && v < target) {
-            if ((uint64_t)(wall_clock64() - t0) > g.waitTicks) {  // only a barrier that is still open can be aborted
-                uint32_t seen = v;
-                if (__hip_atomic_compare_exchange_strong(arrive, &seen, v | kAbortBit, __ATOMIC_RELAXED,
-                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                    return false;
-                v = seen;
-            } else {
-                v = word(arrive);
-            }
-        }
-        return !(v & kAbortBit);
-    }
-    const uint32_t target = 2u * g.chunks * g.epoch;
-    uint32_t* mine = g.w + kWordRelease + kLine * g.chunk;
-    if (add_word(g.w + kWordChunk + kLine * g.chunk, 1u) == g.chunkBlocks * g.epoch) {
-        const uint32_t v = add_word(arrive, 2u);
-        if (v & kAbortBit) {
-            release_chunks(g, kReleaseAbort);
-            return false;
-        }
-        if (v == target) {
-            release_chunks(g, g.epoch);
-            return true;
-        }
-    }
-    for (;;) {
-        const uint32_t r = word(mine);
-        if (r == kReleaseAbort) return false;
-        if (r >= g.epoch) return true;
-        if ((uint64_t)(wall_clock64() - t0) > g.waitTicks) {
-            uint32_t v = word(arrive);
-            if (v & kAbortBit) return false;
-            if (v >= target) continue;  // complete: its release is being written
-            if (__hip_atomic_compare_exchange_strong(arrive, &v, v | kAbortBit, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT)) {
-                release_chunks(g, kReleaseAbort);
-                return false;
-            }
-        }
-    }
-}
-// Barrier over the launch's blocks, called by every thread; false: the solve is aborted (the same answer in every
-// block). Every wave waits for its own stores before its block arrives.
-__device__ __forceinline__ bool grid_sync(GridSync& g) {
-    __shared__ uint32_t pass;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    g.epoch += 1;
-    if (threadIdx.x == 0) pass = sync_thread(g) ? 1u : 0u;
-    __syncthreads();
-    return pass != 0u;
-}
-// The last block to leave clears the words for the next launch; an aborted solve leaves its mark.
-__device__ __forceinline__ void grid_leave(const GridSync& g, bool aborted) {
-    if (threadIdx.x != 0) return;
-    if (aborted) set_word(g.w + kResidentAbortedAt, 1u);
-    if (add_word(g.w + kWordLeft, 1u) != g.blocks) return;
-    set_word(g.w + kWordArrive, 0u);
-    for (uint32_t c = 0; c < 8; ++c) {
-        set_word(g.w + kWordChunk + kLine * c, 0u);
-        set_word(g.w + kWordRelease + kLine * c, 0u);
-    }
-    set_word(g.w + kWordLeft, 0u);
-}
 
 // ---- one block's group ----------------------------------------------------------------------------------------------
 // Loaders of groups whose halo is not staged: exchanged values are gathered at agent scope. The staged list is read
@@ -628,8 +555,8 @@ __device__ __forceinline__ void jacobi_solve(const SceneParams* __restrict__ P, 
     uint32_t iterations = 0;
     f3 a = mk3(0.0f, 0.0f, 0.0f);
     for (;;) {
-        if (!grid_sync(r.gs)) {
-            grid_leave(r.gs, true);
+        if (!grid_sync<DeviceOps>(r.gs)) {
+            grid_leave<DeviceOps>(r.gs, true);
             return;
         }
         if (iterations)
@@ -653,8 +580,8 @@ __device__ __forceinline__ void jacobi_solve(const SceneParams* __restrict__ P, 
         if (on && (act || !live)) a = sums.accel(k, kap);
         if (!live) break;  // the accelerations of the final kappa
         if (on && act) put_agent(F.ap + c.i, a);
-        if (!grid_sync(r.gs)) {
-            grid_leave(r.gs, true);
+        if (!grid_sync<DeviceOps>(r.gs)) {
+            grid_leave<DeviceOps>(r.gs, true);
             return;
         }
         sums.fill_accel();
@@ -693,7 +620,7 @@ __device__ __forceinline__ void jacobi_solve(const SceneParams* __restrict__ P, 
         }
         if (!kPressure) F.acc[c.i] = make_float4(p.gx, p.gy, p.gz, 0.0f);
     }
-    grid_leave(r.gs, false);
+    grid_leave<DeviceOps>(r.gs, false);
 }
 template <unsigned kTiles, bool kPressure>
 __global__ void __launch_bounds__(kTiles * kTile, 1) k_jacobi_solve(const SceneParams* __restrict__ P,
@@ -704,7 +631,7 @@ __global__ void __launch_bounds__(kTiles * kTile, 1) k_jacobi_solve(const SceneP
     if (!kPressure) note_time(stamps, kStampDivergence);
     extern __shared__ float4 lds[];
     __shared__ SceneCtl ctl[kResidentScenes];
-    if (words[kResidentAbortedAt]) return;  // an earlier solve of this step was aborted
+    if (!solve_open<DeviceOps>(words)) return;
     Group<kTiles> r;
     if (!resident_group(r, P, tileScene, F, cap, tg, words, waitTicks, reinterpret_cast<float*>(lds))) return;
     if (kTiles < 4 && r.src.rec) {  // block-uniform
@@ -737,7 +664,7 @@ __global__ void __launch_bounds__(kTiles * kTile, 1) k_visc_solve(const ScenePar
                                                                          long long* stamps) {
     note_time(stamps, kStampViscosity);
     __shared__ SceneCtl ctl[kResidentScenes];
-    if (words[kResidentAbortedAt]) return;  // an earlier solve of this step was aborted
+    if (!solve_open<DeviceOps>(words)) return;
     VFD_HALO_KERNEL_PROLOGUE(kh)
     constexpr uint32_t kThreads = kTiles * kTile;
     Group<kTiles> r;
@@ -783,8 +710,8 @@ __global__ void __launch_bounds__(kTiles * kTile, 1) k_visc_solve(const ScenePar
         v3[2] = (double)dot3(res, z);
     }
     exchange_partials<kTiles, 3>(v3, F.partials, r.tile, 0, r.tile < tg.tiles && p.enableVisc);
-    if (!grid_sync(r.gs)) {
-        grid_leave(r.gs, true);
+    if (!grid_sync<DeviceOps>(r.gs)) {
+        grid_leave<DeviceOps>(r.gs, true);
         return;
     }
     // k_cg_begin_finish
@@ -835,8 +762,8 @@ __global__ void __launch_bounds__(kTiles * kTile, 1) k_visc_solve(const ScenePar
         if (act && !firstIteration) dir = dir * ctl[c.s].beta + z;
         if (gathered) {
             if (act) put_agent(F.cgP + c.i, dir);
-            if (!grid_sync(r.gs)) {
-                grid_leave(r.gs, true);
+            if (!grid_sync<DeviceOps>(r.gs)) {
+                grid_leave<DeviceOps>(r.gs, true);
                 return;
             }
         } else {
@@ -850,8 +777,8 @@ __global__ void __launch_bounds__(kTiles * kTile, 1) k_visc_solve(const ScenePar
             v1[0] = (double)dot3(dir, ap);
         }
         exchange_partials<kTiles, 1>(v1, F.partials, r.tile, 3, act || (r.tile < tg.tiles && ctl[c.s].active));
-        if (!grid_sync(r.gs)) {
-            grid_leave(r.gs, true);
+        if (!grid_sync<DeviceOps>(r.gs)) {
+            grid_leave<DeviceOps>(r.gs, true);
             return;
         }
         // k_cg_alpha
@@ -870,8 +797,8 @@ __global__ void __launch_bounds__(kTiles * kTile, 1) k_visc_solve(const ScenePar
             v2[1] = (double)dot3(res, z);
         }
         exchange_partials<kTiles, 2>(v2, F.partials, r.tile, 0, r.tile < tg.tiles && ctl[c.s].active);
-        if (!grid_sync(r.gs)) {
-            grid_leave(r.gs, true);
+        if (!grid_sync<DeviceOps>(r.gs)) {
+            grid_leave<DeviceOps>(r.gs, true);
             return;
         }
         // k_cg_update_finish
@@ -912,7 +839,7 @@ __global__ void __launch_bounds__(kTiles * kTile, 1) k_visc_solve(const ScenePar
         F.acc[c.i] = st4(ld3(F.acc[c.i]) + (1.0f / dt) * d);
         F.dv[c.i] = st4(d);
     }
-    grid_leave(r.gs, false);
+    grid_leave<DeviceOps>(r.gs, false);
 }
 
 // ---- host side ----------------------------------------------------------------------------------------------------
