@@ -55,9 +55,19 @@ struct Block {
 struct Wave {
     Block* block = nullptr;
     uint32_t wave = 0;
-    std::function<void()> afterMark;  // called between a read of the abort mark and its use
+    std::function<void()> afterMark;             // called between a read of the abort mark and its use
+    std::function<void()> beforeLeave;           // called before the block leaves
+    uint32_t* slow = nullptr;                    // a word to which this wave's stores take their time, as long as it
+    std::vector<uint32_t> underway;              // does not wait for them
+    void land();
 };
 static thread_local Wave self;
+
+void Wave::land() {
+    std::lock_guard<std::mutex> lk(mu);
+    if (!underway.empty()) *slow = underway.back();
+    underway.clear();
+}
 
 struct Ops {
     static uint32_t load(const uint32_t* p) {
@@ -71,6 +81,10 @@ struct Ops {
         return v;
     }
     static void store(uint32_t* p, uint32_t v) {
+        if (p == self.slow) {
+            self.underway.push_back(v);
+            return;
+        }
         std::lock_guard<std::mutex> lk(mu);
         *p = v;
     }
@@ -89,7 +103,7 @@ struct Ops {
     }
     static long long ticks() { return ++now; }
     static bool leader() { return self.wave == 0; }
-    static void settle() {}
+    static void settle() { self.land(); }
     static void meet() { self.block->meet(); }
     template <class Fn> static uint32_t one(Fn&& f) {
         if (leader()) self.block->shared = f();
@@ -99,7 +113,7 @@ struct Ops {
 };
 
 static GridSync grid_of(uint32_t block, uint32_t blocks, uint32_t limit) {  // as resident_group lays the blocks out
-    const uint32_t per = (blocks + 7) / 8, chunk = block / per;
+    const uint32_t per = ((blocks + 7) / 8 + 3) / 4 * 4, chunk = block / per;
     return GridSync{words, blocks, chunk, std::min(per, blocks - chunk * per), (blocks + per - 1) / per, 0u, limit};
 }
 
@@ -120,6 +134,7 @@ static void solve(GridSync g, uint32_t barriers, std::atomic<uint32_t>* arrived,
         if (arrived && arrived[k] != g.blocks) wrong("a barrier was passed before every block had come to it");
         ++out.passed;
     }
+    if (self.beforeLeave) self.beforeLeave();
     grid_leave<Ops>(g, false);
 }
 
@@ -127,8 +142,10 @@ static void run(Block& b, uint32_t waves, std::vector<std::thread>& threads, con
     b.waves = waves;
     for (uint32_t w = 0; w < waves; ++w)
         threads.emplace_back([&b, w, body] {
-            self = Wave{&b, w, nullptr};
+            self.block = &b;
+            self.wave = w;
             body(w);
+            self.land();
             b.wave_ends();
         });
 }
@@ -225,6 +242,36 @@ static void late(uint32_t blocks) {
     }
 }
 
+// The block that completes the last barrier is alone in its chunk, so nobody waits for its store to the chunk's release
+// word; another block is the last to leave and clears the words.
+static void slow_store() {
+    constexpr uint32_t kBlocks = 73, kAlone = 72;
+    if (grid_of(kAlone, kBlocks, 0u).chunkBlocks != 1u) wrong("the scenario's last chunk has more than one block");
+    std::vector<Block> b(kBlocks);
+    std::vector<Outcome> out(kBlocks);
+    std::vector<std::thread> threads;
+    const auto until = [](uint32_t word, uint32_t value) {
+        for (;; std::this_thread::yield()) {
+            std::lock_guard<std::mutex> lk(mu);
+            if (words[word] == value) return;
+        }
+    };
+    for (uint32_t k = 0; k < kBlocks; ++k)
+        run(b[k], 1, threads, [&, k](uint32_t) {
+            const GridSync g = grid_of(k, kBlocks, 0xFFFFFFFFu);
+            if (k == kAlone) {
+                until(kWordArrive, 2u * (g.chunks - 1u));
+                self.slow = words + kWordRelease + kLine * g.chunk;
+            }
+            if (k == 0) self.beforeLeave = [&] { until(kWordLeft, kBlocks - 1u); };
+            solve(g, 1, nullptr, out[k]);
+            if (k == kAlone) until(kWordLeft, 0u);  // and only then its store lands
+        });
+    join(threads);
+    for (uint32_t w : words)
+        if (w) wrong("a word was left behind");
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     const uint32_t blocks = argc > 2 ? (uint32_t)std::atoi(argv[2]) : 1u;
@@ -234,6 +281,8 @@ int main(int argc, char** argv) {
         no_time(blocks);
     else if (!std::strcmp(what, "late"))
         late(blocks);
+    else if (!std::strcmp(what, "slow_store"))
+        slow_store();
     else
         wrong("unknown scenario");
     std::printf("ok\n");

@@ -33,3 +33,7 @@ def test_blocks_that_may_not_wait_all_leave(model, blocks):
 @pytest.mark.parametrize("blocks", [3, 70])
 def test_a_block_that_starts_after_the_others_gave_up_leaves_as_a_whole(model, blocks):
     model("late", blocks)
+
+
+def test_a_store_that_nobody_waits_for_lands_before_the_words_are_cleared(model):
+    model("slow_store")

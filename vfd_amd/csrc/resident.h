@@ -100,10 +100,13 @@ template <class Ops> VFD_RESIDENT bool grid_sync(GridSync& g) {
     g.epoch += 1;
     return Ops::one([&] { return sync_thread<Ops>(g) ? 1u : 0u; }) != 0u;
 }
-// The last block to leave clears the words for the next launch; an aborted solve leaves its mark.
+// The last block to leave clears the words for the next launch; an aborted solve leaves its mark. A block has waited for
+// its stores to the words before it counts as having left: the one to its own chunk's release word is seen by no other
+// block where it is alone in the chunk (73 blocks, for instance), and must not land after the clearing.
 template <class Ops> VFD_RESIDENT void grid_leave(const GridSync& g, bool aborted) {
     if (!Ops::leader()) return;
     if (aborted) Ops::store(g.w + kResidentAbortedAt, 1u);
+    Ops::settle();
     if (Ops::add(g.w + kWordLeft, 1u) != g.blocks) return;
     Ops::store(g.w + kWordArrive, 0u);
     for (uint32_t c = 0; c < 8; ++c) {
