@@ -171,6 +171,31 @@ static void all_pass(uint32_t blocks) {
     for (uint32_t w : words)
         if (w) wrong("a word was left behind");
 }
+// A solve so long that the arrivals no longer fit 32 bits between two of its barriers: all of them hold.
+static void wrap(uint32_t blocks) {
+    constexpr uint32_t kBarriers = 8;
+    const uint32_t chunks = grid_of(0, blocks, 0u).chunks, perBarrier = blocks <= kFlatBlocks ? blocks : chunks;
+    const uint32_t before = (uint32_t)((1ull << 32) / (2u * perBarrier)) - kBarriers / 2;  // barriers passed so far
+    words[kWordArrive] = 2u * perBarrier * before;
+    for (uint32_t k = 0; k < blocks; ++k) {
+        const GridSync g = grid_of(k, blocks, 0u);
+        words[kWordChunk + kLine * g.chunk] = g.chunkBlocks * before;
+        words[kWordRelease + kLine * g.chunk] = before;
+    }
+    std::vector<Block> b(blocks);
+    std::vector<Outcome> out(blocks);
+    std::vector<std::thread> threads;
+    std::atomic<uint32_t> arrived[kBarriers] = {};
+    for (uint32_t k = 0; k < blocks; ++k)
+        run(b[k], 1, threads, [&, k](uint32_t) {
+            GridSync g = grid_of(k, blocks, 0xFFFFFFFFu);
+            g.epoch = before;
+            solve(g, kBarriers, arrived, out[k]);
+        });
+    join(threads);
+    for (const Outcome& o : out)
+        if (o.passed != kBarriers) wrong("a block did not pass every barrier");
+}
 // No time to wait: blocks give up at barriers that are still open; every wave leaves.
 static void no_time(uint32_t blocks) {
     constexpr uint32_t kBarriers = 3, kWaves = 2;
@@ -281,6 +306,8 @@ int main(int argc, char** argv) {
         no_time(blocks);
     else if (!std::strcmp(what, "late"))
         late(blocks);
+    else if (!std::strcmp(what, "wrap"))
+        wrap(blocks);
     else if (!std::strcmp(what, "slow_store"))
         slow_store();
     else

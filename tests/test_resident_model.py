@@ -35,5 +35,10 @@ def test_a_block_that_starts_after_the_others_gave_up_leaves_as_a_whole(model, b
     model("late", blocks)
 
 
+@pytest.mark.parametrize("blocks", [3, 64, 100])
+def test_barriers_hold_past_the_arrivals_32_bits(model, blocks):
+    model("wrap", blocks)
+
+
 def test_a_store_that_nobody_waits_for_lands_before_the_words_are_cleared(model):
     model("slow_store")

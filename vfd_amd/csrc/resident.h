@@ -46,6 +46,9 @@ template <class Ops> VFD_RESIDENT bool solve_open(const uint32_t* words) {
 template <class Ops> VFD_RESIDENT void release_chunks(const GridSync& g, uint32_t v) {
     for (uint32_t c = 0; c < g.chunks; ++c) Ops::store(g.w + kWordRelease + kLine * c, v);
 }
+// Arrivals are counted on through a solve and may pass 2^32 (64 blocks: after 16 million Jacobi iterations), as may the
+// target; they are never farther apart than a barrier's arrivals.
+VFD_RESIDENT bool short_of(uint32_t arrivals, uint32_t target) { return (int32_t)(arrivals - target) < 0; }
 // the wait of one thread; target = arrivals (times 2) that complete the barrier
 template <class Ops> VFD_RESIDENT bool sync_thread(const GridSync& g) {
     const long long t0 = Ops::ticks();
@@ -53,7 +56,7 @@ template <class Ops> VFD_RESIDENT bool sync_thread(const GridSync& g) {
     if (g.blocks <= kFlatBlocks) {
         const uint32_t target = 2u * g.blocks * g.epoch;
         uint32_t v = Ops::add(arrive, 2u);
-        while (!(v & kAbortBit) && v < target) {
+        while (!(v & kAbortBit) && short_of(v, target)) {
             if ((uint64_t)(Ops::ticks() - t0) > g.waitTicks) {  // only a barrier that is still open can be aborted
                 uint32_t seen = v;
                 if (Ops::swap(arrive, seen, v | kAbortBit)) return false;
@@ -84,7 +87,7 @@ template <class Ops> VFD_RESIDENT bool sync_thread(const GridSync& g) {
         if ((uint64_t)(Ops::ticks() - t0) > g.waitTicks) {
             uint32_t v = Ops::load(arrive);
             if (v & kAbortBit) return false;
-            if (v >= target) continue;  // complete: its release is being written
+            if (!short_of(v, target)) continue;  // complete: its release is being written
             if (Ops::swap(arrive, v, v | kAbortBit)) {
                 release_chunks<Ops>(g, kReleaseAbort);
                 return false;
