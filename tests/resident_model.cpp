@@ -308,7 +308,10 @@ int main(int argc, char** argv) {
         late(blocks);
     else if (!std::strcmp(what, "wrap"))
         wrap(blocks);
-    else if (!std::strcmp(what, "slow_store"))
+    else if (!std::strcmp(what, "rule")) {  // tiles, scenes, CUs, tiles per group
+        if (argc != 6 || resident_tiles(blocks, std::atoi(argv[3]), std::atoi(argv[4])) != (uint32_t)std::atoi(argv[5]))
+            wrong("the rule for the groups");
+    } else if (!std::strcmp(what, "slow_store"))
         slow_store();
     else
         wrong("unknown scenario");

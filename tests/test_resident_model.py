@@ -42,3 +42,13 @@ def test_barriers_hold_past_the_arrivals_32_bits(model, blocks):
 
 def test_a_store_that_nobody_waits_for_lands_before_the_words_are_cleared(model):
     model("slow_store")
+
+
+@pytest.mark.parametrize("tiles,scenes,cus,group", [
+    (0, 1, 256, 0), (1, 1, 256, 1), (256, 1, 256, 1), (257, 1, 256, 2), (512, 1, 256, 2), (513, 1, 256, 4),
+    (1024, 1, 256, 4), (1025, 1, 256, 0), (1024, 1, 304, 4), (1025, 1, 304, 0), (64, 1, 64, 1), (257, 1, 64, 0),
+    # a wave decides for at most twelve scenes, a solve for at most 64
+    (48, 48, 256, 1), (49, 49, 256, 0), (128, 128, 256, 0), (256, 256, 256, 0), (300, 64, 256, 2), (300, 65, 256, 0),
+    (1000, 64, 256, 4), (1000, 250, 256, 0)])
+def test_which_simulations_have_resident_solves(model, tiles, scenes, cus, group):
+    model("rule", tiles, scenes, cus, group)

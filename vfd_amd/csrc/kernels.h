@@ -321,14 +321,10 @@ void launch_pres_iter(const Launch& L, const KTabHost& kt, const Fields& F);
 // aborted (null: none): positions are not written when *aborted is set
 void launch_pres_final(const Launch& L, const KTabHost& kt, const Fields& F, int writeNext, const uint32_t* aborted);
 // ---- solve.hip: whole solves as one launch ----------------------------------------------------------------------
-constexpr uint32_t kResidentScenes = 256;        // scenes of a resident solve (their scalars live in LDS)
 struct Resident {
     uint32_t* words;
     uint32_t waitTicks;  // longest wait at a barrier, in ticks of the 100 MHz wall clock
 };
-// Tiles per group with which every group has a block of its own on numCU CUs, the fewest of 1, 2 and 4; 0: none, or
-// too many scenes. Solves, halo build and density of a step take the same value.
-uint32_t resident_group_tiles(const Launch& L, uint32_t numCU);
 void launch_div_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt, const Fields& F, const Resident& r);
 void launch_pres_solve(const Launch& L, uint32_t groupTiles, const KTabHost& kt, const Fields& F, const Resident& r,
                        int writeNext);

@@ -31,6 +31,28 @@ constexpr uint32_t kAbortBit = 1u, kReleaseAbort = 0xFFFFFFFFu;
 // chunk's word and poll a release word per chunk (2.5 us at 121 blocks, 2.9 at 248, where one polled word takes 5.8).
 constexpr uint32_t kFlatBlocks = 64;
 
+constexpr uint32_t kResidentScenes = 64;  // most scenes of a resident solve (their scalars live in LDS)
+// Tiles per group of a simulation's resident solves, the fewest of 1, 2 and 4 with which every group has a CU to itself;
+// 0: no resident solves (more groups than CUs, or too many scenes). Solves, halo build and density of a step take the
+// same value.
+//
+// The fewest tiles per group win: a group's neighbour sums are bound by its CU's LDS and VALU (1024 particles 7-8 us a
+// sum, 256 particles about 2), and more blocks cost a barrier at most 1.4 us.
+//
+// Scenes: every block decides for every scene, its waves (4 a tile) taking the scenes in turn, one after the other about
+// 1.5 us each. Where a wave has more than 12 that is more than the launches saved. ms a step, launched -> resident, with up
+// to 100 CG iterations and with 2: 48 scenes of 200 particles (12 a wave) 7.54 -> 7.42 and 4.09 -> 3.80, 56 scenes 8.10 ->
+// 8.42 and 4.80 -> 4.46, 128 scenes 13.8 -> 17.3 and 10.3 -> 10.2, 256 scenes 23.1 -> 32.5; larger groups, whose blocks
+// wait for the few scenes that go on: 64 scenes of 1,900 (8 a wave) 9.41 -> 8.83 and 4.61 -> 3.83, 96 of them (6 a wave)
+// 12.3 -> 13.0 and 6.32 -> 5.84.
+inline uint32_t resident_tiles(uint32_t tiles, uint32_t scenes, uint32_t numCU) {
+    if (tiles == 0 || scenes > kResidentScenes) return 0;
+    const uint32_t most = numCU < 256u ? numCU : 256u;
+    for (uint32_t t = 1; t <= 4; t *= 2)
+        if ((tiles + t - 1) / t <= most) return scenes <= 12u * 4u * t ? t : 0u;
+    return 0;
+}
+
 struct GridSync {
     uint32_t* w;
     uint32_t blocks, chunk, chunkBlocks, chunks, epoch;

@@ -1049,7 +1049,7 @@ public:
         VFD_TRY(tileStats.alloc((size_t)std::max<uint32_t>(tiles, 1) * list_stats_per_tile(tiles)));
         {
             const Launch L = launch();
-            const uint32_t rt = resident_group_tiles(L, numCU);
+            const uint32_t rt = resident_tiles(L.tiles, L.sceneCount, numCU);
             const uint32_t groups = std::max(std::max<uint32_t>(L.groups, 1), rt ? L.group_count(rt) : 0u);
             VFD_TRY(haloCount.alloc(groups));
             VFD_TRY(haloIds.alloc((size_t)groups * kHaloMax));
@@ -1285,7 +1285,8 @@ public:
     int step(int last) {
         if (!committed) VFD_TRY(commit());
         if (tiles == 0) return VFD_OK;  // OnUpdate returns for N = 0 (:65-67)
-        uint32_t resident = useGraphs && residentPause == 0 ? resident_group_tiles(launch(), numCU) : 0u;
+        uint32_t resident =
+            useGraphs && residentPause == 0 ? resident_tiles(tiles, (uint32_t)sc.size(), numCU) : 0u;
         if (taping && resident) resident = kGroupTiles;  // recorded Jacobi solves are launched, over these groups
         if (residentPause) --residentPause;
         const int before = cur;

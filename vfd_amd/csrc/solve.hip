@@ -848,14 +848,6 @@ constexpr size_t kLdsVisc = kLdsG + RecQV::kBytes;
 constexpr size_t kLdsStatic = kResidentScenes * sizeof(SceneCtl) + 2048;  // control and reduction arrays, at most
 static_assert(kLdsVisc + kLdsStatic <= 160 * 1024 && PairSums<1>::kLds <= kLdsJacobi, "a resident group must fit a CU's LDS");
 
-// The fewest tiles per group win: a group's neighbour sums are bound by its CU's LDS and VALU (1024 particles 7-8 us a
-// sum, 256 particles about 2), and more blocks cost a barrier at most 1.4 us.
-uint32_t resident_group_tiles(const Launch& L, uint32_t numCU) {
-    if (L.tiles == 0 || L.sceneCount > kResidentScenes) return 0;
-    for (uint32_t t : {1u, 2u, 4u})
-        if ((L.tiles + t - 1) / t <= std::min(numCU, 256u)) return t;
-    return 0;
-}
 template <class Run> static void with_tiles(uint32_t groupTiles, Run&& run) {
     if (groupTiles == 1)
         run(std::integral_constant<unsigned, 1>());
