@@ -297,6 +297,31 @@ static void slow_store() {
         if (w) wrong("a word was left behind");
 }
 
+// Two simulations that keep aborting each other's solves: the limit costs them little of their time.
+static void pause() {
+    ResidentPause p;
+    uint32_t aborts = 0, steps = 0;
+    for (; steps < 10000; ++steps) {
+        if (p.over()) {
+            ++aborts;
+            p.aborted();
+        } else {
+            p.stepped(false);
+        }
+    }
+    if (aborts > 9) wrong("every attempt fails and they are not far enough apart");
+    if (aborts * (double)kResidentWait / 100.0 > 0.02 * steps * 300.0)  // us; a launched step takes 300 us and more
+        wrong("the barrier's limit costs more than 2% of the steps");
+    while (!p.over()) p.stepped(false);
+    p.stepped(true);  // one that passes: the next abort is followed by a short pause again
+    p.aborted();
+    for (uint32_t k = 0; k < ResidentPause::kFirst; ++k) {
+        if (p.over()) wrong("a pause shorter than the first");
+        p.stepped(false);
+    }
+    if (!p.over()) wrong("a pause longer than the first");
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     const uint32_t blocks = argc > 2 ? (uint32_t)std::atoi(argv[2]) : 1u;
@@ -308,6 +333,8 @@ int main(int argc, char** argv) {
         late(blocks);
     else if (!std::strcmp(what, "wrap"))
         wrap(blocks);
+    else if (!std::strcmp(what, "pause"))
+        pause();
     else if (!std::strcmp(what, "rule")) {  // tiles, scenes, CUs, tiles per group
         if (argc != 6 || resident_tiles(blocks, std::atoi(argv[3]), std::atoi(argv[4])) != (uint32_t)std::atoi(argv[5]))
             wrong("the rule for the groups");

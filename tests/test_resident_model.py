@@ -52,3 +52,7 @@ def test_a_store_that_nobody_waits_for_lands_before_the_words_are_cleared(model)
     (1000, 64, 256, 4), (1000, 250, 256, 0)])
 def test_which_simulations_have_resident_solves(model, tiles, scenes, cus, group):
     model("rule", tiles, scenes, cus, group)
+
+
+def test_simulations_that_abort_each_other_lose_little_time(model):
+    model("pause")

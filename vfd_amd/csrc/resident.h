@@ -53,6 +53,28 @@ inline uint32_t resident_tiles(uint32_t tiles, uint32_t scenes, uint32_t numCU) 
     return 0;
 }
 
+// Longest wait at a barrier, in ticks of the 100 MHz wall clock: 3 ms. A barrier takes 2-3 us and a whole solve under one
+// millisecond, so what is waited for longer is a block that other work keeps from its CU - another simulation's resident
+// solve among it, dispatched in the same microseconds, each holding CUs that the other waits for.
+constexpr uint32_t kResidentWait = 300000;
+// Steps taken with launched iterations after an aborted solve: twice as many after each abort, until a step's resident
+// solves have passed. What an abort costs (the limit, and the step begun) stays a few percent of the steps between.
+struct ResidentPause {
+    static constexpr uint32_t kFirst = 64, kMost = 4096;
+    uint32_t left = 0, next = kFirst;
+    bool over() const { return left == 0; }
+    void aborted() {
+        left = next;
+        next = next < kMost ? 2 * next : kMost;
+    }
+    void stepped(bool resident) {  // a step has been completed, with resident solves or without
+        if (resident)
+            next = kFirst;
+        else if (left)
+            --left;
+    }
+};
+
 struct GridSync {
     uint32_t* w;
     uint32_t blocks, chunk, chunkBlocks, chunks, epoch;

@@ -539,7 +539,7 @@ public:
     uint32_t lastIterations[3] = {0, 0, 0};
     // Resident solvers (solve.hip): used when every neighbour group has a block of its own and UseGraphs is on. After
     // an aborted one (other work held the CUs past the barrier's limit) the step is taken again with launched
-    // iterations, and so are the next kResidentPause steps.
+    // iterations, and so are the next ones, as ResidentPause has it.
     DevBuf<uint32_t> residentWords;
     // Pinned memory that kernels write and the host reads (or the host writes and a copy reads) without a copy of its
     // own in between: the step's report and its scenes', the grid bounds, the grids of many scenes.
@@ -550,11 +550,10 @@ public:
     DevBuf<long long> stamps;
     DevBuf<float> bakedX, bakedV;  // the baked particles, three floats a slot (Simulate restores them)
     DevBuf<float> fieldStage;      // a field in the caller's order, on its way to or from the caller
-    uint32_t residentPause = 0;
-    static constexpr uint32_t kResidentPause = 64;
-    // longest wait at a resident solve's barrier: 100 ms, or VFD_RESIDENT_WAIT_US from the environment (the aborted
+    ResidentPause residentPause;
+    // longest wait at a resident solve's barrier, or VFD_RESIDENT_WAIT_US from the environment (the aborted
     // solves of a short limit are a testing aid; results do not depend on it)
-    uint32_t residentWait = 10000000;
+    uint32_t residentWait = kResidentWait;
     Resident resident_words() const { return Resident{residentWords.p, residentWait}; }
     hipStream_t ownStream = nullptr;  // default stream (capture needs a stream other than the legacy null stream)
     // frame output: frames are packed in original order on the simulation's stream into one of two device staging
@@ -1286,20 +1285,20 @@ public:
         if (!committed) VFD_TRY(commit());
         if (tiles == 0) return VFD_OK;  // OnUpdate returns for N = 0 (:65-67)
         uint32_t resident =
-            useGraphs && residentPause == 0 ? resident_tiles(tiles, (uint32_t)sc.size(), numCU) : 0u;
+            useGraphs && residentPause.over() ? resident_tiles(tiles, (uint32_t)sc.size(), numCU) : 0u;
         if (taping && resident) resident = kGroupTiles;  // recorded Jacobi solves are launched, over these groups
-        if (residentPause) --residentPause;
         const int before = cur;
         const size_t records = tapeCount;
         int rc = step_once(last, resident);
         if (rc == kStepAborted) {  // the state the step started from is still whole: posNext, [before] and the host's
-            residentPause = kResidentPause;
+            residentPause.aborted();
             cur = before;
             tapeCount = records;
             launch_fill_u32(stream, residentWords.p, 0u, kResidentWords);
             VFD_TRY(push_state());
-            rc = step_once(last, 0);
+            return step_once(last, 0);
         }
+        residentPause.stepped(resident && !taping && last >= VFD_PHASE_DIVERGENCE);
         return rc;
     }
     static constexpr int kStepAborted = -1;
