@@ -335,7 +335,16 @@ int main(int argc, char** argv) {
         wrap(blocks);
     else if (!std::strcmp(what, "pause"))
         pause();
-    else if (!std::strcmp(what, "rule")) {  // tiles, scenes, CUs, tiles per group
+    else if (!std::strcmp(what, "recorded")) {  // groups of groupTiles have a CU each wherever they are taken
+        for (uint32_t tiles = 0; tiles < 2000; ++tiles)
+            for (uint32_t cus : {32u, 64u, 256u, 304u})
+                for (uint32_t groupTiles : {1u, 2u, 4u}) {
+                    const uint32_t fitting = resident_tiles(tiles, 1, cus), t = recorded_tiles(fitting, groupTiles);
+                    const uint32_t most = std::min(cus, 256u);
+                    if (t && (t != groupTiles || (tiles + t - 1) / t > most)) wrong("groups that do not fit the CUs");
+                    if (!t && tiles && (tiles + groupTiles - 1) / groupTiles <= most) wrong("groups that fit are refused");
+                }
+    } else if (!std::strcmp(what, "rule")) {  // tiles, scenes, CUs, tiles per group
         if (argc != 6 || resident_tiles(blocks, std::atoi(argv[3]), std::atoi(argv[4])) != (uint32_t)std::atoi(argv[5]))
             wrong("the rule for the groups");
     } else if (!std::strcmp(what, "slow_store"))

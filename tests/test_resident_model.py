@@ -56,3 +56,7 @@ def test_which_simulations_have_resident_solves(model, tiles, scenes, cus, group
 
 def test_simulations_that_abort_each_other_lose_little_time(model):
     model("pause")
+
+
+def test_groups_of_recorded_steps_fit_the_chip(model):
+    model("recorded")

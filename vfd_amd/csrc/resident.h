@@ -53,6 +53,12 @@ inline uint32_t resident_tiles(uint32_t tiles, uint32_t scenes, uint32_t numCU) 
     return 0;
 }
 
+// Tiles per group of a recorded step, whose Jacobi solves are launched, over groups of groupTiles, with the viscosity solve
+// resident over the same groups if those fit the CUs; 0: they do not. fitting: resident_tiles.
+inline uint32_t recorded_tiles(uint32_t fitting, uint32_t groupTiles) {
+    return fitting && fitting <= groupTiles ? groupTiles : 0;
+}
+
 // Longest wait at a barrier, in ticks of the 100 MHz wall clock: 3 ms. A barrier takes 2-3 us and a whole solve under one
 // millisecond, so what is waited for longer is a block that other work keeps from its CU - another simulation's resident
 // solve among it, dispatched in the same microseconds, each holding CUs that the other waits for.

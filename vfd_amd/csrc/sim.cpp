@@ -1286,7 +1286,7 @@ public:
         if (tiles == 0) return VFD_OK;  // OnUpdate returns for N = 0 (:65-67)
         uint32_t resident =
             useGraphs && residentPause.over() ? resident_tiles(tiles, (uint32_t)sc.size(), numCU) : 0u;
-        if (taping && resident) resident = kGroupTiles;  // recorded Jacobi solves are launched, over these groups
+        if (taping) resident = recorded_tiles(resident, kGroupTiles);
         const int before = cur;
         const size_t records = tapeCount;
         int rc = step_once(last, resident);
