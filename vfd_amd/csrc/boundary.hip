@@ -703,8 +703,10 @@ __global__ void __launch_bounds__(kWaves * kWave) k_mesh_field0(MeshDev mesh, co
     if (lives == 0ull) return;
     const int lead = __ffsll((long long)lives) - 1;
     f3 p = live ? node_position(map, l) : mk3(0.0f, 0.0f, 0.0f);
-    p = mk3(live ? p.x : __shfl(p.x, lead, kWave), live ? p.y : __shfl(p.y, lead, kWave),
-            live ? p.z : __shfl(p.z, lead, kWave));  // lanes without a node follow the first one that has one
+    // lanes without a node follow the first one that has one (shuffled by every lane: one that is off reads as zero, and
+    // the brick's sphere would reach to the origin)
+    const f3 q = mk3(__shfl(p.x, lead, kWave), __shfl(p.y, lead, kWave), __shfl(p.z, lead, kWave));
+    p = mk3(live ? p.x : q.x, live ? p.y : q.y, live ? p.z : q.z);
     // sphere about the brick's nodes
     auto most = [](float v) { return wave_max(v); };
     const f3 mid = mk3(0.5f * (most(p.x) - most(-p.x)), 0.5f * (most(p.y) - most(-p.y)), 0.5f * (most(p.z) - most(-p.z)));
