@@ -258,6 +258,15 @@ def _kname(raw):
     return re.sub(r"^(?:void )?(?:vfd::)?", "", raw).split("(")[0]
 
 
+def _entry(table, kernel):
+    """The entry of `kernel` in a table by kernel name, or of its one instantiation where the kernel is a template (the
+    trace names k_density_factor as k_density_factor<4u>)."""
+    if kernel in table:
+        return table[kernel]
+    named = [k for k in table if k.startswith(kernel + "<")]
+    return table[named[0]] if len(named) == 1 else None
+
+
 def _pmc_table(path):
     """{kernel: {counter: mean value}} from a rocprofv3 --pmc counter_collection.csv (or the directory holding it),
     over the live dispatches (>= LIVE_US) of the solver-loop kernels and every dispatch of the others."""
@@ -345,7 +354,7 @@ def counter_summary(lds_dir, valu_dir, kernels=("div_iter", "div_accel", "pres_i
     lines = ["| kernel | duration cycles | LDS active | bank-conflict share | LDS busy | LDS insts | LDS issue wait | "
              "VALU insts | VALU busy | VMEM reads | wait any (issue) |", "|---|" + "---:|" * 10]
     for k in kernels:
-        a, b = lds.get("k_" + k), valu.get("k_" + k)
+        a, b = _entry(lds, "k_" + k), _entry(valu, "k_" + k)
         if not a or not b:
             continue
         dur = a["SQ_BUSY_CYCLES"] / SHADER_ENGINES
@@ -367,7 +376,7 @@ def memory_unit_summary(path, kernels=("build_lists", "div_iter", "div_accel", "
     t = _pmc_table(path)
     lines = ["| kernel | duration cycles | TA busy | TD busy | VMEM reads |", "|---|---:|---:|---:|---:|"]
     for k in kernels:
-        a = t.get("k_" + k)
+        a = _entry(t, "k_" + k)
         if not a:
             continue
         dur = a["SQ_BUSY_CYCLES"] / SHADER_ENGINES
