@@ -682,13 +682,14 @@ __global__ void __launch_bounds__(kTile) k_mesh_spheres(MeshDev mesh, float4* ou
 // squared distances stays below 1e-6 u^2.
 //   1. every node's bound over all clusters, and the triangles of the cluster nearest to the brick, so that s starts
 //      near the minimum;
-//   2. 64 triangles at a time, a lane per triangle: its sphere against the brick's with the largest s of the nodes;
+//   2. 64 triangles of another cluster at a time, a lane per triangle: its sphere against the brick's with the largest s
+//      of the nodes;
 //   3. what is left, triangle by triangle: each node's sphere test, then the distance where some node needs it (40
 //      instructions and more, as the lanes fall into different regions).
 // The triangles are read at wave-uniform addresses (scalar loads). Most bricks test a few dozen triangles, but those
-// near the middle of a round body test them all, and a wave to itself took 2.7 ms for one of 5,120 triangles, the whole
-// kernel with it (0.36 ms of VALU work); 406k nodes now take 0.97 ms, 0.63 ms of it VALU work. The winner's closest point and feature give the sign: negative
-// where (p - closest) points against the feature's normal.
+// near the middle of a round body test them all, and a wave to itself takes 1.8 ms for one of 5,120 triangles and 406k
+// nodes, the whole kernel with it (0.35 ms of VALU work); eight waves take 0.67 ms. The winner's closest point and
+// feature give the sign: negative where (p - closest) points against the feature's normal.
 constexpr float kFarA = 1.01289f, kFarB = 1.00646f;  // (1 + e) / (1 - e) and 1 / (1 - e), e = 6.4e-3, rounded up
 template <uint32_t kWaves>
 __global__ void __launch_bounds__(kWaves * kWave) k_mesh_field0(MeshDev mesh, const float4* __restrict__ spheres,
@@ -762,6 +763,7 @@ __global__ void __launch_bounds__(kWaves * kWave) k_mesh_field0(MeshDev mesh, co
     s = fminf(s, reach_of(least(best)));
     float smax = most(s);
     for (uint32_t c = w; c < clusters; c += kWaves) {
+        if (c == first) continue;  // tested above
         const uint32_t t = c * kMeshCluster + lane;
         bool keep = false, tested = false;
         if (t < mesh.triCount) {
@@ -806,7 +808,11 @@ __global__ void __launch_bounds__(kWaves * kWave) k_mesh_field0(MeshDev mesh, co
     nodes0[l] = sign * (d - tol);
 }
 
-// A wave per cluster of the brick, up to eight: fewer triangles leave the further ones nothing to do.
+// Waves that share a brick's clusters: one, two from two clusters on, eight from eight. us with 1, 2 and 8 waves on maps
+// of 12^3 and of 40^3 cells: 60 triangles 48 and 72 whatever their number; 120 triangles 95, 72, 55 and 110, 101, 144; 250
+// triangles 189, 122, 65 and 225, 170, 181; 440 triangles 317, 209, 72 and 335, 247, 204; 512 triangles 350, 211, 72 and
+// 385, 258, 208; 5,120 triangles 3113, 1737, 556 and 1826, 1124, 665. Few bricks leave the chip idle and gain from more
+// waves at once; many bricks only once a wave has a cluster to itself or nearly so, and the line follows those.
 void launch_mesh_field0(hipStream_t st, const MeshDev& mesh, float4* triSpheres, const MapDev& map, float sign, float tol,
                         float* nodes0) {
     const uint32_t bricks = NodeBricks(map).waves(), clusters = (mesh.triCount + kMeshCluster - 1) / kMeshCluster;
