@@ -770,7 +770,56 @@ void launch_visc_apply(const Launch& L, const Fields& F) {
 // lane per Monte-Carlo sample. A thread that walked the samples of its candidate against its neighbours was one serial
 // chain of up to 50 x 40 distance tests while its wave's other lanes waited: 214 us for 990 particles and 132 us for
 // 250k; both launches together now take 14 and 95 us.
+// Where a wave's particles are nearly all candidates (a thin layer), their samples few and the waves so many that their
+// chains overlap, the thread that walks them is still the better one and stays (sample_in_place): a candidate's wave waits
+// longer for its neighbours than a thread takes for a few samples. us of the whole phase on a layer, a wave each -> in
+// place: 250,000 particles with 3 samples 198 -> 54, with 16 228 -> 125; 100,000 with 16 102 -> 85; 30,000 with 3 41 -> 31,
+// with 8 43 either way, with 16 44 -> 68. With fewer candidates a wave its thread's chain is not hidden: waves of 17 and
+// more in place took the phase of a 100,000 block with 8 samples from 52 to 76.
 // F.surface: [0] the number of candidates, [1 + k] their slots (any order: each is sampled by itself).
+// the normal and the curvature of a candidate with `count` uncovered samples, their sum nsum
+__device__ __forceinline__ void note_samples(const SceneParams& p, const Fields& F, uint32_t i, uint32_t count, f3 nsum,
+                                             const float* __restrict__ mcTab) {
+    if (count > 0) {
+        if (length2(nsum) > 0.0f) nsum = normalize(nsum);
+        F.nMC[i] = st4(nsum);
+        F.kMC[i] = 1.0f / p.R * -2.0f * sqrtf(1.0f - p.NR * p.NR / (p.r * p.r)) * mcTab[count];
+    } else {
+        F.kMC[i] = 0.0f;
+    }
+}
+constexpr uint32_t kStBatch = 8;  // neighbours whose positions are loaded together, so that their latencies overlap
+__device__ __forceinline__ bool sample_in_place(uint32_t candidates, uint32_t S, uint32_t tiles) {
+    return candidates >= 56u && S <= 16u && tiles >= 24u * S;
+}
+// one thread's candidate: its samples one after the other against its n neighbours
+__device__ __forceinline__ void sample_candidate(const SceneParams& p, const Fields& F, uint32_t cap, uint32_t i, f3 xi,
+                                                 uint32_t n, uint32_t S, const float* __restrict__ mcTab) {
+    const float R = p.R;
+    const uint32_t s = F.id[i] * S / 3u * 3u;
+    const float rr = p.NR / p.r;
+    const float lim = rr * rr * p.R2;
+    uint32_t count = 0;
+    f3 nsum = mk3(0.0f, 0.0f, 0.0f);
+    for (uint32_t q = 0; q < S; ++q) {
+        const uint32_t i3 = s + 3u * q;
+        const f3 pt = R * mk3(F.halton[i3 % kHaltonFloats], F.halton[(i3 + 1u) % kHaltonFloats],
+                              F.halton[(i3 + 2u) % kHaltonFloats]);
+        bool covered = false;
+        for (uint32_t j0 = 0; j0 < n && !covered; j0 += kStBatch) {
+            f3 xb[kStBatch];
+#pragma unroll
+            for (uint32_t u = 0; u < kStBatch; ++u) xb[u] = ld3(F.pos[nbr(F, cap, i, min(j0 + u, n - 1u))]);
+#pragma unroll
+            for (uint32_t u = 0; u < kStBatch; ++u)
+                if (j0 + u < n && length2(pt - (xb[u] - xi)) <= lim) covered = true;
+        }
+        if (covered) continue;
+        nsum = nsum + pt;
+        ++count;
+    }
+    note_samples(p, F, i, count, nsum, mcTab);
+}
 __global__ void __launch_bounds__(kTile) k_st_classify(const SceneParams* __restrict__ P,
                                                        const uint32_t* __restrict__ tileScene, Fields F,
                                                        uint32_t cap, long long* stamps) {
@@ -778,17 +827,17 @@ __global__ void __launch_bounds__(kTile) k_st_classify(const SceneParams* __rest
     const TileCtx c = tile_ctx(tileScene, P);
     const SceneParams& p = P[c.s];
     bool candidate = false;
+    f3 xi = mk3(0.0f, 0.0f, 0.0f);
+    uint32_t n = 0;
     if (c.valid && p.enableST) {
         const float R = p.R;
-        const f3 xi = ld3(F.pos[c.i]);
-        const uint32_t n = F.nbrCount[c.i];
+        xi = ld3(F.pos[c.i]);
+        n = F.nbrCount[c.i];
         F.nMC[c.i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (n == 0) {
             F.kMC[c.i] = 1.0f / R;
         } else {
-            // neighbour positions are loaded kStBatch at a time so that their latencies overlap; sums in list order
-            constexpr uint32_t kStBatch = 8;
-            f3 com = mk3(0.0f, 0.0f, 0.0f);
+            f3 com = mk3(0.0f, 0.0f, 0.0f);  // sums in list order
             for (uint32_t j0 = 0; j0 < n; j0 += kStBatch) {
                 f3 xb[kStBatch];
 #pragma unroll
@@ -804,6 +853,11 @@ __global__ void __launch_bounds__(kTile) k_st_classify(const SceneParams* __rest
     }
     const unsigned long long b = __ballot(candidate);
     if (b == 0ull) return;
+    const uint32_t S = F.state[c.s].S;
+    if (sample_in_place((uint32_t)__popcll(b), S, gridDim.x)) {  // wave-uniform
+        if (candidate) sample_candidate(p, F, cap, c.i, xi, n, S, F.mcTab + F.mcOff[c.s]);
+        return;
+    }
     const int lane = threadIdx.x & (kWave - 1), first = __ffsll((long long)b) - 1;
     uint32_t at = 0;
     if (lane == first) at = atomicAdd(&F.surface[0], (uint32_t)__popcll(b));
@@ -858,15 +912,7 @@ __global__ void __launch_bounds__(kTile) k_st_sample(const SceneParams* __restri
                 nsum = nsum + mk3(__shfl(pt.x, q, kWave), __shfl(pt.y, q, kWave), __shfl(pt.z, q, kWave));
             }
         }
-        if (lane == 0) {
-            if (count > 0) {
-                if (length2(nsum) > 0.0f) nsum = normalize(nsum);
-                F.nMC[i] = st4(nsum);
-                F.kMC[i] = 1.0f / R * -2.0f * sqrtf(1.0f - p.NR * p.NR / (p.r * p.r)) * F.mcTab[F.mcOff[scene] + count];
-            } else {
-                F.kMC[i] = 0.0f;
-            }
-        }
+        if (lane == 0) note_samples(p, F, i, count, nsum, F.mcTab + F.mcOff[scene]);
         __builtin_amdgcn_wave_barrier();  // the next candidate's positions follow this one's reads
     }
 }
@@ -885,7 +931,7 @@ __global__ void __launch_bounds__(kTile) k_st_normals(const SceneParams* __restr
     f3 nc = mk3(0.0f, 0.0f, 0.0f);
     float cc = 0.0f, cf = 0.0f;
     const uint32_t n = F.nbrCount[c.i];
-    constexpr uint32_t kStBatch = 8;  // neighbours whose loads are in flight together; terms in list order
+    // kStBatch neighbours' loads are in flight together; terms in list order
     for (uint32_t j0 = 0; j0 < n; j0 += kStBatch) {
         f3 nj[kStBatch], xj[kStBatch];
         float kj[kStBatch];
