@@ -427,7 +427,8 @@ typedef struct vfd_tuning {
     uint32_t SolverCheckInterval; /* Jacobi / CG iterations enqueued between two convergence checks, >= 1 */
     uint32_t HaloLimit;           /* largest group halo staged in LDS (<= 3808); 0: every neighbour from HBM */
     uint32_t UseGraphs;           /* 1: each chunk of iterations is one launch of a captured HIP graph, and in a
-                                     simulation of at most 1024 particles per compute unit each solve is one launch;
+                                     simulation of at most 1024 particles per compute unit and 64 scenes (48 up to
+                                     256 particles per compute unit) each solve is one launch;
                                      0: every kernel of an iteration is launched by itself */
     uint32_t PredictIterations;   /* 1: a solver's first chunk is one iteration short of what it ran in the
                                      previous step, so that few empty iterations follow its convergence (default 0) */

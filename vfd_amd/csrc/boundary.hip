@@ -688,7 +688,7 @@ __global__ void __launch_bounds__(kTile) k_mesh_spheres(MeshDev mesh, float4* ou
 //      instructions and more, as the lanes fall into different regions).
 // The triangles are read at wave-uniform addresses (scalar loads). Most bricks test a few dozen triangles, but those
 // near the middle of a round body test them all, and a wave to itself takes 1.8 ms for one of 5,120 triangles and 406k
-// nodes, the whole kernel with it (0.35 ms of VALU work); eight waves take 0.67 ms. The winner's closest point and
+// nodes, the whole kernel with it; eight waves take 0.67 ms, 0.3 ms of it VALU work. The winner's closest point and
 // feature give the sign: negative where (p - closest) points against the feature's normal.
 constexpr float kFarA = 1.01289f, kFarB = 1.00646f;  // (1 + e) / (1 - e) and 1 / (1 - e), e = 6.4e-3, rounded up
 template <uint32_t kWaves>

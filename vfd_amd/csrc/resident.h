@@ -59,9 +59,9 @@ inline uint32_t recorded_tiles(uint32_t fitting, uint32_t groupTiles) {
     return fitting && fitting <= groupTiles ? groupTiles : 0;
 }
 
-// Longest wait at a barrier, in ticks of the 100 MHz wall clock: 3 ms. A barrier takes 2-3 us and a whole solve under one
-// millisecond, so what is waited for longer is a block that other work keeps from its CU - another simulation's resident
-// solve among it, dispatched in the same microseconds, each holding CUs that the other waits for.
+// Longest wait at a barrier, in ticks of the 100 MHz wall clock: 3 ms. A barrier takes 2-3 us and a whole solve 0.03 to 2
+// ms, so what is waited for longer is a block that other work keeps from its CU - another simulation's resident solve
+// among it, dispatched in the same microseconds, each holding CUs that the other waits for.
 constexpr uint32_t kResidentWait = 300000;
 // Steps taken with launched iterations after an aborted solve: twice as many after each abort, until a step's resident
 // solves have passed. What an abort costs (the limit, and the step begun) stays a few percent of the steps between.

@@ -253,9 +253,11 @@ __device__ __forceinline__ uint32_t neighbor_list(const TileCtx& c, const SceneP
 // k_build_lists takes as long as its longest thread, 30 us of waiting on some 30 batches of candidates one after the
 // other, however few particles there are. Where the chip is not full the nine rows of a particle (three cells each) are
 // given to nine lanes of sixteen: a lane tests its row, the lanes' counts are summed up so that each knows where its
-// neighbours begin in the list, and it stores them there. Same candidates, same tests, same order, same cap. Up to
-// kRowTiles tiles: 34.1 -> 9.3 us on 990 particles, 36 -> 9.9 on 8,000; its sixteen lanes a particle cost about 0.5 us
-// per thousand, so that it meets the other's 35 us near 50,000 particles (79 us against 60 on 123,000).
+// neighbours begin in the list, and it stores them there. Same candidates, same tests, same order, same cap.
+// us, a thread a particle -> a lane a row, on lattices of 2 and of 1.6 radii: 990 particles 33 -> 9 and 71 -> 24, 8,000
+// 37 -> 9 and 81 -> 25, 32,768 37 -> 21 and 82 -> 51, 50,000 38 -> 31 and 84 -> 74, 65,536 39 -> 38 and 84 -> 90, 123,000
+// 46 -> 65 and 97 -> 154: sixteen lanes a particle cost about 0.5 us per thousand, and the two meet at about 60,000. The
+// line lies at half of that, 128 tiles, where a lane a row is far ahead on either lattice; up to 50,000 it would still be.
 constexpr uint32_t kRowTiles = 128;
 constexpr uint32_t kRowLanes = 16;                       // nine rows
 constexpr uint32_t kRowParticles = kTile / kRowLanes;    // particles of a block

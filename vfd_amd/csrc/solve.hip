@@ -3,7 +3,7 @@
 // DFSPHImplementation.cu:443-808).
 //
 // For a simulation whose neighbour groups all fit the chip at once (one group of 256, 512 or 1024 particles per block,
-// one block per CU: 262,144 particles on 256 CUs) an iteration launched as separate kernels is bound by the launches:
+// one block per CU: 262,144 particles on 256 CUs; resident.h has the rule) an iteration launched as separate kernels is bound by the launches:
 // each pays about 4.5 us of start and end, 4-5 us to copy the kernel table into LDS and the latency of refilling the halo's
 // positions, around 2-5 us of neighbour sums; iterations enqueued past convergence pay the launches too. Here a block
 // keeps the table, its halo's positions and slots and its particles' own data for the whole solve, and the blocks
