@@ -1,6 +1,6 @@
-"""Surface tension where nearly every particle is a surface candidate, against the oracle: where a wave has 56 candidates or
-more, at most 16 samples each, and there are 24 tiles a sample, a thread samples its own candidate, else a wave does. Sizes
-and sample counts on both sides of the rule; the layer's last tile holds a wave of fewer candidates."""
+"""Surface tension where nearly every particle is a surface candidate, against the oracle: where all of a wave's particles are
+candidates, with at most 16 samples each, and there are 24 tiles a sample, a thread samples its own candidate, else a wave
+does. Sizes and sample counts on both sides of the rule; the layer's last wave is not full."""
 import numpy as np
 import pytest
 

@@ -770,12 +770,13 @@ void launch_visc_apply(const Launch& L, const Fields& F) {
 // lane per Monte-Carlo sample. A thread that walked the samples of its candidate against its neighbours was one serial
 // chain of up to 50 x 40 distance tests while its wave's other lanes waited: 214 us for 990 particles and 132 us for
 // 250k; both launches together now take 14 and 95 us.
-// Where a wave's particles are nearly all candidates (a thin layer), their samples few and the waves so many that their
+// Where a wave's particles are all candidates (a thin layer), their samples few and the waves so many that their
 // chains overlap, the thread that walks them is still the better one and stays (sample_in_place): a candidate's wave waits
 // longer for its neighbours than a thread takes for a few samples. us of the whole phase on a layer, a wave each -> in
 // place: 250,000 particles with 3 samples 198 -> 54, with 16 228 -> 125; 100,000 with 16 102 -> 85; 30,000 with 3 41 -> 31,
-// with 8 43 either way, with 16 44 -> 68. With fewer candidates a wave its thread's chain is not hidden: waves of 17 and
-// more in place took the phase of a 100,000 block with 8 samples from 52 to 76.
+// with 8 43 either way, with 16 44 -> 68. Where waves have other particles too there are fewer of them, and
+// a thread's chain is not hidden: waves of 17 candidates and more in place took the phase of a 100,000 block with 8
+// samples from 52 to 76, waves of 56 and more that of the viscous column's third step from 86 to 121.
 // F.surface: [0] the number of candidates, [1 + k] their slots (any order: each is sampled by itself).
 // the normal and the curvature of a candidate with `count` uncovered samples, their sum nsum
 __device__ __forceinline__ void note_samples(const SceneParams& p, const Fields& F, uint32_t i, uint32_t count, f3 nsum,
@@ -790,7 +791,7 @@ __device__ __forceinline__ void note_samples(const SceneParams& p, const Fields&
 }
 constexpr uint32_t kStBatch = 8;  // neighbours whose positions are loaded together, so that their latencies overlap
 __device__ __forceinline__ bool sample_in_place(uint32_t candidates, uint32_t S, uint32_t tiles) {
-    return candidates >= 56u && S <= 16u && tiles >= 24u * S;
+    return candidates == kWave && S <= 16u && tiles >= 24u * S;
 }
 // one thread's candidate: its samples one after the other against its n neighbours
 __device__ __forceinline__ void sample_candidate(const SceneParams& p, const Fields& F, uint32_t cap, uint32_t i, f3 xi,
